@@ -335,3 +335,17 @@ def test_kernel_choice_by_shape():
         ops._workspace(_Probe(), M, 4096, 11008, 128, None, None)
         ops._ws_need.pop((M, 4096, 11008, 128), None)
     assert asked == [(17, 4096, 11008, 128)]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: the answer has to come from the host")
+def test_an_unpadded_w_is_refused_by_kernels_that_gather_it():
+    """gemm_generic and gemm_skinny read W without a range check: a W whose rows end before the padded contraction does is copied
+    for them by the caller (8 rows x 65600 -> 262144 at block 64: past gemv_staged's 32-bit scale offsets)"""
+    lib = _lib.load()
+    M, N, K, kw = 8, 262144, 65664, 65600
+    assert lib.bi8_gemm_kernel_name(M, N, K, K, kw, 64, 0) == b"gemm_skinny"
+    gemm = lib.bi8x_gemm
+    gemm.argtypes = _lib.SIGNATURES["bi8_gemm_nt_dequant_ws"][1][:11] + [ctypes.c_int64] + _lib.SIGNATURES["bi8_gemm_nt_dequant_ws"][1][11:]
+    p = ctypes.c_void_p(1 << 20)
+    assert gemm(p, p, p, p, None, 0, p, 1, M, N, K, kw, K, kw, N, 64, None, 0, None) == _lib.ERR_UNSUPPORTED
+    assert gemm(p, p, p, p, None, 0, p, 1, 300, 500, 512, 448, 512, 448, 500, 48, None, 0, None) == _lib.ERR_UNSUPPORTED
