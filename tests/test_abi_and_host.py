@@ -230,15 +230,18 @@ def test_kernel_choice_by_shape():
     assert name(8192, 8192, 8192, 128) == "gemm_wide" and name(8192, 8192, 8192, 64) == "gemm_wide"
     assert name(8192, 8192, 8192, 32) == "gemm_wide"                 # (the 32x32x32-MFMA form of the 256x256 kernel)
     assert name(2048, 4096, 4096, 32) == "gemm_tile_128x128"         # block 32 has no 256x128 tile
-    assert name(2944, 2944, 512, 128) == "gemm_wide"                 # 12 x 12 = 144 tiles of 256x256
+    assert name(2944, 2944, 4096, 128) == "gemm_wide"                # 12 x 12 = 144 tiles of 256x256
+    assert name(2944, 2944, 512, 128) == "gemm_wide_128x96" and name(5200, 5101, 384, 128) == "gemm_wide_128x128"
     # a last round of 256x256 tiles that is mostly empty: whole rows (columns) of tiles cut off for a second launch
     assert name(1536, 11008, 4096, 128) == "gemm_wide+gemm_tile_128x128" and name(2048, 11008, 4096, 128) == "gemm_wide+gemm_wide_256x128"
     assert name(1536, 11008, 4096, 128, 1 << 30) == "gemm_wide+gemm_tile_64x128_splitk"
-    assert name(2048, 12288, 4096, 128) == "gemm_wide" and name(1280, 11008, 4096, 128) == "gemm_wide"   # half a round left / one round
+    assert name(2048, 12288, 4096, 128) == "gemm_wide_256x128" and name(1280, 11008, 4096, 128) == "gemm_wide"   # half a round left / one round
     # more than 256 tiles of 128x128 that do not fill the chip with 256x256 tiles: the 256x256 kernel's loop on 256x128 tiles
-    assert name(8192, 768, 3072, 64) == "gemm_wide_256x128" and name(8192, 768, 3072, 128) == "gemm_wide_256x128"
+    # ... or, where those fill the last round better, on tiles of 128x128 or 128x96 with two workgroups per CU
+    assert name(8192, 768, 3072, 64) == "gemm_wide_128x96" and name(8192, 768, 3072, 128) == "gemm_wide_128x96"
+    assert name(4500, 4400, 256, 64) == "gemm_wide+gemm_wide_128x128" and name(4128, 5000, 512, 64) == "gemm_wide+gemm_wide_256x128"
     assert name(2048, 4096, 4096, 128) == "gemm_wide_256x128"        # 128 tiles of 256x256: one round of 256x128 tiles
-    assert name(2048, 4096, 512, 64) == "gemm_wide_256x128" and name(2048, 2304, 512, 64) == "gemm_wide_256x128"
+    assert name(2048, 4096, 512, 64) == "gemm_wide_256x128" and name(2048, 2304, 512, 64) == "gemm_wide_128x96"
     assert name(2048, 4096, 4096, 128, 0, 1 << 21, 4096) == "gemm_tile_256x128"     # rows 2 MiB apart: beyond its 32-bit offsets
     assert name(1500, 1500, 512, 32) == "gemm_tile_128x128" and name(48, 5000, 640, 32) == "gemm_tile_64x128"
     assert name(1024, 3072, 4096, 64) == "gemm_tile_128x128"         # block 64: 384 tiles of 128 x 64 are more than one round of the square form
@@ -262,7 +265,7 @@ def test_kernel_choice_by_shape():
     # 33 to 64 rows: the same on tiles of 64 rows x 32 ... 128 columns, where gemv_staged (below) does not apply or K is at most 1024
     assert name(64, 5000, 640, 128) == "gemm_panel" and name(48, 11008, 4096, 128, 1 << 30) == "gemm_panel" and name(33, 16384, 4096, 64) == "gemm_panel"
     assert name(48, 700, 640, 128) == "gemm_panel" and name(64, 2048, 1024, 64) == "gemm_panel" and name(64, 2048, 1152, 64) == "gemv_staged"
-    assert name(64, 33000, 768, 128) == "gemm_wide"                  # too many columns for one round
+    assert name(64, 33000, 768, 128) == "gemm_wide_128x96"                  # too many columns for one round
     # 3 to 32 rows against 5120 columns or more: the same on tiles of 32 rows x 64 ... 256 columns
     assert name(32, 11008, 768, 128) == "gemm_panel" and name(16, 11008, 4096, 64) == "gemm_panel" and name(3, 5120, 4096, 128, 1 << 30) == "gemm_panel"
     assert name(32, 11008, 4096, 64, 1 << 30) == "gemm_panel" and name(16, 32000, 4096, 128) == "gemm_panel" and name(8, 50257, 768, 128) == "gemm_panel"

@@ -149,7 +149,7 @@ def test_bias_dtypes_on_the_persistent_kernel(ops, out, block):
     that walks on to a second tile fetches that tile's bias after a barrier.  Odd N: the last tile's bias ends mid-dword."""
     from blockwise_int8_linear_amd import _lib
     g = torch.Generator().manual_seed(7 + block)
-    M, N, K = 5200, 5101, 256
+    M, N, K = 5658, 5101, 512 if block == 64 else 384                  # 460 tiles
     assert _lib.load().bi8_gemm_kernel_name(M, N, K, K, K, block, 0).decode() == "gemm_wide"
     A, W = _codes(g, M, K).to(DEV), _codes(g, N, K).to(DEV)
     sa = (torch.rand(K // block, M, generator=g) + 0.1).to(DEV)
@@ -438,7 +438,8 @@ def _run_nonfinite_few_rows(ops, A, W, block, g):
 
 # (M, N, K, kernel family)
 NONFINITE_SHAPES = [(300, 500, 512, "gemm_panel"), (1500, 1500, 256, "gemm_panel_square"), (16, 6400, 256, "gemm_panel_few_rows"),
-                    (1500, 1500, 256, "gemm_tile_128x128", 32), (2600, 2900, 256, "gemm_wide"), (5200, 5100, 256, "gemm_wide"),
+                    (1500, 1500, 256, "gemm_tile_128x128", 32), (1708, 5200, 384, "gemm_wide"), (4876, 5000, 384, "gemm_wide"),
+                    (2600, 2900, 256, "gemm_wide_128x128"), (5200, 5100, 256, "gemm_wide_128x128"), (2944, 2900, 384, "gemm_wide_128x96"),
                     (4400, 4500, 256, "gemm_wide+gemm_tile_128x128"), (2048, 2304, 256, "gemm_wide_256x128"),
                     (8, 256, 512, "gemv_staged"), (24, 256, 512, "gemv_staged_two_row_groups"), (24, 256, 512, "gemm_skinny", 32),
                     (70, 90, 200, "gemm_generic"), (8, 256, 2560, "gemv_staged_long"), (2, 256, 1536, "gemv_rows")]

@@ -72,15 +72,21 @@ def _device_codes(A, pitch):
 
 # (M, N, K, block, kernel the shipped operator runs on it)
 CASES = [
-    (2944, 2944, 512, 128, "gemm_wide"),            # 144 tiles of 256x256, four stages
-    (2944, 2900, 384, 128, "gemm_wide"),            # odd number of stages (the loop runs a padding stage), ragged N
-    (2944, 2944, 512, 64, "gemm_wide"),             # two K-blocks per stage
-    (2900, 2944, 384, 64, "gemm_wide"),
+    (1708, 5200, 512, 128, "gemm_wide"),            # 147 tiles of 256x256, four stages
+    (1796, 5000, 384, 128, "gemm_wide"),            # odd number of stages (the loop runs a padding stage), ragged edges
+    (2324, 5200, 256, 64, "gemm_wide"),             # two K-blocks per stage
+    (3116, 3841, 384, 64, "gemm_wide"),
+    (2944, 2944, 512, 128, "gemm_wide_128x96"),     # 713 tiles of 128x96, two workgroups per CU: they walk on to a second tile
+    (2944, 2900, 384, 128, "gemm_wide_128x96"),
+    (2944, 2944, 512, 64, "gemm_wide_128x96"),
+    (2900, 2944, 384, 64, "gemm_wide_128x96"),
     (5200, 5200, 384, 128, "gemm_wide"),            # 441 tiles: workgroups of the persistent grid walk on to a second tile
-    (5200, 5100, 256, 64, "gemm_wide"),
+    (4876, 5000, 640, 64, "gemm_wide"),             # 400 tiles
+    (5200, 5100, 256, 64, "gemm_wide_128x96"),
     # 324 tiles = one full round and 68: the leading 14 rows of tiles on the 256x256 kernel, the other rows on 128x128 tiles
     (4400, 4500, 384, 128, "gemm_wide+gemm_tile_128x128"),
-    (4500, 4400, 256, 64, "gemm_wide+gemm_wide_256x128"),          # ... on the same loop, 256x128 tiles from tile row 14 on
+    (4128, 5000, 512, 64, "gemm_wide+gemm_wide_256x128"),          # ... on the same loop, 256x128 tiles
+    (4500, 4400, 256, 64, "gemm_wide+gemm_wide_128x128"),          # ... 128x128 tiles, two workgroups per CU
     (2048, 8900, 256, 128, "gemm_wide+gemm_tile_128x128"),         # cut by columns: 8 x 35 tiles, the last 3 columns of tiles apart
     (2000, 8900, 384, 64, "gemm_wide+gemm_tile_128x128"),
     (4352, 4096, 2048, 128, "gemm_wide+gemm_tile_64x128_splitk"),  # the rest (one row of 16 tiles) splits K
@@ -91,12 +97,14 @@ CASES = [
     (4300, 4096, 4096, 64, "gemm_wide+gemm_tile_128x128_splitk"),
     (2944, 2944, 256, 32, "gemm_wide"),             # block 32: the 32x32x32-MFMA form, four K-blocks per stage
     (2900, 2944, 384, 32, "gemm_wide"),
-    (2048, 2304, 512, 128, "gemm_wide_256x128"),    # 256x128 tiles on the 256x256 kernel's loop, 64x64 per wave
-    (2000, 2304, 384, 128, "gemm_wide_256x128"),    # odd number of stages, ragged M
+    (1182, 5000, 384, 128, "gemm_wide_256x128"),    # 256x128 tiles on the 256x256 kernel's loop, 64x64 per wave; odd number of stages, ragged M
+    (1444, 4097, 640, 64, "gemm_wide_256x128"),     # ... two K-blocks per stage, a last column of tiles of one column
+    (2048, 2304, 512, 128, "gemm_wide_128x96"),
+    (2000, 2304, 384, 128, "gemm_wide_128x96"),
     (2048, 4096, 512, 64, "gemm_wide_256x128"),
-    (2048, 2304, 512, 64, "gemm_wide_256x128"),
-    (8192, 768, 256, 64, "gemm_wide_256x128"),
-    (8100, 760, 384, 64, "gemm_wide_256x128"),      # ragged M and N
+    (2048, 2304, 512, 64, "gemm_wide_128x96"),
+    (8192, 768, 256, 64, "gemm_wide_128x96"),
+    (8100, 760, 384, 64, "gemm_wide_128x96"),       # ragged M and N
     # rows of A 4 MiB apart put the operand beyond the 32-bit offsets of the 256x256 kernel's loop: the tile kernel's
     # software-pipelined block-128 instantiation, and its three-buffer form at block 64 (sixth entry: row pitch of A)
     (600, 11008, 256, 128, "gemm_tile_256x128", (1 << 22) - 128),
