@@ -7,6 +7,8 @@
 // Replaces triton_functions.py:142-168, :221-233, :492-500 (the launchers) and block_linear.py:69-112 (the autograd function).
 #include <Python.h>
 
+#include <cstring>
+
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
@@ -145,6 +147,14 @@ bool whole_chunks(const Tensor &w, int64_t contraction) {
 }
 // M*N*K below which the general kernel is as quick as a padded copy
 constexpr int64_t kPadMinWork = 1 << 22;
+bool small_product(int64_t M, int64_t N, int64_t K) { return (double)M * (double)N * (double)K < (double)kPadMinWork; }
+// Whether the layer multiplies codes padded along a contraction of K.  Small products with a ragged contraction stay with the general
+// kernel, as the operator's do: the tiled kernels round the column scales to 22 bits (twice its fp32 error in the 2-norm) and make
+// an infinite one NaN.  The few-row kernels take the scales as they are, so products that run on those are padded whatever the size.
+bool pad_contraction(int64_t M, int64_t N, int64_t K, int64_t block) {
+    const int64_t kp = up(K, 128);
+    return kp == K || !small_product(M, N, K) || std::strncmp(bi8_gemm_kernel_name(M, N, kp, kp, kp, (int)block, scratch_for(M, N, kp, block)), "gemv_", 5) == 0;
+}
 
 // a [M,K] codes, w [N,K] codes (both with contiguous rows), any block size and alignment.
 //  * A K-block of 256, 512, ... codes is two, four, ... runs of 128 codes that share their scales: with every scale row repeated
@@ -154,9 +164,8 @@ constexpr int64_t kPadMinWork = 1 << 22;
 //    would fall to the general kernel.  Zero codes add nothing to any block partial, so A is copied once into rows padded with zero
 //    codes up to the next multiple of 128 (and its scales with zero rows if that adds K-blocks); W too where its rows are not 16-byte
 //    aligned or the block is 32, which the kernels that read W through range-checked buffers do not serve.
-// `tiled`: pad whatever the size, so that the layer's results do not depend on how its codes came about.
 // `scratch`: memory that the split of K may use, instead of an allocation of its own.
-Tensor gemm(Tensor a, Tensor w, Tensor sx, Tensor sw, const Tensor &bias_in, int64_t block, ScalarType out_type, bool tiled, const Tensor &scratch = Tensor()) {
+Tensor gemm(Tensor a, Tensor w, Tensor sx, Tensor sw, const Tensor &bias_in, int64_t block, ScalarType out_type, const Tensor &scratch = Tensor()) {
     const int64_t M = a.size(0), N = w.size(0);
     int64_t K = a.size(1);
     require(sx.is_cuda() && sw.is_cuda(), "scales must be device tensors");
@@ -165,7 +174,7 @@ Tensor gemm(Tensor a, Tensor w, Tensor sx, Tensor sw, const Tensor &bias_in, int
     c10::DeviceGuard guard(a.device());
     sx = scales_in(sx);
     sw = scales_in(sw);
-    const bool worth = K > 0 && (tiled || (double)M * (double)N * (double)K >= (double)kPadMinWork);
+    const bool worth = K > 0 && !small_product(M, N, K);
     if (block > 128 && (block & (block - 1)) == 0 && worth) {
         sx = sx.repeat_interleave(block / 128, 0).slice(0, 0, ceil_div(K, 128)).contiguous();
         sw = sw.repeat_interleave(block / 128, 0).slice(0, 0, ceil_div(K, 128)).contiguous();
@@ -252,6 +261,13 @@ std::pair<Tensor, Tensor> padded_operand(const Tensor &w, const Tensor &state, i
 // y = a @ w.T on codes that are a packed operand and a ready one (or any, which is then copied)
 void multiply_ready(const Packed &aq, const Tensor &t, const Tensor &w, const Tensor &state, int64_t contraction, const Bias &bias, const Tensor &out, int64_t M, int64_t N,
                     int64_t block, void *ws, int64_t need, void *stream) {
+    const Tensor rows = rows_of(w);
+    if (!pad_contraction(M, N, contraction, block) || (small_product(M, N, contraction) && (ld_of(rows) % 16 != 0 || (uintptr_t)rows.data_ptr() % 16 != 0))) {
+        const Tensor s = scales_in(state);
+        return check(gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)rows.data_ptr(), (const float *)s.data_ptr(), ld_of(rows), bias, out.data_ptr(), float_code(out),
+                              M, N, contraction, contraction, block, nullptr, 0, stream),
+                     "bi8x_gemm");
+    }
     if (ready_operand(w, state, contraction, block)) {
         const int rc = gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)w.data_ptr(), (const float *)state.data_ptr(), ld_of(w), bias, out.data_ptr(), float_code(out), M,
                                 N, aq.ld, up(contraction, 16), block, ws, need, stream);
@@ -289,7 +305,8 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
     if (fast_block(B) && M > 0 && N > 0 && K > 0) {
         // one allocation for what does not outlive the call
         const Packed xq = pack(M, K, B), wq = pack(w.defined() ? N : 0, K, B, xq.end()), xtq = pack(K, M, B), wtq = pack(K, N, B);
-        const int64_t kp = xq.ld, need = scratch_for(M, N, kp, B), ws_at = wq.end();
+        const bool pad = pad_contraction(M, N, K, B);
+        const int64_t kp = pad ? xq.ld : K, need = pad ? scratch_for(M, N, kp, B) : 0, ws_at = wq.end();
         const Tensor t = empty({ws_at + need}, at::kByte, x);
         if (need_xt) xt.codes = empty({xtq.end()}, at::kByte, x);
         if (need_wt) wt.codes = empty({wtq.end()}, at::kByte, x);
@@ -318,7 +335,7 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
         const Bias bias(bias_in, N);
         void *const ws = need > 0 ? (uint8_t *)t.data_ptr() + ws_at : nullptr;
         if (w.defined()) {
-            check(gemm_raw(xq.codes(t), xq.scales(t), kp, wq.codes(t), wq.scales(t), kp, bias, out.data_ptr(), float_code(out), M, N, kp, kp, B, ws, need, stream), "bi8x_gemm");
+            check(gemm_raw(xq.codes(t), xq.scales(t), xq.ld, wq.codes(t), wq.scales(t), wq.ld, bias, out.data_ptr(), float_code(out), M, N, kp, kp, B, ws, need, stream), "bi8x_gemm");
         } else {
             multiply_ready(xq, t, w_int8, w_state, K, bias, out, M, N, B, ws, need, stream);
         }
@@ -337,7 +354,7 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
         std::tie(wt.codes, wt.scales) = quantize_transposed(w, B, cfg.scale_type);
         wt.packed = false;
     }
-    return gemm(xq, rows_of(wq), xs, ws, bias_in, B, cfg.out_type, true).view(with_last(x_in, N));
+    return gemm(xq, rows_of(wq), xs, ws, bias_in, B, cfg.out_type).view(with_last(x_in, N));
 }
 
 struct LinearBackward : public torch::autograd::Node {
@@ -390,7 +407,8 @@ struct LinearBackward : public torch::autograd::Node {
             const Packed gq = pack(need_gx ? M : 0, N, B), gtq = pack(need_gw ? N : 0, M, B, gq.end());
             const bool both = need_gx && need_gw, sums = both && need_gb;
             const int64_t part_at = gtq.end(), ws_at = up(part_at + (sums ? bi8_colsum_workspace_bytes(M, N) : 0), 256);
-            const int64_t need1 = need_gx ? scratch_for(M, K, gq.ld, B) : 0, need2 = need_gw ? scratch_for(N, K, gtq.ld, B) : 0;
+            const int64_t kx = pad_contraction(M, K, N, B) ? gq.ld : N, kw = pad_contraction(N, K, M, B) ? gtq.ld : M;      // the contractions as multiplied
+            const int64_t need1 = need_gx && kx == gq.ld ? scratch_for(M, K, kx, B) : 0, need2 = need_gw && kw == gtq.ld ? scratch_for(N, K, kw, B) : 0;
             const Tensor t = empty({ws_at + std::max(need1, need2)}, at::kByte, G);
             uint8_t *const base = (uint8_t *)t.data_ptr();
             if (both) {
@@ -410,7 +428,7 @@ struct LinearBackward : public torch::autograd::Node {
                 Tensor gx = empty(x_sizes, cfg.out_type, G);
                 void *const ws = need1 > 0 ? base + ws_at : nullptr;
                 if (wt_packed) {
-                    check(gemm_raw(gq.codes(t), gq.scales(t), gq.ld, wtq.codes(held[2]), wtq.scales(held[2]), wtq.ld, none, gx.data_ptr(), float_code(gx), M, K, gq.ld, gq.ld, B,
+                    check(gemm_raw(gq.codes(t), gq.scales(t), gq.ld, wtq.codes(held[2]), wtq.scales(held[2]), wtq.ld, none, gx.data_ptr(), float_code(gx), M, K, kx, kx, B,
                                    ws, need1, stream),
                           "bi8x_gemm");
                 } else {
@@ -420,8 +438,8 @@ struct LinearBackward : public torch::autograd::Node {
             }
             if (need_gw) {
                 Tensor gw = empty({N, K}, cfg.out_type, G);
-                check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, gtq.ld,
-                               gtq.ld, B, need2 > 0 ? base + ws_at : nullptr, need2, stream),
+                check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, kw, kw, B,
+                               need2 > 0 ? base + ws_at : nullptr, need2, stream),
                       "bi8x_gemm");
                 result[1] = gw;
             }
@@ -433,11 +451,11 @@ struct LinearBackward : public torch::autograd::Node {
         } else {
             if (need_gx) {
                 auto [q, s] = quantize_rowwise(G, B, cfg.scale_type);
-                result[0] = gemm(q, rows_of(held[2]), s, held[3], Tensor(), B, cfg.out_type, true).view(x_sizes);
+                result[0] = gemm(q, rows_of(held[2]), s, held[3], Tensor(), B, cfg.out_type).view(x_sizes);
             }
             if (need_gw) {
                 auto [q, s] = quantize_transposed(G, B, cfg.scale_type);
-                result[1] = gemm(q, held[0], s, held[1], Tensor(), B, cfg.out_type, true);
+                result[1] = gemm(q, held[0], s, held[1], Tensor(), B, cfg.out_type);
             }
         }
         if (need_gb && !result[2].defined()) {
@@ -617,7 +635,7 @@ PyObject *py_gemm(PyObject *, PyObject *const *v, Py_ssize_t n) {               
         const ScalarType ot = a.dtype(6);
         return wrapped(without_gil([&] {
             at::AutoGradMode no_grad(false);
-            return gemm(rows_of(A), rows_of(b.t()), sx, sw, bias, block, ot, false, scratch);
+            return gemm(rows_of(A), rows_of(b.t()), sx, sw, bias, block, ot, scratch);
         }));
     });
 }

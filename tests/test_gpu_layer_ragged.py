@@ -65,3 +65,47 @@ def test_layer_is_the_composition_of_its_operators(case, scale_type):
             ref = oracle_torch.int8_matmul_block_dequantize(xq.cpu(), wq.cpu(), xs.cpu(), ws.cpu(), block, b.detach().cpu(), DTYPES[xt])
             unit = {"f32": 4e-6, "bf16": 1.6e-2, "f16": 2e-3}[xt]        # the product's and the sum's rounding at the largest magnitude
             assert (y.detach().cpu().double() - ref.double()).abs().max() <= unit * ref.double().abs().max()
+
+
+# (rows, in, out): fewer than 2^22 multiplications in every product, contractions that are no multiples of 128
+SMALL = [(70, 192, 130), (100, 64, 64), (500, 72, 100), (20, 320, 400), (5, 200, 300), (1, 192, 130)]
+
+
+@pytest.mark.parametrize("block", [32, 64, 128])
+@pytest.mark.parametrize("case", SMALL, ids=lambda c: "x".join(map(str, c)))
+def test_small_products_take_the_scales_as_they_are(case, block):
+    """An infinite column scale gives infinities, not a column of NaN, and the column scales are not rounded: fp32 results within three
+    roundings of their products and sums (2-norm: 2^-24 each at most, rms less than half of that) plus one per K-block."""
+    import blockwise_int8_linear_amd as pkg
+    M, K, N = case
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g).to(DEV).requires_grad_(True)
+    w = (torch.randn(N, K, generator=g) * 0.05).to(DEV).requires_grad_(True)
+    G = torch.randn(M, N, generator=g).to(DEV)
+
+    def exact(a, sa, b, sb):
+        out = 0
+        for j in range(sa.shape[0]):
+            cols = slice(j * block, (j + 1) * block)
+            out = out + (a[:, cols].double() @ b[:, cols].double().t()) * sa[j].double()[:, None] * sb[j].double()[None, :]
+        return out / 127.0 ** 2
+
+    with config_as(pkg, block, torch.float32):
+        mul, q, qt = pkg.int8_matmul_block64_rowwise_dequantize, pkg.quantize_block_rowwise, pkg.quantize_block_transposed
+        y = pkg.blockwise_int8_linear.apply(x, w, None)
+        y.backward(G)
+        with torch.no_grad():
+            (xq, xs), (wq, ws), (gq, gs) = q(x), q(w), q(G)
+            (xtq, xts), (wtq, wts), (gtq, gts) = qt(x), qt(w), qt(G)
+            products = ((y.detach(), (xq, xs, wq, ws)), (x.grad, (gq, gs, wtq, wts)), (w.grad, (gtq, gts, xtq, xts)))
+            for got, (a, sa, b, sb) in products:
+                want = exact(a, sa, b, sb)
+                assert (got.double() - want).norm() <= 0.5 * (3 + sa.shape[0]) * 2.0 ** -24 * want.norm()
+                if a.shape[0] > 64:
+                    assert torch.equal(got, mul(a, b.t(), sa, sb))
+            ws = ws.clone()
+            ws[-1, 2] = float("inf")
+            ref = oracle_torch.int8_matmul_block_dequantize(xq.cpu(), wq.cpu(), xs.cpu(), ws.cpu(), block, None, torch.float32)
+            assert ref[:, 2].isinf().any()
+            got = pkg.blockwise_int8_linear_Wint8.apply(x.detach(), wq, ws, None, wtq, wts).cpu()
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
