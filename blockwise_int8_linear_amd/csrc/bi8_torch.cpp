@@ -247,33 +247,29 @@ void quantize_rows(const Tensor &x, const Tensor &t, const Packed &q, const Conf
     round_scales(t, q, cfg.scale_type);
 }
 
-// Codes of a weight made ahead of the call, int8 [N,K] with scales [ceil(K/block), N], as a GEMM operand that only A is padded for.
-bool ready_operand(const Tensor &w, const Tensor &state, int64_t contraction, int64_t block) {
-    return fast_block(block) && (contraction % 128 == 0 || block != 32) && (w.stride(1) == 1 || w.size(1) == 1) && ld_of(w) % 16 == 0 && ld_of(w) >= contraction &&
-           (uintptr_t)w.data_ptr() % 16 == 0 && whole_chunks(w, contraction) && state.scalar_type() == at::kFloat && state.is_contiguous();
+// Codes of a weight made ahead of the call, int8 [N,K] with contiguous rows, as a GEMM operand that only A is padded for.
+bool ready_operand(const Tensor &w, int64_t contraction, int64_t block) {
+    return fast_block(block) && (contraction % 128 == 0 || block != 32) && ld_of(w) % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0 && whole_chunks(w, contraction);
 }
 // ... and the copy of one that is none, padded itself
-std::pair<Tensor, Tensor> padded_operand(const Tensor &w, const Tensor &state, int64_t contraction, int64_t block) {
-    const int64_t kp = up(contraction, 128), extra = kp / block - state.size(0);
-    const Tensor s = scales_in(state);
+std::pair<Tensor, Tensor> padded_operand(const Tensor &w, const Tensor &s, int64_t contraction, int64_t block) {
+    const int64_t kp = up(contraction, 128), extra = kp / block - s.size(0);
     return {at::constant_pad_nd(w, {0, kp - contraction}).contiguous(), extra > 0 ? at::constant_pad_nd(s, {0, 0, 0, extra}) : s};
 }
 // y = a @ w.T on codes that are a packed operand and a ready one (or any, which is then copied)
-void multiply_ready(const Packed &aq, const Tensor &t, const Tensor &w, const Tensor &state, int64_t contraction, const Bias &bias, const Tensor &out, int64_t M, int64_t N,
+void multiply_ready(const Packed &aq, const Tensor &t, const Tensor &w_in, const Tensor &state, int64_t contraction, const Bias &bias, const Tensor &out, int64_t M, int64_t N,
                     int64_t block, void *ws, int64_t need, void *stream) {
-    const Tensor rows = rows_of(w);
-    if (!pad_contraction(M, N, contraction, block) || (small_product(M, N, contraction) && (ld_of(rows) % 16 != 0 || (uintptr_t)rows.data_ptr() % 16 != 0))) {
-        const Tensor s = scales_in(state);
-        return check(gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)rows.data_ptr(), (const float *)s.data_ptr(), ld_of(rows), bias, out.data_ptr(), float_code(out),
+    const Tensor w = rows_of(w_in), s = scales_in(state);      // (scales kept in another type are converted, the codes are not touched)
+    if (!pad_contraction(M, N, contraction, block) || (small_product(M, N, contraction) && (ld_of(w) % 16 != 0 || (uintptr_t)w.data_ptr() % 16 != 0)))
+        return check(gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)w.data_ptr(), (const float *)s.data_ptr(), ld_of(w), bias, out.data_ptr(), float_code(out),
                               M, N, contraction, contraction, block, nullptr, 0, stream),
                      "bi8x_gemm");
-    }
-    if (ready_operand(w, state, contraction, block)) {
-        const int rc = gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)w.data_ptr(), (const float *)state.data_ptr(), ld_of(w), bias, out.data_ptr(), float_code(out), M,
+    if (ready_operand(w, contraction, block)) {
+        const int rc = gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)w.data_ptr(), (const float *)s.data_ptr(), ld_of(w), bias, out.data_ptr(), float_code(out), M,
                                 N, aq.ld, up(contraction, 16), block, ws, need, stream);
         if (rc != BI8_ERR_UNSUPPORTED) return check(rc, "bi8x_gemm");    // (rows too far apart for the kernels' 32-bit offsets: copied)
     }
-    const auto [wp, sp] = padded_operand(w, state, contraction, block);
+    const auto [wp, sp] = padded_operand(w, s, contraction, block);
     check(gemm_raw(aq.codes(t), aq.scales(t), aq.ld, (const int8_t *)wp.data_ptr(), (const float *)sp.data_ptr(), aq.ld, bias, out.data_ptr(), float_code(out), M, N, aq.ld, aq.ld,
                    block, ws, need, stream),
           "bi8x_gemm");

@@ -109,3 +109,25 @@ def test_small_products_take_the_scales_as_they_are(case, block):
             assert ref[:, 2].isinf().any()
             got = pkg.blockwise_int8_linear_Wint8.apply(x.detach(), wq, ws, None, wtq, wts).cpu()
         assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+
+
+@pytest.mark.parametrize("kept", [False, True], ids=["evaluation", "kept_codes"])
+def test_scales_of_another_type_leave_the_weight_codes_where_they_are(kept):
+    """the scales are converted for the call, the codes (the layer's memory) are not copied"""
+    import blockwise_int8_linear_amd as pkg
+    with config_as(pkg, 64, torch.bfloat16):
+        cfg = pkg.block_linear_config
+        cfg.SHARED_EXP_TORCH_TYPE = torch.bfloat16
+        try:
+            K, N = 2048, 4096
+            lin = pkg.BlockInt8Linear(K, N, False, DEV, torch.bfloat16, quantized_weight_training=kept).train(kept)
+            x = torch.randn(24, K, device=DEV, dtype=torch.bfloat16)
+            with torch.no_grad():
+                lin(x)
+                torch.cuda.synchronize()
+                torch.cuda.reset_peak_memory_stats()
+                before = torch.cuda.memory_allocated()
+                lin(x)
+            assert torch.cuda.max_memory_allocated() - before < N * K // 2
+        finally:
+            cfg.SHARED_EXP_TORCH_TYPE = torch.float32
