@@ -499,7 +499,7 @@ Tensor few_rows(const Tensor &x_in, const Tensor &w, const Tensor &state, const 
         w.dim() != 2 || w.stride(1) != 1 || x_in.size(-1) != w.size(1) || state.dim() != 2 || state.size(1) != w.size(0) || state.size(0) != ceil_div(w.size(1), block))
         return Tensor();
     require(x_in.is_cuda() && w.is_cuda() && state.is_cuda(), "operands must be device tensors");
-    const Tensor x = x_in.dim() == 2 && (x_in.stride(1) == 1) ? x_in : matrix_of(x_in);
+    const Tensor x = matrix_of(x_in);              // (also rows that overlap, an expanded row for instance, become rows)
     const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
     if (M < 1 || M > 2 || (block != 64 && block != 128) || K % 128 != 0 || N < 1 || K < 1) return Tensor();
     c10::DeviceGuard guard(x.device());

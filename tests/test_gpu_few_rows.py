@@ -136,3 +136,12 @@ def test_module_decode_uses_it_and_matches_prefill_rows(pkg):
         assert one.shape == (1, 1, N)
         assert torch.equal(one.view(-1), two.view(-1))
         assert torch.allclose(one.float().view(-1), full[1, 7].float(), rtol=2e-2, atol=1e-3)
+
+
+@pytest.mark.parametrize("strides", [(0, 1), (128, 1)], ids=["expanded_row", "overlapping_rows"])
+def test_rows_that_share_memory(pkg, strides):
+    """two rows of one stretch of memory (an expanded row, a sliding window) give what their copies give"""
+    with cfg_as(pkg, 128, torch.bfloat16), torch.no_grad():
+        lin = pkg.BlockInt8Linear(256, 96, True, DEV, torch.bfloat16).eval()
+        x = torch.randn(384, device=DEV).to(torch.bfloat16).as_strided((2, 256), strides)
+        assert torch.equal(lin(x), lin(x.contiguous()))
