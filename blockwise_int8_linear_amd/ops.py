@@ -173,15 +173,13 @@ def int8_matmul_block64_rowwise_dequantize(a, b, state_x, state_w, bias=None):
 
 
 _ws_need = {}                       # (M, N, K, block) -> bytes of scratch memory the library's split of K wants (0: none)
-_ws_held = {}                       # (device index, stream) -> uint8 tensor, grown on demand
 
 
 def _workspace(lib, M, N, K, block, device, stream):
     """Scratch memory for a GEMM of fewer output tiles than compute units (the library then splits K over the
-    workgroups and sums the pieces): (tensor or None, bytes).  What a shape wants is asked once; the memory is one
-    tensor per device and stream, kept for the life of the process (at most 32 MiB each) and shared by the GEMMs of
-    that stream, which run one after the other.  While the stream is being captured into a graph the memory comes from
-    the capture's own pool instead, so that graphs replayed side by side do not share it.
+    workgroups and sums the pieces): (tensor or None, bytes).  What a shape wants is asked once; the memory (at most 32 MiB) is
+    the call's own, from torch's allocator on the current stream: the split and its sum are two launches, and those of two
+    threads that use one stream may be queued in between one another.
     (Up to 16 rows at blocks 64 / 128 run the one-pass decode kernels whatever they are given: not asked.)"""
     if M <= 16 and block != 32:
         return None, 0
@@ -189,16 +187,7 @@ def _workspace(lib, M, N, K, block, device, stream):
     need = _ws_need.get(key)
     if need is None:
         need = _ws_need[key] = lib.bi8_gemm_workspace_bytes(M, N, K, block)
-    if not need:
-        return None, 0
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(need, device=device, dtype=torch.uint8), need
-    held = _ws_held.get((device.index, stream))
-    if held is None or held.numel() < need:
-        # (allocated on the current stream, which is `stream`: torch's allocator orders a later reuse of a replaced
-        # tensor's memory behind the work already queued there)
-        held = _ws_held[(device.index, stream)] = torch.empty(need, device=device, dtype=torch.uint8)
-    return held, need
+    return (torch.empty(need, device=device, dtype=torch.uint8), need) if need else (None, 0)
 
 
 _FEW_ROWS = 2

@@ -340,6 +340,14 @@ def test_kernel_choice_by_shape():
     assert asked == [(17, 4096, 11008, 128)]
 
 
+def test_every_gemm_has_scratch_memory_of_its_own():
+    """a split of K and its sum are two launches: two threads that queue them on one stream must not share the memory between"""
+    from blockwise_int8_linear_amd import ops
+    held = [ops._workspace(_lib.load(), 100, 4096, 11008, 128, torch.device("cpu"), 0) for _ in range(2)]
+    assert held[0][1] > 0 and held[0][1] == held[1][1] == held[0][0].numel()
+    assert held[0][0].data_ptr() != held[1][0].data_ptr()
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="made-up addresses: the answer has to come from the host")
 def test_an_unpadded_w_is_refused_by_kernels_that_gather_it():
     """gemm_generic and gemm_skinny read W without a range check: a W whose rows end before the padded contraction does is copied
