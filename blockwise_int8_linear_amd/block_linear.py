@@ -104,7 +104,7 @@ class blockwise_int8_linear(torch.autograd.Function):
     The backward pass needs X and W quantized along the other direction (blocks over the tokens for grad_W, over the
     output features for grad_X; block_linear.py:93-94, :100-103).  Those codes are produced in the forward pass by the
     same read of X and W and saved in place of X and W; the numbers are the ones the reference computes from the saved X
-    and W in its backward.  Forward and backward are native code (``LinearBackward`` in csrc/bi8_torch.cpp)."""
+    and W in its backward.  Forward and backward are native code (``BlockInt8LinearFunction`` in csrc/bi8_torch.cpp)."""
 
     @classmethod
     def apply(cls, X_3D, W, bias):
@@ -245,12 +245,16 @@ class BlockInt8Linear(nn.Linear):
     def forward(self, x):
         if not self.training:
             return self.infer(x)
+        # (read directly, as in infer(); a weight that is no parameter of its own -- parametrized, replaced -- is an attribute)
+        params = self._parameters
+        weight = params["weight"] if "weight" in params else self.weight
+        bias = params["bias"] if "bias" in params else self.bias
         if self.quantized_weight_training:
             if self._train_cache is None or self._train_cache[0] != self._weight_state():
                 self.prepare_for_quantized_weight_training()
             _, W_int8, state_W, Wt_int8, Wt_state, Wt_store = self._train_cache
-            return blockwise_int8_linear_Wint8.apply(x, W_int8, state_W, self.bias, Wt_int8, Wt_state, self.weight, Wt_store)
-        return blockwise_int8_linear.apply(x, self.weight, self.bias)
+            return blockwise_int8_linear_Wint8.apply(x, W_int8, state_W, bias, Wt_int8, Wt_state, weight, Wt_store)
+        return blockwise_int8_linear.apply(x, weight, bias)
 
     def train(self, mode: bool = True):
         if mode and "W_int8" in self._buffers:

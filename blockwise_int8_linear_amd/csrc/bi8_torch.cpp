@@ -15,10 +15,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
-#include <torch/csrc/autograd/function.h>
-#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
-#include <torch/csrc/autograd/saved_variable.h>
 
 #include "bi8_internal.h"
 
@@ -353,41 +351,46 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
     return gemm(xq, rows_of(wq), xs, ws, bias_in, B, cfg.out_type).view(with_last(x_in, N));
 }
 
-struct LinearBackward : public torch::autograd::Node {
+// What a call multiplies x with: the float weight, or its codes made ahead; and the bias, if any.
+struct Operands {
     Config cfg;
-    int64_t M = 0, K = 0, N = 0;
-    std::vector<int64_t> x_sizes;
-    torch::autograd::SavedVariable saved[4];       // codes and scales of X transposed, of W transposed
-    bool has_xt = false, xt_packed = true, has_wt = false, wt_packed = true;
+    Tensor w, w_int8, w_state, bias;
+    Kept wt_ready;
+    bool need_gx = false, need_gw = false;
+};
 
-    std::string name() const override { return "BlockInt8LinearBackward"; }
-    void keep(const Kept &xt, const Kept &wt) {
-        has_xt = xt.codes.defined();
-        has_wt = wt.codes.defined();
-        xt_packed = xt.packed;
-        wt_packed = wt.packed;
-        const Tensor *t[4] = {&xt.codes, &xt.scales, &wt.codes, &wt.scales};
-        for (int i = 0; i < 4; ++i)
-            if (t[i]->defined()) saved[i] = torch::autograd::SavedVariable(*t[i], false);
-    }
-    void release_variables() override {
-        std::lock_guard<std::mutex> lock(mutex_);
-        for (auto &v : saved) v.reset_data();
+// The differentiable layer: autograd's inputs are x, the tensor that receives grad_W (the float weight itself, or what stands for
+// it where its codes come ready) and the bias; an empty tensor where there is none.  torch's C++ form of an autograd function: saved-tensor hooks, retained and
+// freed graphs, materialized zeros and compiled autograd are torch's own.
+struct BlockInt8LinearFunction : public torch::autograd::Function<BlockInt8LinearFunction> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &, const Tensor &, const Operands &op) {
+        Kept xt, wt;
+        const Tensor out = linear_forward(x, op.w, op.w_int8, op.w_state, op.bias, op.cfg, op.need_gw, op.need_gx && op.w.defined(), xt, wt);
+        if (op.need_gx && !op.w.defined()) wt = op.wt_ready;
+        int64_t m = 1;
+        for (int64_t d = 0; d + 1 < x.dim(); ++d) m *= x.size(d);
+        torch::autograd::variable_list kept(4);
+        kept[0] = std::move(xt.codes);
+        kept[1] = std::move(xt.scales);
+        kept[2] = std::move(wt.codes);
+        kept[3] = std::move(wt.scales);
+        const bool wt_packed = wt.packed;
+        ctx->save_for_backward(std::move(kept));
+        std::vector<int64_t> of = {m, x.size(-1), out.size(-1), op.cfg.block, (int64_t)op.cfg.out_type, (int64_t)op.cfg.scale_type, wt_packed};
+        of.insert(of.end(), x.sizes().begin(), x.sizes().end());
+        ctx->saved_data["of"] = std::move(of);
+        return out;
     }
     // grad_X [M,K] = G [M,N] @ W [N,K], contracted over N; grad_W [N,K] = G.T [N,M] @ X [M,K], contracted over the rows
-    // (block_linear.py:88-112); grad_bias = the column sums of G.  Outputs: x, weight, bias.
-    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
-        torch::autograd::variable_list result(3);
-        // (no gradient reached the output: zeros, as an autograd function of torch gets them)
-        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
-        Tensor held[4];
-        {
-            std::lock_guard<std::mutex> lock(mutex_);
-            const bool used[4] = {has_xt, has_xt && !xt_packed, has_wt, has_wt && !wt_packed};
-            for (int i = 0; i < 4; ++i)
-                if (used[i]) held[i] = saved[i].unpack(shared_from_this());
-        }
-        const bool need_gx = has_wt && task_should_compute_output(0), need_gw = has_xt && task_should_compute_output(1), need_gb = task_should_compute_output(2);
+    // (block_linear.py:88-112); grad_bias = the column sums of G.
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        torch::autograd::variable_list result(4);
+        const torch::autograd::variable_list held = ctx->get_saved_variables();
+        const std::vector<int64_t> of = ctx->saved_data["of"].toIntVector(), x_sizes(of.begin() + 7, of.end());
+        const int64_t M = of[0], K = of[1], N = of[2];
+        const Config cfg{of[3], (ScalarType)of[4], (ScalarType)of[5]};
+        const bool wt_packed = of[6] != 0;
+        const bool need_gx = held[2].defined() && ctx->needs_input_grad(0), need_gw = held[0].defined() && ctx->needs_input_grad(1), need_gb = ctx->needs_input_grad(2);
         const bool graph = at::GradMode::is_enabled();
         at::AutoGradMode no_grad(false);
         const Tensor &G_in = grads[0];
@@ -462,35 +465,20 @@ struct LinearBackward : public torch::autograd::Node {
     }
 };
 
-// The differentiable layer: autograd's inputs are x, `stands_for_w` (the tensor that receives grad_W: the float weight itself, or what
-// stands for it where its codes come ready) and the bias.
-Tensor linear_apply(const Tensor &x, const Tensor &w, const Tensor &w_int8, const Tensor &w_state, const Tensor &stands_for_w, const Kept &wt_ready, const Tensor &bias,
-                    const Config &cfg) {
+Tensor linear_apply(const Tensor &x, const Tensor &stands_for_w, Operands op) {
+    static const Tensor *const none = new Tensor(at::empty({0}));
     require(x.is_cuda(), "x must be a device tensor");
-    for (const Tensor *t : {&x, &w, &stands_for_w, &bias})
+    for (const Tensor *t : {&x, &std::as_const(op.w), &stands_for_w, &std::as_const(op.bias)})
         TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), "blockwise_int8_linear has no forward-mode derivative");
     const bool grad = at::GradMode::is_enabled();
-    const bool need_gx = grad && x.requires_grad(), need_gw = grad && stands_for_w.defined() && stands_for_w.requires_grad(), need_gb = grad && bias.defined() && bias.requires_grad();
+    op.need_gx = grad && x.requires_grad();
+    op.need_gw = grad && stands_for_w.defined() && stands_for_w.requires_grad();
     c10::DeviceGuard guard(x.device());
+    if (op.need_gx || op.need_gw || (grad && op.bias.defined() && op.bias.requires_grad()))
+        return BlockInt8LinearFunction::apply(x, stands_for_w.defined() ? stands_for_w : *none, op.bias.defined() ? op.bias : *none, op);
+    at::AutoGradMode no_grad(false);
     Kept xt, wt;
-    Tensor out;
-    {
-        at::AutoGradMode no_grad(false);
-        out = linear_forward(x, w, w_int8, w_state, bias, cfg, need_gw, need_gx && w.defined(), xt, wt);
-    }
-    if (need_gx || need_gw || need_gb) {
-        std::shared_ptr<LinearBackward> node(new LinearBackward(), torch::autograd::deleteNode);
-        node->set_next_edges(torch::autograd::collect_next_edges(x, stands_for_w, bias));
-        node->cfg = cfg;
-        node->K = x.size(-1);
-        node->N = out.size(-1);
-        node->M = 1;
-        for (int64_t d = 0; d + 1 < x.dim(); ++d) node->M *= x.size(d);
-        node->x_sizes.assign(x.sizes().begin(), x.sizes().end());
-        node->keep(xt, w.defined() || !need_gx ? wt : wt_ready);
-        torch::autograd::set_history(out, node);
-    }
-    return out;
+    return linear_forward(x, op.w, op.w_int8, op.w_state, op.bias, op.cfg, false, false, xt, wt);
 }
 
 // Quantize + GEMM in one launch for one or two rows, where the library covers it (bi8_linear_few_rows); undefined otherwise.
@@ -639,7 +627,7 @@ PyObject *py_linear(PyObject *, PyObject *const *v, Py_ssize_t n) {             
     return guarded("linear", 6, v, n, [](Args a) {
         const Tensor x = a.tensor(0), w = a.tensor(1), bias = a.optional_tensor(2);
         const Config cfg{a.block(3), a.dtype(4), a.dtype(5)};
-        return wrapped(without_gil([&] { return linear_apply(x, w, Tensor(), Tensor(), w, Kept(), bias, cfg); }));
+        return wrapped(without_gil([&] { return linear_apply(x, w, Operands{cfg, w, Tensor(), Tensor(), bias, Kept()}); }));
     });
 }
 // x, W codes, W scales, bias, transposed W codes, their scales, weight or None, block, output dtype, scale dtype
@@ -653,7 +641,7 @@ PyObject *py_linear_kept(PyObject *, PyObject *const *v, Py_ssize_t n) {
         const Config cfg{a.block(7), a.dtype(8), a.dtype(9)};
         return wrapped(without_gil([&] {
             check_codes(wt.codes, wt.scales, wq.size(0), cfg.block);
-            return linear_apply(x, Tensor(), wq, ws, weight, wt, bias, cfg);
+            return linear_apply(x, weight, Operands{cfg, Tensor(), wq, ws, bias, wt});
         }));
     });
 }

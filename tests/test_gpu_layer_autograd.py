@@ -66,6 +66,17 @@ def test_a_trace_records_the_call(layer):
     assert torch.equal(traced(other), layer(other))
 
 
+def test_compiled_autograd(layer):
+    from torch._dynamo import compiled_autograd
+    enable = getattr(compiled_autograd, "_enable", None) or compiled_autograd.enable
+    x, g = torch.randn(70, 192, device=DEV), torch.randn(70, 130, device=DEV)
+    want = _grads(layer, x, g)
+    for _ in range(2):
+        with enable(torch.compile(backend="eager")):
+            got = _grads(layer, x, g)
+        assert all(map(torch.equal, got, want))
+
+
 def test_refused_transforms(layer):
     x = torch.randn(3, 7, 192, device=DEV)
     with pytest.raises(RuntimeError):
