@@ -81,6 +81,7 @@ def _forward_kept(ctx, call, tensors):
     trace = torch._C._get_tracing_state()
     torch._C._set_tracing_state(None)
     try:
+        ctx.save_for_backward(X.new_empty(0))      # (nothing of use: reading it fails once the graph is freed, as it does for any function)
         ctx.inputs = [t.detach().requires_grad_(need) if isinstance(t, torch.Tensor) else t for t, need in zip(tensors, ctx.needs_input_grad)]
         with torch.enable_grad():
             ctx.output = call(*ctx.inputs)
@@ -90,8 +91,10 @@ def _forward_kept(ctx, call, tensors):
 
 
 def _backward_kept(ctx, G):
+    ctx.saved_tensors
     at = [i for i, need in enumerate(ctx.needs_input_grad) if need]
-    grads = torch.autograd.grad(ctx.output, [ctx.inputs[i] for i in at], G, allow_unused=True)
+    # (whether the outer graph is retained is not known here: the native one lives as long as ctx does)
+    grads = torch.autograd.grad(ctx.output, [ctx.inputs[i] for i in at], G, allow_unused=True, retain_graph=True)
     result = [None] * len(ctx.needs_input_grad)
     for i, grad in zip(at, grads):
         result[i] = grad

@@ -77,6 +77,33 @@ def test_compiled_autograd(layer):
         assert all(map(torch.equal, got, want))
 
 
+@pytest.mark.parametrize("traced", [False, True], ids=["eager", "traced"])
+def test_a_graph_is_retained_where_that_is_asked_for(layer, traced):
+    x, g = torch.randn(70, 192, device=DEV, requires_grad=True), torch.randn(70, 130, device=DEV)
+    if layer.quantized_weight_training:
+        layer.prepare_for_quantized_weight_training()
+    seen = []
+
+    class Keeps(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.layer = layer
+
+        def forward(self, x):
+            seen.append(self.layer(x))
+            return seen[0]
+    if traced:
+        torch.jit.trace(Keeps(), x, check_trace=False)
+    else:
+        Keeps()(x)
+    inputs = (x, layer.weight, layer.bias)
+    first = torch.autograd.grad(seen[0], inputs, g, retain_graph=True)
+    second = torch.autograd.grad(seen[0], inputs, g)
+    assert all(map(torch.equal, first, second)) and torch.equal(first[0], _grads(layer, x, g)[1])
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(seen[0], inputs, g)
+
+
 def test_refused_transforms(layer):
     x = torch.randn(3, 7, 192, device=DEV)
     with pytest.raises(RuntimeError):
