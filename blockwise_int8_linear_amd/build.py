@@ -10,7 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 
 
 def build(force: bool = False, jobs: int = 8, quiet: bool = True) -> str:
-    cmd = ["make", "-C", CSRC, f"-j{jobs}"] + (["-B"] if force else [])
+    cmd = ["make", "-C", CSRC, f"-j{jobs}", f"PYTHON={sys.executable}"] + (["-B"] if force else [])
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0 or not quiet:
         # hipcc's host pass prints a harmless note about the packed-fp32 feature flag
