@@ -68,10 +68,13 @@ def _count_optimizer_step(optimizer, args, kwargs):
 register_optimizer_step_post_hook(_count_optimizer_step)
 
 
+_tracing_state, _transforms_active = torch._C._get_tracing_state, torch._C._are_functorch_transforms_active
+
+
 def _as_function():
     """Whether a call has to go through ``torch.autograd.Function`` itself: a trace records it as one node (a native call would
     leave its result in the trace as a constant), and torch.func's transforms refuse it there."""
-    return torch._C._get_tracing_state() is not None or torch._C._are_functorch_transforms_active()
+    return _tracing_state() is not None or _transforms_active()
 
 
 def _forward_kept(ctx, call, tensors):
@@ -107,7 +110,7 @@ class blockwise_int8_linear(torch.autograd.Function):
     The backward pass needs X and W quantized along the other direction (blocks over the tokens for grad_W, over the
     output features for grad_X; block_linear.py:93-94, :100-103).  Those codes are produced in the forward pass by the
     same read of X and W and saved in place of X and W; the numbers are the ones the reference computes from the saved X
-    and W in its backward.  Forward and backward are native code (``BlockInt8LinearFunction`` in csrc/bi8_torch.cpp)."""
+    and W in its backward.  Forward and backward are native code (``LinearBackward`` in csrc/bi8_torch.cpp)."""
 
     @classmethod
     def apply(cls, X_3D, W, bias):
@@ -195,7 +198,8 @@ class BlockInt8Linear(nn.Linear):
         assignments move the data, every ``torch.optim`` optimizer step anywhere in the process moves the step count
         (an optimizer that writes through ``p.data`` bumps no version), and ``invalidate_quantized_weight()`` covers
         the writes that none of these see (``p.data.copy_(ema)`` outside an optimizer)."""
-        w = self.weight
+        params = self._parameters                  # (read directly, as in forward())
+        w = params["weight"] if "weight" in params else self.weight
         return (w._version, w.data_ptr(), block_linear_config.GROUP_SIZE, _optimizer_steps[0], self._invalidations)
 
     def invalidate_quantized_weight(self):

@@ -16,6 +16,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "bi8_internal.h"
@@ -281,7 +282,7 @@ void check_codes(const Tensor &w, const Tensor &state, int64_t contraction, int6
 
 // What a forward pass keeps for the backward pass of X and of W: their codes along the other direction, [K,M] and [K,N].
 struct Kept {
-    Tensor codes, scales;              // packed: both in `codes`
+    Tensor codes, scales;              // packed: both in `codes`, W's behind X's in one tensor where both are kept
     bool packed = true;
 };
 
@@ -298,12 +299,13 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
 
     if (fast_block(B) && M > 0 && N > 0 && K > 0) {
         // one allocation for what does not outlive the call
-        const Packed xq = pack(M, K, B), wq = pack(w.defined() ? N : 0, K, B, xq.end()), xtq = pack(K, M, B), wtq = pack(K, N, B);
+        const Packed xq = pack(M, K, B), wq = pack(w.defined() ? N : 0, K, B, xq.end()), xtq = pack(K, M, B), wtq = pack(K, N, B, need_xt ? xtq.end() : 0);
         const bool pad = pad_contraction(M, N, K, B);
         const int64_t kp = pad ? xq.ld : K, need = pad ? scratch_for(M, N, kp, B) : 0, ws_at = wq.end();
         const Tensor t = empty({ws_at + need}, at::kByte, x);
-        if (need_xt) xt.codes = empty({xtq.end()}, at::kByte, x);
-        if (need_wt) wt.codes = empty({wtq.end()}, at::kByte, x);
+        // ... and one for what is kept
+        if (need_xt) xt.codes = empty({need_wt ? wtq.end() : xtq.end()}, at::kByte, x);
+        if (need_wt) wt.codes = need_xt ? xt.codes : empty({wtq.end()}, at::kByte, x);
         Bi8DualTask task[2];
         int n = 0;
         if (need_xt) task[n++] = dual_task(x, xt.codes, xq, t, xtq);
@@ -351,134 +353,200 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
     return gemm(xq, rows_of(wq), xs, ws, bias_in, B, cfg.out_type).view(with_last(x_in, N));
 }
 
-// What a call multiplies x with: the float weight, or its codes made ahead; and the bias, if any.
-struct Operands {
+// What a backward pass needs to know besides the codes: autograd's node keeps it.
+struct Shape {
     Config cfg;
-    Tensor w, w_int8, w_state, bias;
-    Kept wt_ready;
-    bool need_gx = false, need_gw = false;
+    int64_t M = 0, K = 0, N = 0;
+    std::vector<int64_t> x_sizes;
+    bool wt_packed = true, together = false;       // together: W's codes are behind X's in one tensor
 };
 
-// The differentiable layer: autograd's inputs are x, the tensor that receives grad_W (the float weight itself, or what stands for
-// it where its codes come ready) and the bias; an empty tensor where there is none.  torch's C++ form of an autograd function: saved-tensor hooks, retained and
-// freed graphs, materialized zeros and compiled autograd are torch's own.
-struct BlockInt8LinearFunction : public torch::autograd::Function<BlockInt8LinearFunction> {
-    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &, const Tensor &, const Operands &op) {
-        Kept xt, wt;
-        const Tensor out = linear_forward(x, op.w, op.w_int8, op.w_state, op.bias, op.cfg, op.need_gw, op.need_gx && op.w.defined(), xt, wt);
-        if (op.need_gx && !op.w.defined()) wt = op.wt_ready;
-        int64_t m = 1;
-        for (int64_t d = 0; d + 1 < x.dim(); ++d) m *= x.size(d);
-        torch::autograd::variable_list kept(4);
-        kept[0] = std::move(xt.codes);
-        kept[1] = std::move(xt.scales);
-        kept[2] = std::move(wt.codes);
-        kept[3] = std::move(wt.scales);
-        const bool wt_packed = wt.packed;
-        ctx->save_for_backward(std::move(kept));
-        std::vector<int64_t> of = {m, x.size(-1), out.size(-1), op.cfg.block, (int64_t)op.cfg.out_type, (int64_t)op.cfg.scale_type, wt_packed};
-        of.insert(of.end(), x.sizes().begin(), x.sizes().end());
-        ctx->saved_data["of"] = std::move(of);
-        return out;
-    }
-    // grad_X [M,K] = G [M,N] @ W [N,K], contracted over N; grad_W [N,K] = G.T [N,M] @ X [M,K], contracted over the rows
-    // (block_linear.py:88-112); grad_bias = the column sums of G.
-    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
-        torch::autograd::variable_list result(4);
-        const torch::autograd::variable_list held = ctx->get_saved_variables();
-        const std::vector<int64_t> of = ctx->saved_data["of"].toIntVector(), x_sizes(of.begin() + 7, of.end());
-        const int64_t M = of[0], K = of[1], N = of[2];
-        const Config cfg{of[3], (ScalarType)of[4], (ScalarType)of[5]};
-        const bool wt_packed = of[6] != 0;
-        const bool need_gx = held[2].defined() && ctx->needs_input_grad(0), need_gw = held[0].defined() && ctx->needs_input_grad(1), need_gb = ctx->needs_input_grad(2);
-        const bool graph = at::GradMode::is_enabled();
-        at::AutoGradMode no_grad(false);
-        const Tensor &G_in = grads[0];
-        require(G_in.is_cuda(), "the gradient must be a device tensor");
-        c10::DeviceGuard guard(G_in.device());
-        const Tensor G = matrix_of(G_in);
-        const int g_code = float_code(G);
-        const int64_t B = cfg.block;
-        void *const stream = stream_of(G);
-        const Packed xtq = pack(K, M, B), wtq = pack(K, N, B);
+// grad_X [M,K] = G [M,N] @ W [N,K], contracted over N; grad_W [N,K] = G.T [N,M] @ X [M,K], contracted over the rows
+// (block_linear.py:88-112); grad_bias = the column sums of G.  held: codes and scales of X transposed, of W transposed.
+torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &s, const Tensor *held, bool need_gx, bool need_gw, bool need_gb) {
+    torch::autograd::variable_list result(3);
+    const Config &cfg = s.cfg;
+    const int64_t M = s.M, K = s.K, N = s.N;
+    const bool graph = at::GradMode::is_enabled();
+    at::AutoGradMode no_grad(false);
+    require(G_in.is_cuda(), "the gradient must be a device tensor");
+    c10::DeviceGuard guard(G_in.device());
+    const Tensor G = matrix_of(G_in);
+    const int g_code = float_code(G);
+    const int64_t B = cfg.block;
+    void *const stream = stream_of(G);
+    const Packed xtq = pack(K, M, B), wtq = pack(K, N, B, s.together ? xtq.end() : 0);
 
-        if (fast_block(B) && M > 0 && N > 0 && K > 0 && (need_gx || need_gw)) {
-            const Packed gq = pack(need_gx ? M : 0, N, B), gtq = pack(need_gw ? N : 0, M, B, gq.end());
-            const bool both = need_gx && need_gw, sums = both && need_gb;
-            const int64_t part_at = gtq.end(), ws_at = up(part_at + (sums ? bi8_colsum_workspace_bytes(M, N) : 0), 256);
-            const int64_t kx = pad_contraction(M, K, N, B) ? gq.ld : N, kw = pad_contraction(N, K, M, B) ? gtq.ld : M;      // the contractions as multiplied
-            const int64_t need1 = need_gx && kx == gq.ld ? scratch_for(M, K, kx, B) : 0, need2 = need_gw && kw == gtq.ld ? scratch_for(N, K, kw, B) : 0;
-            const Tensor t = empty({ws_at + std::max(need1, need2)}, at::kByte, G);
-            uint8_t *const base = (uint8_t *)t.data_ptr();
-            if (both) {
-                const Bi8DualTask task = dual_task(G, t, gq, t, gtq);
-                check(bi8x_quantize_dual(&task, 1, g_code, (int)B, sums ? (float *)(base + part_at) : nullptr, stream), "bi8x_quantize_dual");
-                round_scales(t, gq, cfg.scale_type);
-                round_scales(t, gtq, cfg.scale_type);
-            } else if (need_gx) {
-                quantize_rows(G, t, gq, cfg, stream);
-            } else {
-                if (gtq.ld != M) t.slice(0, 0, gtq.end()).zero_();       // (the single-direction quantizer writes no padding)
-                check(bi8_quantize_transposed(G.data_ptr(), g_code, gtq.codes(t), gtq.scales(t), M, N, ld_of(G), gtq.ld, (int)B, stream), "bi8_quantize_transposed");
-                round_scales(t, gtq, cfg.scale_type);
-            }
-            const Bias none(Tensor(), 0);
-            if (need_gx) {
-                Tensor gx = empty(x_sizes, cfg.out_type, G);
-                void *const ws = need1 > 0 ? base + ws_at : nullptr;
-                if (wt_packed) {
-                    check(gemm_raw(gq.codes(t), gq.scales(t), gq.ld, wtq.codes(held[2]), wtq.scales(held[2]), wtq.ld, none, gx.data_ptr(), float_code(gx), M, K, kx, kx, B,
-                                   ws, need1, stream),
-                          "bi8x_gemm");
-                } else {
-                    multiply_ready(gq, t, held[2], held[3], N, none, gx, M, K, B, ws, need1, stream);
-                }
-                result[0] = gx;
-            }
-            if (need_gw) {
-                Tensor gw = empty({N, K}, cfg.out_type, G);
-                check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, kw, kw, B,
-                               need2 > 0 ? base + ws_at : nullptr, need2, stream),
-                      "bi8x_gemm");
-                result[1] = gw;
-            }
-            if (sums) {
-                Tensor gb = empty({N}, G.scalar_type(), G);
-                check(bi8x_colsum_finish((const float *)(base + part_at), gb.data_ptr(), g_code, M, N, stream), "bi8x_colsum_finish");
-                result[2] = gb;
-            }
+    if (fast_block(B) && M > 0 && N > 0 && K > 0 && (need_gx || need_gw)) {
+        const Packed gq = pack(need_gx ? M : 0, N, B), gtq = pack(need_gw ? N : 0, M, B, gq.end());
+        const bool both = need_gx && need_gw, sums = both && need_gb;
+        const int64_t part_at = gtq.end(), ws_at = up(part_at + (sums ? bi8_colsum_workspace_bytes(M, N) : 0), 256);
+        const int64_t kx = pad_contraction(M, K, N, B) ? gq.ld : N, kw = pad_contraction(N, K, M, B) ? gtq.ld : M;      // the contractions as multiplied
+        const int64_t need1 = need_gx && kx == gq.ld ? scratch_for(M, K, kx, B) : 0, need2 = need_gw && kw == gtq.ld ? scratch_for(N, K, kw, B) : 0;
+        const Tensor t = empty({ws_at + std::max(need1, need2)}, at::kByte, G);
+        uint8_t *const base = (uint8_t *)t.data_ptr();
+        if (both) {
+            const Bi8DualTask task = dual_task(G, t, gq, t, gtq);
+            check(bi8x_quantize_dual(&task, 1, g_code, (int)B, sums ? (float *)(base + part_at) : nullptr, stream), "bi8x_quantize_dual");
+            round_scales(t, gq, cfg.scale_type);
+            round_scales(t, gtq, cfg.scale_type);
+        } else if (need_gx) {
+            quantize_rows(G, t, gq, cfg, stream);
         } else {
-            if (need_gx) {
-                auto [q, s] = quantize_rowwise(G, B, cfg.scale_type);
-                result[0] = gemm(q, rows_of(held[2]), s, held[3], Tensor(), B, cfg.out_type).view(x_sizes);
-            }
-            if (need_gw) {
-                auto [q, s] = quantize_transposed(G, B, cfg.scale_type);
-                result[1] = gemm(q, held[0], s, held[1], Tensor(), B, cfg.out_type);
-            }
+            if (gtq.ld != M) t.slice(0, 0, gtq.end()).zero_();       // (the single-direction quantizer writes no padding)
+            check(bi8_quantize_transposed(G.data_ptr(), g_code, gtq.codes(t), gtq.scales(t), M, N, ld_of(G), gtq.ld, (int)B, stream), "bi8_quantize_transposed");
+            round_scales(t, gtq, cfg.scale_type);
         }
-        if (need_gb && !result[2].defined()) {
-            at::AutoGradMode as_called(graph);         // (plain torch operators: differentiable under create_graph)
-            result[2] = G_in.reshape({M, N}).sum(0);
+        const Bias none(Tensor(), 0);
+        if (need_gx) {
+            Tensor gx = empty(s.x_sizes, cfg.out_type, G);
+            void *const ws = need1 > 0 ? base + ws_at : nullptr;
+            if (s.wt_packed) {
+                check(gemm_raw(gq.codes(t), gq.scales(t), gq.ld, wtq.codes(held[2]), wtq.scales(held[2]), wtq.ld, none, gx.data_ptr(), float_code(gx), M, K, kx, kx, B,
+                               ws, need1, stream),
+                      "bi8x_gemm");
+            } else {
+                multiply_ready(gq, t, held[2], held[3], N, none, gx, M, K, B, ws, need1, stream);
+            }
+            result[0] = gx;
         }
-        return result;
+        if (need_gw) {
+            Tensor gw = empty({N, K}, cfg.out_type, G);
+            check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, kw, kw, B,
+                           need2 > 0 ? base + ws_at : nullptr, need2, stream),
+                  "bi8x_gemm");
+            result[1] = gw;
+        }
+        if (sums) {
+            Tensor gb = empty({N}, G.scalar_type(), G);
+            check(bi8x_colsum_finish((const float *)(base + part_at), gb.data_ptr(), g_code, M, N, stream), "bi8x_colsum_finish");
+            result[2] = gb;
+        }
+    } else {
+        if (need_gx) {
+            auto [q, qs] = quantize_rowwise(G, B, cfg.scale_type);
+            result[0] = gemm(q, rows_of(held[2]), qs, held[3], Tensor(), B, cfg.out_type).view(s.x_sizes);
+        }
+        if (need_gw) {
+            auto [q, qs] = quantize_transposed(G, B, cfg.scale_type);
+            result[1] = gemm(q, held[0], qs, held[1], Tensor(), B, cfg.out_type);
+        }
+    }
+    if (need_gb && !result[2].defined()) {
+        at::AutoGradMode as_called(graph);         // (plain torch operators: differentiable under create_graph)
+        result[2] = G_in.reshape({M, N}).sum(0);
+    }
+    return result;
+}
+
+// The same node for compiled autograd, which asks a node to describe itself and to run on stand-ins: torch's C++ autograd functions can.
+// (Not used in eager mode: an autograd function of torch costs the host 1.4 us more in the forward pass and 1.1 us in the backward.)
+struct CompiledBackward : public torch::autograd::Function<CompiledBackward> {
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        torch::autograd::variable_list held = ctx->get_saved_variables();
+        const std::vector<int64_t> of = ctx->saved_data["of"].toIntVector();
+        const Shape s{{of[0], (ScalarType)of[1], (ScalarType)of[2]}, of[3], of[4], of[5], {of.begin() + 9, of.end()}, of[6] != 0, of[7] != 0};
+        if (s.together) held[2] = held[0];
+        if (!grads[0].defined()) {
+            std::vector<int64_t> size = s.x_sizes;
+            size.back() = s.N;
+            grads[0] = at::zeros(size, at::TensorOptions().dtype(s.cfg.out_type).device(at::kCUDA, (c10::DeviceIndex)of[8]));
+        }
+        return linear_backward(grads[0], s, held.data(), held[2].defined() && ctx->needs_input_grad(0), held[0].defined() && ctx->needs_input_grad(1), ctx->needs_input_grad(2));
     }
 };
 
-Tensor linear_apply(const Tensor &x, const Tensor &stands_for_w, Operands op) {
-    static const Tensor *const none = new Tensor(at::empty({0}));
+struct LinearBackward : public torch::autograd::Node {
+    using Compiled = torch::autograd::CppNode<CompiledBackward>;
+    Shape s;
+    c10::DeviceIndex device = 0;
+    torch::autograd::SavedVariable saved[4];
+    bool has[4] = {false, false, false, false}, freed = false;
+    mutable std::shared_ptr<Compiled> compiled;
+
+    std::string name() const override { return "BlockInt8LinearBackward"; }
+    void keep(const Kept &xt, const Kept &wt) {
+        s.wt_packed = wt.packed;
+        s.together = wt.packed && xt.codes.defined() && wt.codes.is_same(xt.codes);
+        const Tensor *t[4] = {&xt.codes, &xt.scales, &wt.codes, &wt.scales};
+        for (int i = 0; i < 4; ++i) {
+            has[i] = t[i]->defined() && !(i == 2 && s.together);
+            if (has[i]) saved[i] = torch::autograd::SavedVariable(*t[i], false);
+        }
+    }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        freed = true;
+        compiled.reset();
+        for (auto &v : saved) v.reset_data();
+    }
+    void unpack(Tensor *held, const std::shared_ptr<torch::autograd::Node> &self) const {
+        TORCH_CHECK(!freed, torch::autograd::ERR_BACKWARD_TWICE);
+        for (int i = 0; i < 4; ++i)
+            if (has[i]) held[i] = saved[i].unpack(self);
+    }
+    torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
+        // (no gradient reached the output: zeros, as an autograd function of torch gets them)
+        if (!grads[0].defined()) grads[0] = input_metadata(0).zeros_like();
+        Tensor held[4];
+        {
+            std::lock_guard<std::mutex> lock(mutex_);
+            unpack(held, shared_from_this());
+        }
+        if (s.together) held[2] = held[0];
+        return linear_backward(grads[0], s, held, held[2].defined() && task_should_compute_output(0), held[0].defined() && task_should_compute_output(1),
+                               task_should_compute_output(2));
+    }
+    void compiled_args(torch::dynamo::autograd::CompiledNodeArgs &args) const override {
+        torch::autograd::variable_list held(4);
+        unpack(held.data(), std::const_pointer_cast<torch::autograd::Node>(shared_from_this()));
+        compiled = std::shared_ptr<Compiled>(new Compiled(), torch::autograd::deleteNode);
+        compiled->set_ctx_grad_fn(compiled);
+        compiled->set_next_edges(torch::autograd::edge_list(next_edges()));
+        compiled->is_variable_input_ = {true, true, true};
+        std::vector<int64_t> of = {s.cfg.block, (int64_t)s.cfg.out_type, (int64_t)s.cfg.scale_type, s.M, s.K, s.N, s.wt_packed, s.together, device};
+        of.insert(of.end(), s.x_sizes.begin(), s.x_sizes.end());
+        compiled->ctx_.saved_data["of"] = std::move(of);
+        compiled->ctx_.set_materialize_grads(false);
+        compiled->ctx_.save_for_backward(std::move(held));
+        compiled->save_variables_to_ctx();
+        compiled->compiled_args(args);
+    }
+    torch::autograd::variable_list apply_with_saved(const torch::autograd::variable_list &grads, torch::dynamo::autograd::SwapSavedVariables &swapped) override {
+        return compiled->apply_with_saved(grads, swapped);
+    }
+};
+
+// The differentiable layer: autograd's inputs are x, `stands_for_w` (the tensor that receives grad_W: the float weight itself, or what
+// stands for it where its codes come ready) and the bias.
+Tensor linear_apply(const Tensor &x, const Tensor &w, const Tensor &w_int8, const Tensor &w_state, const Tensor &stands_for_w, const Kept &wt_ready, const Tensor &bias,
+                    const Config &cfg) {
     require(x.is_cuda(), "x must be a device tensor");
-    for (const Tensor *t : {&x, &std::as_const(op.w), &stands_for_w, &std::as_const(op.bias)})
+    for (const Tensor *t : {&x, &w, &stands_for_w, &bias})
         TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(), "blockwise_int8_linear has no forward-mode derivative");
     const bool grad = at::GradMode::is_enabled();
-    op.need_gx = grad && x.requires_grad();
-    op.need_gw = grad && stands_for_w.defined() && stands_for_w.requires_grad();
+    const bool need_gx = grad && x.requires_grad(), need_gw = grad && stands_for_w.defined() && stands_for_w.requires_grad(), need_gb = grad && bias.defined() && bias.requires_grad();
     c10::DeviceGuard guard(x.device());
-    if (op.need_gx || op.need_gw || (grad && op.bias.defined() && op.bias.requires_grad()))
-        return BlockInt8LinearFunction::apply(x, stands_for_w.defined() ? stands_for_w : *none, op.bias.defined() ? op.bias : *none, op);
-    at::AutoGradMode no_grad(false);
     Kept xt, wt;
-    return linear_forward(x, op.w, op.w_int8, op.w_state, op.bias, op.cfg, false, false, xt, wt);
+    Tensor out;
+    {
+        at::AutoGradMode no_grad(false);
+        out = linear_forward(x, w, w_int8, w_state, bias, cfg, need_gw, need_gx && w.defined(), xt, wt);
+    }
+    if (need_gx || need_gw || need_gb) {
+        std::shared_ptr<LinearBackward> node(new LinearBackward(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(x, stands_for_w, bias));
+        node->s.cfg = cfg;
+        node->s.K = x.size(-1);
+        node->s.N = out.size(-1);
+        node->s.M = 1;
+        for (int64_t d = 0; d + 1 < x.dim(); ++d) node->s.M *= x.size(d);
+        node->s.x_sizes.assign(x.sizes().begin(), x.sizes().end());
+        node->device = x.device().index();
+        node->keep(xt, w.defined() || !need_gx ? wt : wt_ready);
+        torch::autograd::set_history(out, node);
+    }
+    return out;
 }
 
 // Quantize + GEMM in one launch for one or two rows, where the library covers it (bi8_linear_few_rows); undefined otherwise.
@@ -627,7 +695,7 @@ PyObject *py_linear(PyObject *, PyObject *const *v, Py_ssize_t n) {             
     return guarded("linear", 6, v, n, [](Args a) {
         const Tensor x = a.tensor(0), w = a.tensor(1), bias = a.optional_tensor(2);
         const Config cfg{a.block(3), a.dtype(4), a.dtype(5)};
-        return wrapped(without_gil([&] { return linear_apply(x, w, Operands{cfg, w, Tensor(), Tensor(), bias, Kept()}); }));
+        return wrapped(without_gil([&] { return linear_apply(x, w, Tensor(), Tensor(), w, Kept(), bias, cfg); }));
     });
 }
 // x, W codes, W scales, bias, transposed W codes, their scales, weight or None, block, output dtype, scale dtype
@@ -641,7 +709,7 @@ PyObject *py_linear_kept(PyObject *, PyObject *const *v, Py_ssize_t n) {
         const Config cfg{a.block(7), a.dtype(8), a.dtype(9)};
         return wrapped(without_gil([&] {
             check_codes(wt.codes, wt.scales, wq.size(0), cfg.block);
-            return linear_apply(x, weight, Operands{cfg, Tensor(), wq, ws, bias, wt});
+            return linear_apply(x, Tensor(), wq, ws, weight, wt, bias, cfg);
         }));
     });
 }

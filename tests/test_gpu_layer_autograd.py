@@ -66,15 +66,46 @@ def test_a_trace_records_the_call(layer):
     assert torch.equal(traced(other), layer(other))
 
 
-def test_compiled_autograd(layer):
+@pytest.mark.parametrize("frozen", ["", "x", "weight", "weight bias", "x weight"])
+def test_compiled_autograd(layer, frozen):
     from torch._dynamo import compiled_autograd
     enable = getattr(compiled_autograd, "_enable", None) or compiled_autograd.enable
-    x, g = torch.randn(70, 192, device=DEV), torch.randn(70, 130, device=DEV)
-    want = _grads(layer, x, g)
+    x, g = torch.randn(70, 192, device=DEV, requires_grad="x" not in frozen), torch.randn(70, 130, device=DEV)
+    layer.weight.requires_grad_("weight" not in frozen)
+    layer.bias.requires_grad_("bias" not in frozen)
+
+    def grads(times=1):
+        x.grad = None
+        layer.zero_grad(set_to_none=True)
+        y = layer(x)
+        for i in range(times):
+            y.backward(g, retain_graph=i + 1 < times)
+        with pytest.raises(RuntimeError, match="second time"):
+            y.backward(g)
+        return [t.grad for t in (x, layer.weight, layer.bias) if t.requires_grad]
+    want, twice = grads(), grads(2)
     for _ in range(2):
         with enable(torch.compile(backend="eager")):
-            got = _grads(layer, x, g)
-        assert all(map(torch.equal, got, want))
+            assert all(map(torch.equal, grads(), want)) and all(map(torch.equal, grads(2), twice))
+
+
+def test_compiled_autograd_of_an_output_that_no_gradient_reaches(layer):
+    from torch._dynamo import compiled_autograd
+    enable = getattr(compiled_autograd, "_enable", None) or compiled_autograd.enable
+
+    class Stop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, y):
+            return y.clone()
+
+        @staticmethod
+        def backward(ctx, g):
+            return None
+    x = torch.randn(5, 192, device=DEV, requires_grad=True)
+    y = Stop.apply(layer(x))
+    with enable(torch.compile(backend="eager")):
+        y.backward(torch.randn(5, 130, device=DEV))
+    assert all(t.grad is not None and not t.grad.any() for t in (x, layer.weight, layer.bias))
 
 
 @pytest.mark.parametrize("traced", [False, True], ids=["eager", "traced"])
