@@ -17,9 +17,11 @@ constexpr int kChunks = 1;                 // 1 KiB wave-loads per row per tile 
 constexpr int kThreads = 256;
 // Codes of more than this (the eight 4 MiB L2s together) leave with ordinary stores, others non-temporal.  Marked non-temporal, a large
 // tensor's codes come back slower to the kernel that reads them next.  us, non-temporal -> ordinary, quantize + dequantize: bf16
-// [8192,8192] 68.1 -> 65.0 (5.2 TB/s of the 338 MB that input, codes and output take once), fp32 [8192,8192] 110.9 -> 102.2, bf16
-// [8320,4096] 38.8 -> 36.3; quantize + GEMM: 8192 x 11008 -> 1024 157.2 -> 149.6, fp32 4096 x 12288 -> 4096 348 -> 330, 8192 x 4224 ->
-// 2048 96.9 -> 96.1.  Below, they gain nothing: 2048 x 4096 -> 11008 (8 MiB) 116.8 -> 117.3.
+// [8192,8192] 68.2 -> 65.1 (5.2 TB/s of the 338 MB that input, codes and output take once; 69.5 -> 69.2 on another machine), fp32
+// [8192,8192] 109 -> 102, bf16 [8320,4096] 37.9 -> 36.3, [8192,12288] 102.4 -> 96.1; quantize + GEMM: 8192 x 11008 -> 1024 158 -> 148,
+// fp32 4096 x 12288 -> 4096 271 -> 252, 8192 x 4224 -> 2048 95.2 -> 95.4.  The quantizer by itself pays for a part of that: bf16
+// [8192,8192] 31.9 -> 34.4, [8320,4096] 17.1 -> 19.5, fp32 [8192,8192] 53.7 -> 52.3.  Below, they gain nothing: 2048 x 4096 -> 11008 (8 MiB)
+// 116.8 -> 117.3.
 constexpr int64_t kKeepCodes = 32 << 20;
 
 // ALIGNED: rows of x on 16-byte boundaries, K a multiple of the elements per 16 bytes, rows of q aligned to their
