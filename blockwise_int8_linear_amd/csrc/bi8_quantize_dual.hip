@@ -45,26 +45,12 @@ constexpr int kQPitch = kTR + 16;  // code tile pitch in bytes: rows stay 16-byt
 // element by element.
 // NH: halves per tile.  2 is the tile described above; 1 (a 128 x 64 tile, blocks of at most 64) doubles the number of
 // workgroups for inputs too small to occupy the chip with full tiles.
-// PAIR: the grid's first pair.blocks0 workgroups work on the first matrix, the others on the second (a layer's X and W: one
-// launch, and the smaller of the two does not have the chip to itself half empty).
-struct DualPair {
-    Bi8DualTask task[2];
-    unsigned blocks0;
-};
-
-template <int DT, int B, bool ALIGNED, bool SUM, int NH, bool PAIR>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DT == BI8_F32 ? 2 : 3))) void quantize_dual_tile(const DualPair pair, float *__restrict__ colsum_part) {
-    const bool second = PAIR && blockIdx.x >= pair.blocks0;
-    const Bi8DualTask &t0 = pair.task[0], &t1 = pair.task[1];
-#define BI8_OF_TASK(f) (second ? t1.f : t0.f)
-    const void *const __restrict__ x = BI8_OF_TASK(x);
-    int8_t *const __restrict__ q = BI8_OF_TASK(q), *const __restrict__ qT = BI8_OF_TASK(qT);
-    float *const __restrict__ scales = BI8_OF_TASK(scales), *const __restrict__ scalesT = BI8_OF_TASK(scalesT);
-    const int64_t R = BI8_OF_TASK(R), C = BI8_OF_TASK(C), ldx = BI8_OF_TASK(ldx), ldq = BI8_OF_TASK(ldq), ldqt = BI8_OF_TASK(ldqt);
-    const int64_t Rp = BI8_OF_TASK(Rp), Cp = BI8_OF_TASK(Cp);        // rows and columns written, the matrix' own or more: zeros past its end
-#undef BI8_OF_TASK
-    const int64_t tiles_c = (Cp + NH * kTC - 1) / (NH * kTC), ntiles = tiles_c * ((Rp + kTR - 1) / kTR);
-    const int64_t first_tile = second ? blockIdx.x - pair.blocks0 : blockIdx.x, tile_step = !PAIR ? gridDim.x : second ? gridDim.x - pair.blocks0 : pair.blocks0;
+// Rp, Cp: rows and columns written, the matrix' own or more: zeros past its end.  The workgroup's tiles: first_tile, first_tile +
+// tile_step, ... of ntiles, tiles_c in a row of tiles.
+template <int DT, int B, bool ALIGNED, bool SUM, int NH>
+__device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales, int8_t *__restrict__ qT,
+                                           float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx, int64_t ldq,
+                                           int64_t ldqt, int64_t Rp, int64_t Cp, int64_t tiles_c, int64_t ntiles, int64_t first_tile, int64_t tile_step) {
     constexpr int VEC = Bi8Vec<DT>::kElems;
     constexpr int64_t ES = 16 / VEC;
     constexpr int LPR = kTC / VEC;                 // lanes per half row: 8 (16-bit) or 16 (fp32)
@@ -347,22 +333,64 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DT == 
     }
 }
 
-template <int DT, int B, bool ALIGNED, int NH> int launch_dual_as(const Bi8DualTask *task, int count, float *colsum_part, int64_t resident, hipStream_t st) {
-    DualPair pair{{task[0], task[count - 1]}, 0};
-    int64_t tiles[2];
-    for (int i = 0; i < 2; ++i) tiles[i] = ((pair.task[i].Rp + kTR - 1) / kTR) * ((pair.task[i].Cp + NH * kTC - 1) / (NH * kTC));
-    if (count == 1) {
-        const int64_t grid = tiles[0] < resident ? tiles[0] : resident;
-        if (colsum_part) hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, true, NH, false>), dim3((unsigned)grid), dim3(kThreads), 0, st, pair, colsum_part);
-        else hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH, false>), dim3((unsigned)grid), dim3(kThreads), 0, st, pair, colsum_part);
-        return bi8_launch_rc();
+#define BI8_DUAL_KERNEL __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DT == BI8_F32 ? 2 : 3)))
+template <int DT, int B, bool ALIGNED, bool SUM, int NH>
+BI8_DUAL_KERNEL void quantize_dual_tile(const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales, int8_t *__restrict__ qT,
+                                        float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx, int64_t ldq, int64_t ldqt,
+                                        int64_t Rp, int64_t Cp, int64_t tiles_c, int64_t ntiles) {
+    dual_tiles<DT, B, ALIGNED, SUM, NH>(x, q, scales, qT, scalesT, colsum_part, R, C, ldx, ldq, ldqt, Rp, Cp, tiles_c, ntiles, blockIdx.x, gridDim.x);
+}
+
+// Two matrices: the grid's first blocks0 workgroups work on the first, the others on the second (a layer's X and W: one launch, and
+// the smaller of the two does not have the chip to itself half empty).
+struct DualPair {
+    Bi8DualTask task[2];
+    int64_t tiles_c[2], ntiles[2];
+    unsigned blocks0;
+};
+template <int DT, int B, bool ALIGNED, int NH> BI8_DUAL_KERNEL void quantize_dual_pair(const DualPair pair) {
+    const bool second = blockIdx.x >= pair.blocks0;
+    const Bi8DualTask &t0 = pair.task[0], &t1 = pair.task[1];
+#define BI8_OF_TASK(f) (second ? t1.f : t0.f)
+    dual_tiles<DT, B, ALIGNED, false, NH>(BI8_OF_TASK(x), BI8_OF_TASK(q), BI8_OF_TASK(scales), BI8_OF_TASK(qT), BI8_OF_TASK(scalesT), nullptr, BI8_OF_TASK(R),
+                                          BI8_OF_TASK(C), BI8_OF_TASK(ldx), BI8_OF_TASK(ldq), BI8_OF_TASK(ldqt), BI8_OF_TASK(Rp), BI8_OF_TASK(Cp),
+                                          second ? pair.tiles_c[1] : pair.tiles_c[0], second ? pair.ntiles[1] : pair.ntiles[0],
+                                          second ? blockIdx.x - pair.blocks0 : blockIdx.x, second ? gridDim.x - pair.blocks0 : pair.blocks0);
+#undef BI8_OF_TASK
+}
+
+template <int DT, int B, bool ALIGNED, int NH> int launch_one(const Bi8DualTask &t, float *colsum_part, int64_t resident, hipStream_t st) {
+    const int64_t tiles_c = (t.Cp + NH * kTC - 1) / (NH * kTC), ntiles = tiles_c * ((t.Rp + kTR - 1) / kTR);
+    const dim3 grid((unsigned)(ntiles < resident ? ntiles : resident));
+    if (colsum_part)
+        hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, true, NH>), grid, dim3(kThreads), 0, st, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx,
+                           t.ldq, t.ldqt, t.Rp, t.Cp, tiles_c, ntiles);
+    else
+        hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH>), grid, dim3(kThreads), 0, st, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx,
+                           t.ldq, t.ldqt, t.Rp, t.Cp, tiles_c, ntiles);
+    return bi8_launch_rc();
+}
+
+// Both matrices in one launch, the resident workgroups in proportion to the tiles; BI8_ERR_UNSUPPORTED where that is not taken: from kPairRounds
+// rounds of workgroups on it has to save one.  The mixed traffic of two matrices costs about 1 % (bf16, block 128, X 4096 x 4096 and W
+// 11008 x 4096, 1024 and 2752 tiles, four rounds either way: 55.6 us in two launches, 56.6 in one; in a training pass 668 against 672), the
+// second launch about 1.5 us.  us, two launches -> one, tiles of X + W and rounds: 48 + 108 (2 -> 1) 12.2 -> 7.0; 1024 + 1024 (2 -> 2) 31.8 ->
+// 30.3; at fp32 (768 workgroups) 1710 + 665 (4 -> 4) 67.7 -> 67.7, 672 + 1120 (3 -> 3) 50.1 -> 49.6; 1836 + 4104 (7 -> 6) 92.1 -> 84.4.
+constexpr int64_t kPairRounds = 4;
+template <int DT, int B, bool ALIGNED, int NH> int launch_pair(const Bi8DualTask *task, int64_t resident, hipStream_t st) {
+    DualPair pair{{task[0], task[1]}, {}, {}, 0};
+    for (int i = 0; i < 2; ++i) {
+        pair.tiles_c[i] = (task[i].Cp + NH * kTC - 1) / (NH * kTC);
+        pair.ntiles[i] = pair.tiles_c[i] * ((task[i].Rp + kTR - 1) / kTR);
     }
-    // the resident workgroups in proportion to the tiles
-    const int64_t all = tiles[0] + tiles[1], grid = all < resident ? all : resident;
+    const int64_t *tiles = pair.ntiles, all = tiles[0] + tiles[1], grid = all < resident ? all : resident;
     int64_t first = all <= resident ? tiles[0] : (grid * tiles[0] + all / 2) / all;
     first = first < 1 ? 1 : first > grid - 1 ? grid - 1 : first;
+    const int64_t apart = (tiles[0] + resident - 1) / resident + (tiles[1] + resident - 1) / resident;
+    const int64_t r0 = (tiles[0] + first - 1) / first, r1 = (tiles[1] + grid - first - 1) / (grid - first);
+    if (apart >= kPairRounds && (r0 > r1 ? r0 : r1) >= apart) return BI8_ERR_UNSUPPORTED;
     pair.blocks0 = (unsigned)first;
-    hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH, true>), dim3((unsigned)grid), dim3(kThreads), 0, st, pair, colsum_part);
+    hipLaunchKernelGGL((quantize_dual_pair<DT, B, ALIGNED, NH>), dim3((unsigned)grid), dim3(kThreads), 0, st, pair);
     return bi8_launch_rc();
 }
 
@@ -370,13 +398,17 @@ template <int DT, int B, bool ALIGNED> int launch_dual(const Bi8DualTask *task, 
     // workgroups per CU: four with 16-bit inputs (29 KiB of LDS, under 128 registers: 62.7 us against 65.9 with three at
     // bf16 [8192,8192]), three with fp32 (42 KiB)
     const int64_t resident = (DT == BI8_F32 ? 3 : 4) * 256;
-    if constexpr (B <= kTC) {
-        // inputs of fewer full tiles than the chip holds workgroups: half tiles, twice as many workgroups
-        int64_t full = 0;
-        for (int i = 0; i < count; ++i) full += ((task[i].Cp + 2 * kTC - 1) / (2 * kTC)) * ((task[i].Rp + kTR - 1) / kTR);
-        if (full < resident) return launch_dual_as<DT, B, ALIGNED, 1>(task, count, colsum_part, resident, st);
-    }
-    return launch_dual_as<DT, B, ALIGNED, 2>(task, count, colsum_part, resident, st);
+    // inputs of fewer full tiles than the chip holds workgroups: half tiles, twice as many workgroups
+    int64_t full = 0;
+    for (int i = 0; i < count; ++i) full += ((task[i].Cp + 2 * kTC - 1) / (2 * kTC)) * ((task[i].Rp + kTR - 1) / kTR);
+    constexpr int kHalf = B <= kTC ? 1 : 2;
+    const bool half = full < resident;
+    if (count == 1)
+        return half ? launch_one<DT, B, ALIGNED, kHalf>(task[0], colsum_part, resident, st) : launch_one<DT, B, ALIGNED, 2>(task[0], colsum_part, resident, st);
+    const int rc = half ? launch_pair<DT, B, ALIGNED, kHalf>(task, resident, st) : launch_pair<DT, B, ALIGNED, 2>(task, resident, st);
+    if (rc != BI8_ERR_UNSUPPORTED) return rc;
+    const int rc0 = launch_dual<DT, B, ALIGNED>(task, 1, nullptr, st);
+    return rc0 != BI8_OK ? rc0 : launch_dual<DT, B, ALIGNED>(task + 1, 1, nullptr, st);
 }
 
 template <int DT, bool ALIGNED> int dispatch(const Bi8DualTask *task, int count, float *colsum_part, int block, hipStream_t st) {

@@ -156,3 +156,42 @@ def test_padded_code_buffers_hold_the_same_codes(ops, dtype):
         assert q_store.shape[1] % 16 == 0 and q_store.shape[1] >= C and q_store.data_ptr() % 16 == 0
         assert torch.equal(qp, q) and torch.equal(qtp, qt) and _same(sp, s) and _same(stp, st)
         assert (q_store[:, C:] == 0).all() and (qt_store[:, R:] == 0).all()          # the padding stays zero
+
+
+@pytest.mark.parametrize("first,second,block,dtype", [
+    ((70, 64), (33, 64), 64, "bf16"),                # one tile each
+    ((1000, 768), (2304, 768), 64, "bf16"),          # fewer tiles than workgroups: half tiles
+    ((300, 513), (4097, 513), 32, "f32"),            # odd rows
+    ((2100, 6272), (1100, 6272), 128, "f16"),        # two rounds of workgroups either way: one launch
+    ((4096, 4096), (11008, 4096), 128, "bf16"),      # four rounds either way: two launches
+    ((3364, 6016), (5696, 6016), 64, "bf16"),        # five rounds in two launches, four in one
+    ((2248, 12160), (896, 12160), 64, "f32"),        # four rounds either way at fp32: two launches
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_two_matrices_in_one_call(first, second, block, dtype):
+    """what the layer asks for X and W, rows padded to multiples of 128 with zero codes and scales: the codes and scales of the
+    single-direction quantizers"""
+    import ctypes
+
+    import blockwise_int8_linear_amd as pkg
+    from blockwise_int8_linear_amd import _lib
+
+    class Task(ctypes.Structure):
+        _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "q", "qT", "scales", "scalesT")] +
+                    [(n, ctypes.c_int64) for n in ("R", "C", "ldx", "ldq", "ldqt", "Rp", "Cp")])
+    g = torch.Generator(device="cuda:0").manual_seed(sum(first) + block)
+    tasks, held = (Task * 2)(), []
+    for i, (R, C) in enumerate((first, second)):
+        Rp, Cp = -(-R // 128) * 128, -(-C // 128) * 128
+        x = torch.randn(R, C, generator=g, device="cuda:0").to(DTYPES[dtype])
+        q, qt = torch.full((R, Cp), 77, device="cuda:0", dtype=torch.int8), torch.full((C, Rp), 77, device="cuda:0", dtype=torch.int8)
+        s, st = torch.full((Cp // block, R), -1.0, device="cuda:0"), torch.full((Rp // block, C), -1.0, device="cuda:0")
+        held.append((x, q, qt, s, st))
+        tasks[i] = Task(x.data_ptr(), q.data_ptr(), qt.data_ptr(), s.data_ptr(), st.data_ptr(), R, C, C, Cp, Rp, Rp, Cp)
+    call = _lib.load().bi8x_quantize_dual
+    call.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    assert call(tasks, 2, {"f32": 0, "bf16": 1, "f16": 2}[dtype], block, None, torch.cuda.current_stream().cuda_stream) == 0
+    for x, q, qt, s, st in held:
+        for got, scales, (want, want_s) in ((q, s, pkg.quantize_block_rowwise(x, block)), (qt, st, pkg.quantize_block_transposed(x, block))):
+            rows, k = want.shape
+            assert torch.equal(got[:, :k], want) and not got[:, k:].any()
+            assert torch.equal(scales[:want_s.shape[0]], want_s) and not scales[want_s.shape[0]:].any()
