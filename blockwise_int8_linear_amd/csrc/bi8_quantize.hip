@@ -1,19 +1,16 @@
 // Block quantize along rows (bi8_quantize_rowwise): per (row, K-block) absmax -> fp32 scale, int8 codes
 // rint_even(127 * (x / absmax)).  HBM-bound: every input byte is read once with 128-bit loads, every
-// code written once; the scales go through LDS so that each K-block's scales leave the workgroup as
-// runs of 16 consecutive rows (the scale array is block-major / row-minor).
+// code written once; with two or four rows per wave the scales go through LDS so that each K-block's scales leave the workgroup as
+// runs of 8 or 16 consecutive rows (the scale array is block-major / row-minor).
 //
 // Replaces _quantize_block_rowwise, triton_functions.py:193-216 (one program per row, serial over the
-// row's blocks) with a 2-D tiling: one workgroup = 16 rows x 1 KiB of row, one lane = 16 input bytes,
+// row's blocks) with a 2-D tiling: one workgroup = 4, 8 or 16 rows x 1 KiB of row, one lane = 16 input bytes,
 // one K-block = L adjacent lanes (L = block * sizeof(elem) / 16), absmax by DPP inside the lane group.
 #include "bi8_common.h"
 #include "bi8_internal.h"
 
 namespace {
 
-constexpr int kRowsPerWave = 4;            // = 16-byte loads in flight per lane; 2 and 8 both measured slower
-constexpr int kRows = 4 * kRowsPerWave;    // rows per workgroup tile
-constexpr int kChunks = 1;                 // 1 KiB wave-loads per row per tile (2 and 4 measured slower)
 constexpr int kThreads = 256;
 // Codes of more than this (the eight 4 MiB L2s together) leave with ordinary stores, others non-temporal.  Marked non-temporal, a large
 // tensor's codes come back slower to the kernel that reads them next.  us, non-temporal -> ordinary, quantize + dequantize: bf16
@@ -24,119 +21,190 @@ constexpr int kThreads = 256;
 // 116.8 -> 117.3.
 constexpr int64_t kKeepCodes = 32 << 20;
 
+// The largest magnitude of a lane's 16 bytes, as bits: magnitudes order like their bits, and a NaN lies above infinity.  16-bit
+// types: the maxima of the low and of the high halves, which magnitude_of() joins.
+template <int DT> __device__ __forceinline__ uint32_t magnitude_bits(const bi8_v4u &raw) {
+    if constexpr (DT == BI8_F32) {
+        uint32_t m = raw[0] & 0x7fffffffu;
+#pragma unroll
+        for (int e = 1; e < 4; ++e) m = max(m, raw[e] & 0x7fffffffu);
+        return m;
+    } else {
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 m = __builtin_bit_cast(u16x2, raw[0] & 0x7fff7fffu);
+#pragma unroll
+        for (int e = 1; e < 4; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, raw[e] & 0x7fff7fffu));
+        return __builtin_bit_cast(uint32_t, m);
+    }
+}
+template <int DT> __device__ __forceinline__ uint32_t larger_bits(uint32_t a, uint32_t b) {
+    if constexpr (DT == BI8_F32) return max(a, b);
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_bits(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true); }
+// over aligned groups of L lanes (the steps of bi8_group_max)
+template <int DT, int L> __device__ __forceinline__ uint32_t group_bits(uint32_t m) {
+    if constexpr (L >= 2) m = larger_bits<DT>(m, dpp_bits<0xB1>(m));
+    if constexpr (L >= 4) m = larger_bits<DT>(m, dpp_bits<0x4E>(m));
+    if constexpr (L >= 8) m = larger_bits<DT>(m, dpp_bits<0x141>(m));
+    if constexpr (L >= 16) m = larger_bits<DT>(m, dpp_bits<0x140>(m));
+    if constexpr (L >= 32) m = larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 16, 64));
+    if constexpr (L >= 64) m = larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+    return m;
+}
+// the magnitude itself; a NaN stays one
+template <int DT> __device__ __forceinline__ float magnitude_of(uint32_t m) {
+    if constexpr (DT == BI8_F32) return bi8_u2f(m);
+    const uint32_t h = max(m & 0xffffu, m >> 16);
+    return DT == BI8_BF16 ? bi8_from_bf16_bits(h) : bi8_from_f16_bits(h);
+}
+
+// One wave = RPW rows x 1 KiB, one workgroup = four of them, one below the other.
 // ALIGNED: rows of x on 16-byte boundaries, K a multiple of the elements per 16 bytes, rows of q aligned to their
 // 4- or 8-byte stores.  Otherwise (odd row length or leading dimension, e.g. the GPT-2 vocabulary 50257) whole chunks
 // move with unaligned 16-byte loads and 4- or 8-byte stores, the last, partial chunk of a row element by element.
 // keep: the codes' stores of aligned rows are not marked non-temporal (see kKeepCodes).
 // Kp: columns written, K or more: zero codes and zero scales past the row's end (the padding that a GEMM contracted over K wants).
-template <int DT, int L, bool ALIGNED>
+// A row past the end reads the last one and is not stored: the rows' loads do not branch, nor does their arithmetic, so that the rows' chains of dependent instructions run side by side: a block that needs the IEEE division (a
+// scale of 0, subnormal, huge or infinite, a NaN) is done over in one place behind them.
+template <int DT, int L, bool ALIGNED, int RPW>
 __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const void *__restrict__ x, int8_t *__restrict__ q,
                                                               float *__restrict__ scales, int64_t M, int64_t K, int64_t Kp,
-                                                              int64_t ldx, int64_t ldq, int64_t nblk, int tiles_k, bool keep) {
+                                                              int64_t ldx, int64_t ldq, int64_t nblk, bool keep) {
     constexpr int VEC = Bi8Vec<DT>::kElems;
     constexpr int B = L * VEC;                       // block size in elements
-    constexpr int TE = kChunks * BI8_WAVE * VEC;     // elements of one row covered by a tile
-    constexpr int NB = TE / B;                       // K-blocks per tile row
+    constexpr int TE = BI8_WAVE * VEC;               // elements of one row covered by a tile
     constexpr int NCORR = (DT == BI8_F32) ? 2 : 1;
     constexpr int64_t ES = 16 / VEC;                 // bytes per element
-    __shared__ float s_tile[NB][kRows + 1];
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int64_t tile_m = blockIdx.x / tiles_k;
-    const int tile_k = blockIdx.x % tiles_k;
-    const int64_t row0 = tile_m * kRows;
-    const int64_t col0 = (int64_t)tile_k * TE;
-    const char *xb = (const char *)x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row0 = (((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * 4 + wave) * RPW;
+    if (RPW == 1 && row0 >= M) return;
+    const int64_t col0 = (int64_t)blockIdx.x * TE;
+    const int64_t left = K - col0;                   // elements of a row from the tile's first column on (none or less: padding only)
+    const char *xb = (const char *)x + col0 * ES;
 
-    bi8_v4u raw[kRowsPerWave][kChunks];
+    auto row_of = [&](int i) { return row0 + i < M ? row0 + i : M - 1; };
+    const int mine = (int)(left < TE ? (left > 0 ? left : 0) : TE) - lane * VEC;      // of the row's elements from this lane's first on
+
+    bi8_v4u raw[RPW];
 #pragma unroll
-    for (int i = 0; i < kRowsPerWave; ++i) {
-        const int64_t row = row0 + wave * kRowsPerWave + i;
+    for (int i = 0; i < RPW; ++i) raw[i] = bi8_v4u{0u, 0u, 0u, 0u};
+    if (mine >= VEC) {
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            const int64_t col = col0 + (c * BI8_WAVE + lane) * VEC;
-            bi8_v4u v = {0u, 0u, 0u, 0u};
-            if (row < M && col < K) {
-                const char *src = xb + (row * ldx + col) * ES;
+        for (int i = 0; i < RPW; ++i) {
+            const char *src = xb + row_of(i) * ldx * ES;
+            if constexpr (ALIGNED) raw[i] = __builtin_nontemporal_load((const bi8_v4u *)(src + lane * 16));
+            else raw[i] = *(const bi8_v4u_unaligned *)(src + lane * 16);
+        }
+    }
+    if constexpr (!ALIGNED) {
+        if (mine > 0 && mine < VEC) {                // the row ends inside this chunk
+#pragma unroll
+            for (int i = 0; i < RPW; ++i) {
+                const char *src = xb + row_of(i) * ldx * ES + lane * 16;
+#pragma unroll
+                for (int e = 0; e < VEC - 1; ++e) {
+                    if (e < mine) {
+                        if constexpr (DT == BI8_F32) raw[i][e] = ((const uint32_t *)src)[e];
+                        else raw[i][e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
+                    }
+                }
+            }
+        }
+    }
+
+    float m[RPW];
+    uint32_t w[RPW][VEC / 4];
+    bool slow = false;
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) m[i] = magnitude_of<DT>(group_bits<DT, L>(magnitude_bits<DT>(raw[i])));
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+        float f[VEC];
+        bi8_unpack<DT>(raw[i], f);
+        slow |= mine > 0 && !bi8_scale_is_ordinary(m[i]);
+        const float y = 1.0f / m[i];                                    // correctly rounded reciprocal
+        uint32_t code[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) code[e] = bi8_code_fast<NCORR>(f[e], m[i], y);
+#pragma unroll
+        for (int e = 0; e < VEC; e += 4) w[i][e / 4] = bi8_pack4(code[e], code[e + 1], code[e + 2], code[e + 3]);
+    }
+    if (left < TE) {                                 // past the row's end: codes of zero
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int e = 0; e < VEC / 4; ++e) w[i][e] = mine > 0 ? w[i][e] : 0u;
+    }
+    if (__builtin_expect(__any(slow), 0)) {
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            if (!bi8_scale_is_ordinary(m[i])) {                         // (the same for all lanes of a block)
+                float f[VEC], s = 0.0f;
+                bi8_unpack<DT>(raw[i], f);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) s = __builtin_fmaxf(s, __builtin_fabsf(f[e]));      // ignores NaN
+                s = bi8_group_max<L>(s);
+                m[i] = s;
+                uint32_t code[VEC];
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) code[e] = bi8_code_slow(f[e], s);
+#pragma unroll
+                for (int e = 0; e < VEC; e += 4) w[i][e / 4] = bi8_pack4(code[e], code[e + 1], code[e + 2], code[e + 3]);
+            }
+        }
+    }
+
+    const int64_t to_write = Kp - col0;
+    const int room = (int)(to_write < TE ? to_write : TE) - lane * VEC;          // columns to write from this lane's first on
+#pragma unroll
+    for (int i = 0; i < RPW; ++i) {
+        if (row0 + i >= M) break;
+        int8_t *dst = q + (row0 + i) * ldq + col0 + lane * VEC;
+        if (room >= VEC) {
+            if constexpr (VEC == 4) {
                 if constexpr (ALIGNED) {
-                    v = __builtin_nontemporal_load((const bi8_v4u *)src);
-                } else if (col + VEC <= K) {
-                    v = *(const bi8_v4u_unaligned *)src;
-                } else {                           // the row ends inside this chunk
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        if (col + e < K) {
-                            if constexpr (DT == BI8_F32) v[e] = ((const uint32_t *)src)[e];
-                            else v[e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
-                        }
-                    }
-                }
-            }
-            raw[i][c] = v;
-        }
-    }
-
-#pragma unroll
-    for (int i = 0; i < kRowsPerWave; ++i) {
-        const int64_t row = row0 + wave * kRowsPerWave + i;
-#pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            const int64_t col = col0 + (c * BI8_WAVE + lane) * VEC;
-            float f[VEC];
-            bi8_unpack<DT>(raw[i][c], f);
-            float m = 0.0f;
-            bool special = false;
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                m = __builtin_fmaxf(m, __builtin_fabsf(f[e]));      // ignores NaN
-                special |= (f[e] != f[e]);
-            }
-            m = bi8_group_max<L>(m);
-            if ((lane & (L - 1)) == 0) s_tile[(c * BI8_WAVE + lane) / L][wave * kRowsPerWave + i] = m;
-            special |= !bi8_scale_is_ordinary(m);
-
-            uint32_t code[VEC];
-            if (__builtin_expect(special, 0)) {
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) code[e] = bi8_code_slow(f[e], m);
-            } else {
-                const float y = 1.0f / m;                               // correctly rounded reciprocal
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) code[e] = bi8_code_fast<NCORR>(f[e], m, y);
-            }
-            if (row < M && col < Kp) {
-                int8_t *dst = q + row * ldq + col;
-                if (ALIGNED || col + VEC <= Kp) {
-                    if constexpr (VEC == 4) {
-                        const uint32_t w = bi8_pack4(code[0], code[1], code[2], code[3]);
-                        if constexpr (ALIGNED) {
-                            if (keep) *(uint32_t *)dst = w;
-                            else __builtin_nontemporal_store(w, (uint32_t *)dst);
-                        }
-                        else *(bi8_u32_unaligned *)dst = w;
-                    } else {
-                        const bi8_v2u w = {bi8_pack4(code[0], code[1], code[2], code[3]), bi8_pack4(code[4], code[5], code[6], code[7])};
-                        if constexpr (ALIGNED) {
-                            if (keep) *(bi8_v2u *)dst = w;
-                            else __builtin_nontemporal_store(w, (bi8_v2u *)dst);
-                        }
-                        else *(bi8_v2u_unaligned *)dst = w;
-                    }
+                    if (keep) *(uint32_t *)dst = w[i][0];
+                    else __builtin_nontemporal_store(w[i][0], (uint32_t *)dst);
                 } else {
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e)
-                        if (col + e < Kp) dst[e] = (int8_t)(code[e] & 0xffu);
+                    *(bi8_u32_unaligned *)dst = w[i][0];
+                }
+            } else {
+                const bi8_v2u c = {w[i][0], w[i][1]};
+                if constexpr (ALIGNED) {
+                    if (keep) *(bi8_v2u *)dst = c;
+                    else __builtin_nontemporal_store(c, (bi8_v2u *)dst);
+                } else {
+                    *(bi8_v2u_unaligned *)dst = c;
                 }
             }
+        } else if constexpr (!ALIGNED) {
+#pragma unroll
+            for (int e = 0; e < VEC - 1; ++e)
+                if (e < room) dst[e] = (int8_t)((w[i][e / 4] >> (8 * (e & 3))) & 0xffu);
         }
     }
-    __syncthreads();
+    // The scales: straight from the lanes that hold them, or through LDS, so that each block's leave as a run of all the workgroup's rows.
     const int64_t jb0 = col0 / B;
-    for (int t = tid; t < NB * kRows; t += kThreads) {
-        const int j = t / kRows, r = t % kRows;
-        if (row0 + r < M && jb0 + j < nblk) scales[(jb0 + j) * M + row0 + r] = s_tile[j][r];
+    if constexpr (RPW == 1) {
+        const int64_t jb = jb0 + lane / L;
+        if ((lane & (L - 1)) == 0 && jb < nblk) scales[jb * M + row0] = m[0];
+    } else {
+        constexpr int kRows = 4 * RPW, NB = BI8_WAVE / L;
+        __shared__ float s_tile[NB][kRows + 1];
+        if ((lane & (L - 1)) == 0) {
+#pragma unroll
+            for (int i = 0; i < RPW; ++i) s_tile[lane / L][wave * RPW + i] = m[i];
+        }
+        __syncthreads();
+        const int64_t first = row0 - wave * RPW;
+        for (int t = threadIdx.x; t < NB * kRows; t += kThreads) {
+            const int j = t / kRows, r = t % kRows;
+            if (first + r < M && jb0 + j < nblk) scales[(jb0 + j) * M + first + r] = s_tile[j][r];
+        }
     }
 }
 
@@ -165,18 +233,36 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_generic(const void *__
     }
 }
 
-template <int DT, int L, bool ALIGNED>
-int launch_vec(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, int64_t Kp, int64_t ldx, int64_t ldq, hipStream_t st) {
+template <int DT, int L, bool ALIGNED, int RPW>
+int launch_rows(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, int64_t Kp, int64_t ldx, int64_t ldq, hipStream_t st) {
     constexpr int VEC = Bi8Vec<DT>::kElems;
     constexpr int B = L * VEC;
-    constexpr int TE = kChunks * BI8_WAVE * VEC;
-    const int64_t tiles_k = (Kp + TE - 1) / TE;
-    const int64_t tiles_m = (M + kRows - 1) / kRows;
-    if (tiles_k * tiles_m > 0x7fffffffLL) return BI8_ERR_TOO_LARGE;
+    constexpr int TE = BI8_WAVE * VEC;
+    constexpr int64_t kGridY = 32768;
+    const int64_t tiles_k = (Kp + TE - 1) / TE, tiles_m = (M + 4 * RPW - 1) / (4 * RPW);
+    const int64_t gy = tiles_m < kGridY ? tiles_m : kGridY, gz = (tiles_m + gy - 1) / gy;
+    if (tiles_k * gy * gz > 0x7fffffffLL || gz > 65535) return BI8_ERR_TOO_LARGE;
     const int64_t nblk = (Kp + B - 1) / B;
-    hipLaunchKernelGGL((quantize_rows_vec<DT, L, ALIGNED>), dim3((unsigned)(tiles_k * tiles_m)), dim3(kThreads), 0, st, x, q, scales, M, K, Kp,
-                       ldx, ldq, nblk, (int)tiles_k, M * Kp > kKeepCodes);
+    hipLaunchKernelGGL((quantize_rows_vec<DT, L, ALIGNED, RPW>), dim3((unsigned)tiles_k, (unsigned)gy, (unsigned)gz), dim3(kThreads), 0, st, x, q, scales, M, K, Kp,
+                       ldx, ldq, nblk, M * Kp > kKeepCodes);
     return bi8_launch_rc();
+}
+// Rows per wave: one where that leaves every CU at most 24 waves (a call of few rows is latency, and a wave's rows follow one another),
+// two up to 72, four beyond, where more loads in flight per wave pay.  us with 1 / 2 / 4 (before: four, 1 KiB loads that waited for
+// one another, and the IEEE path inside each row): bf16, block 128 16 x 4096 1.8 / 2.1 / 2.5 (2.8), 512 x 4096 2.6 / 2.7 / 2.9 (3.2), 2048 x
+// 4096 7.2 / 6.6 / 6.9 (7.4), 3000 x 4096 9.4 / 9.0 / 8.8 (9.3), 4096 x 4096 11.9 / 11.5 / 10.8 (11.5), 8192 x 8192 37.2 / 34.8 / 35.3 (35.4);
+// fp16 100 x 11008 2.3 / 2.7 / 3.0 (3.9), 300 x 16384 4.9 / 4.8 / 5.3 (5.4); fp32, block 32 1000 x 5004 7.6 / 7.5 / 7.0 (7.2).  Rows off 16-byte
+// boundaries run with one whatever the size: bf16 1000 x 5003 5.6 / 5.6 / 7.2 (9.1), 8192 x 50257 267 / 293 / 287 (283).
+constexpr int64_t kOneRowWaves = 24 * 256, kTwoRowWaves = 72 * 256;
+template <int DT, int L, bool ALIGNED>
+int launch_vec(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, int64_t Kp, int64_t ldx, int64_t ldq, hipStream_t st) {
+    constexpr int TE = BI8_WAVE * Bi8Vec<DT>::kElems;
+    const int64_t waves = M * ((Kp + TE - 1) / TE);
+    if constexpr (ALIGNED) {
+        if (waves > kTwoRowWaves) return launch_rows<DT, L, true, 4>(x, q, scales, M, K, Kp, ldx, ldq, st);
+        if (waves > kOneRowWaves) return launch_rows<DT, L, true, 2>(x, q, scales, M, K, Kp, ldx, ldq, st);
+    }
+    return launch_rows<DT, L, ALIGNED, 1>(x, q, scales, M, K, Kp, ldx, ldq, st);
 }
 
 template <int DT, bool ALIGNED>
