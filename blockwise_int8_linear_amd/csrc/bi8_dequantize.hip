@@ -1,15 +1,12 @@
 // Block dequantize (bi8_dequantize_rowwise): out = (scale * float(code)) * fp32(1/127), cast on store.
 // Replaces _dequantize_block_rowwise, triton_functions.py:468-490.  HBM-bound: one lane = one 128-bit store
 // of outputs (8 bf16/f16 or 4 fp32) per step, so every wave store covers 1 KiB of contiguous output.  Same
-// tiling as the quantizer: a workgroup owns 8 rows x 2 KiB of output row and first pulls its scales in
-// through LDS, so the block-major / row-minor scale array is read as runs of 8 consecutive rows.
+// tiling as the quantizer: a workgroup owns 8 rows x 2 KiB of output row (small calls: 4 x 1 KiB, short rows 16 x 1 KiB) and, with more
+// than a row per wave, first pulls its scales in through LDS, so the block-major / row-minor scale array is read as runs of 8 or 16 rows.
 #include "bi8_common.h"
 
 namespace {
 
-constexpr int kLoads = 4;          // wave-loads per lane per tile (8 and 16 measured slower)
-constexpr int kRpw = kLoads / 2;   // rows per wave
-constexpr int kRows = 4 * kRpw;    // rows per workgroup tile
 constexpr int kThreads = 256;
 
 // One lane = kOut outputs = one 16-byte store (8 bf16/f16 or 4 fp32), so every store instruction of a wave
@@ -42,95 +39,127 @@ template <int DT, bool ALIGNED> __device__ __forceinline__ void store_vec(void *
     }
 }
 
-// workgroup tile: 8 rows x (2 * 64 * kOut) codes; wave w owns rows 2w, 2w+1, two chunks of 64 * kOut codes each
+// One wave = R rows x NC chunks of 64 * kOut codes, one workgroup = four of them, one below the other.
 // ALIGNED: rows of q on boundaries of their 4- or 8-byte loads, rows of out on 16-byte boundaries, K a multiple of the elements per
 // store.  Otherwise (odd row lengths) whole chunks move with unaligned accesses and the last, partial chunk of a row element by
 // element, as in the quantizer; these stores are not marked non-temporal: a wave's run starts and ends inside a cache line whose
 // other part comes from the next wave, and the two are to meet in the L2.  Quantize + dequantize of fp32 [1000,5003], block 32:
 // 19.0 -> 15.3 us against dequantize_rows_generic (one code, one division and one scale read per output).
-template <int DT, bool ALIGNED>
+template <int DT, bool ALIGNED, int R, int NC>
 __global__ __launch_bounds__(kThreads) void dequantize_rows_vec(const int8_t *__restrict__ q, const float *__restrict__ scales,
                                                                 void *__restrict__ out, int64_t M, int64_t K, int64_t ldq,
-                                                                int64_t ldo, int64_t nblk, int log2b, int tiles_k) {
+                                                                int64_t ldo, int64_t nblk, int log2b) {
     constexpr int VEC = Out<DT>::kElems;
-    constexpr int TE = 2 * BI8_WAVE * VEC;         // codes per tile row
-    __shared__ float s_tile[TE / 8][kRows + 1];    // block size >= 8 on this path
+    constexpr int kRows = 4 * R;
+    constexpr int TE = NC * BI8_WAVE * VEC;        // codes per tile row
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int64_t tile_m = blockIdx.x / tiles_k;
-    const int tile_k = blockIdx.x % tiles_k;
-    const int64_t row0 = tile_m * kRows;
-    const int64_t col0 = (int64_t)tile_k * TE;
-    const int nb = (TE >> log2b) > 0 ? (TE >> log2b) : 1;      // blocks per tile row
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t first = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * kRows, row0 = first + wave * R;
+    if (R == 1 && row0 >= M) return;
+    const int64_t col0 = (int64_t)blockIdx.x * TE;
     const int64_t jb0 = col0 >> log2b;
+    const int left = (int)(K - col0 < TE ? K - col0 : TE);          // of a row's codes, from the tile's first column on
+    auto row_of = [&](int i) { return row0 + i < M ? row0 + i : M - 1; };
 
-    uint32_t raw[kLoads][VEC / 4];
+    uint32_t raw[R][NC][VEC / 4];
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int64_t row = row0 + wave * kRpw + (i >> 1);
-        const int64_t col = col0 + ((i & 1) * BI8_WAVE + lane) * VEC;
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int e = 0; e < VEC / 4; ++e) raw[i][e] = 0u;
-        if (row < M && col < K) {
-            const int8_t *src = q + row * ldq + col;
-            if constexpr (!ALIGNED) {
-                if (col + VEC <= K) {
-                    if constexpr (VEC == 8) {
-                        const bi8_v2u v = *(const bi8_v2u_unaligned *)src;
-                        raw[i][0] = v[0];
-                        raw[i][1] = v[1];
-                    } else {
-                        raw[i][0] = *(const bi8_u32_unaligned *)src;
-                    }
-                } else {                           // the row ends inside this chunk
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e)
-                        if (col + e < K) raw[i][e >> 2] |= (uint32_t)(uint8_t)src[e] << (8 * (e & 3));
+            for (int e = 0; e < VEC / 4; ++e) raw[i][c][e] = 0u;
+    auto load = [&](int i, int c) {
+        const int8_t *src = q + row_of(i) * ldq + col0 + c * BI8_WAVE * VEC + lane * VEC;
+        if constexpr (VEC == 8) {
+            const bi8_v2u v = ALIGNED ? __builtin_nontemporal_load((const bi8_v2u *)src) : (bi8_v2u)*(const bi8_v2u_unaligned *)src;
+            raw[i][c][0] = v[0];
+            raw[i][c][1] = v[1];
+        } else {
+            raw[i][c][0] = ALIGNED ? __builtin_nontemporal_load((const uint32_t *)src) : (uint32_t)*(const bi8_u32_unaligned *)src;
+        }
+    };
+    if (left == TE) {                              // (one branch: the first use of a load need not wait for the others)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) load(i, c);
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int mine = left - (c * BI8_WAVE + lane) * VEC;          // of the row's codes from this lane's first on
+            if (mine >= VEC) {
+#pragma unroll
+                for (int i = 0; i < R; ++i) load(i, c);
+            } else if (!ALIGNED && mine > 0) {                            // the row ends inside this chunk
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    const int8_t *src = q + row_of(i) * ldq + col0 + (c * BI8_WAVE + lane) * VEC;
+#pragma unroll
+                    for (int e = 0; e < VEC - 1; ++e)
+                        if (e < mine) raw[i][c][e >> 2] |= (uint32_t)(uint8_t)src[e] << (8 * (e & 3));
                 }
-            } else if constexpr (VEC == 8) {
-                const bi8_v2u v = __builtin_nontemporal_load((const bi8_v2u *)src);
-                raw[i][0] = v[0];
-                raw[i][1] = v[1];
-            } else {
-                raw[i][0] = __builtin_nontemporal_load((const uint32_t *)src);
             }
         }
     }
-    for (int t = tid; t < nb * kRows; t += kThreads) {
-        const int j = t / kRows, r = t % kRows;
-        float s = 0.0f;
-        if (row0 + r < M && jb0 + j < nblk) s = scales[(jb0 + j) * M + row0 + r];
-        s_tile[j][r] = s;
+
+    // one row per wave: its scales straight from memory; otherwise through LDS, read as runs of the workgroup's rows
+    constexpr int kMaxBlocks = R == 1 ? 1 : TE / 8;                       // block size >= 8 on this path
+    __shared__ float s_tile[kMaxBlocks][kRows + 1];
+    float s_lane = 0.0f;
+    if constexpr (R == 1) {
+        if (lane * VEC < left) s_lane = scales[(jb0 + ((lane * VEC) >> log2b)) * M + row0];
+    } else {
+        const int nb = (TE >> log2b) > 0 ? (TE >> log2b) : 1;             // blocks per tile row
+        for (int t = tid; t < nb * kRows; t += kThreads) {
+            const int j = t / kRows, r = t % kRows;
+            float s = 0.0f;
+            if (first + r < M && jb0 + j < nblk) s = scales[(jb0 + j) * M + first + r];
+            s_tile[j][r] = s;
+        }
+        __syncthreads();
     }
-    __syncthreads();
 
     const float inv127 = (float)(1.0 / 127.0);
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-        const int64_t row = row0 + wave * kRpw + (i >> 1);
-        const int incol = ((i & 1) * BI8_WAVE + lane) * VEC;
-        const int64_t col = col0 + incol;
-        if (row < M && col < K) {
-            const float s = s_tile[incol >> log2b][wave * kRpw + (i >> 1)];
+    for (int i = 0; i < R; ++i) {
+        if (row0 + i >= M) break;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int incol = (c * BI8_WAVE + lane) * VEC, mine = left - incol;
+            if (mine <= 0) continue;
+            const float s = R == 1 ? s_lane : s_tile[R == 1 ? 0 : incol >> log2b][wave * R + i];
             float v[VEC];
 #pragma unroll
             for (int e = 0; e < VEC / 4; ++e) {
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const int code = (int)(raw[i][e] << (24 - 8 * b)) >> 24;     // sign-extended byte b
-                    v[4 * e + b] = (s * (float)code) * inv127;                   // two roundings, left to right
+                    const int code = (int)(raw[i][c][e] << (24 - 8 * b)) >> 24;     // sign-extended byte b
+                    v[4 * e + b] = (s * (float)code) * inv127;                      // two roundings, left to right
                 }
             }
-            if (ALIGNED || col + VEC <= K) {
-                store_vec<DT, ALIGNED>(out, row * ldo + col, v);
+            const int64_t at = (row0 + i) * ldo + col0 + incol;
+            if (ALIGNED || mine >= VEC) {
+                store_vec<DT, ALIGNED>(out, at, v);
             } else {
 #pragma unroll
-                for (int e = 0; e < VEC; ++e)
-                    if (col + e < K) bi8_store_elem<DT>(out, row * ldo + col + e, v[e]);
+                for (int e = 0; e < VEC - 1; ++e)
+                    if (e < mine) bi8_store_elem<DT>(out, at + e, v[e]);
             }
         }
     }
+}
+
+template <int DT, bool ALIGNED, int R, int NC>
+int launch_rows(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block, hipStream_t st) {
+    constexpr int TE = NC * BI8_WAVE * Out<DT>::kElems;
+    constexpr int64_t kGridY = 32768;
+    const int64_t tiles_k = (K + TE - 1) / TE, tiles_m = (M + 4 * R - 1) / (4 * R);
+    const int64_t gy = tiles_m < kGridY ? tiles_m : kGridY, gz = (tiles_m + gy - 1) / gy;
+    if (tiles_k * gy * gz > 0x7fffffffLL || gz > 65535) return BI8_ERR_TOO_LARGE;
+    hipLaunchKernelGGL((dequantize_rows_vec<DT, ALIGNED, R, NC>), dim3((unsigned)tiles_k, (unsigned)gy, (unsigned)gz), dim3(kThreads), 0, st, q, scales, out, M, K, ldq, ldo,
+                       (K + block - 1) / block, __builtin_ctz((unsigned)block));
+    return bi8_launch_rc();
 }
 
 template <int DT>
@@ -154,28 +183,30 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_generic(const int8_t
     }
 }
 
+// One row and one chunk per wave where that is few waves (a call of few rows is latency; rows off 16-byte boundaries: up to more of
+// them), else two rows of two chunks, or four rows where a row is one chunk.  us with one / two rows (before: two, loads that waited for
+// one another): bf16, block 128 16 x 4096 1.7 / 2.4 (2.7), 512 x 4096 2.6 / 3.1 (3.2), 2048 x 4096 6.3 / 5.2 (5.1), 8192 x 8192 37.3 / 32.6
+// (33.6); fp16 100 x 11008 2.1 / 2.8 (2.9), 300 x 16384 4.3 / 3.9 (4.1); odd rows fp32 1000 x 5003 6.4 / 6.8 (6.9), bf16 8192 x 5001 34.5 / 31.0
+// (31.1).
+constexpr int64_t kOneRowWaves = 24 * 256, kOneRowWavesRagged = 96 * 256;
+template <int DT, bool ALIGNED>
+int launch_vec(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block, hipStream_t st) {
+    constexpr int kChunk = BI8_WAVE * Out<DT>::kElems;
+    if (M * ((K + kChunk - 1) / kChunk) <= (ALIGNED ? kOneRowWaves : kOneRowWavesRagged)) return launch_rows<DT, ALIGNED, 1, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+    if (K <= kChunk) return launch_rows<DT, ALIGNED, 4, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+    return launch_rows<DT, ALIGNED, 2, 2>(q, scales, out, M, K, ldq, ldo, block, st);
+}
+
 template <int DT>
 int dispatch(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block,
              hipStream_t st) {
     constexpr int VEC = Out<DT>::kElems;
-    constexpr int TE = 2 * BI8_WAVE * VEC;
     // Blocks that no chunk straddles, and elements on boundaries of their own size (what the unaligned accesses need); a row shorter
     // than a chunk would be all element by element.
     const bool vec_ok = bi8_pow2(block) && block >= 8 && K >= VEC && bi8_aligned(out, DT == BI8_F32 ? 4 : 2);
     if (vec_ok) {
         const bool aligned = K % VEC == 0 && ldq % VEC == 0 && ldo % VEC == 0 && bi8_aligned(q, VEC) && bi8_aligned(out, 16);
-        const int64_t tiles_k = (K + TE - 1) / TE;
-        const int64_t tiles_m = (M + kRows - 1) / kRows;
-        if (tiles_k * tiles_m > 0x7fffffffLL) return BI8_ERR_TOO_LARGE;
-        const int64_t nblk = (K + block - 1) / block;
-        const dim3 grid((unsigned)(tiles_k * tiles_m));
-        const int log2b = __builtin_ctz((unsigned)block);
-        if (aligned) {
-            hipLaunchKernelGGL((dequantize_rows_vec<DT, true>), grid, dim3(kThreads), 0, st, q, scales, out, M, K, ldq, ldo, nblk, log2b, (int)tiles_k);
-        } else {
-            hipLaunchKernelGGL((dequantize_rows_vec<DT, false>), grid, dim3(kThreads), 0, st, q, scales, out, M, K, ldq, ldo, nblk, log2b, (int)tiles_k);
-        }
-        return bi8_launch_rc();
+        return aligned ? launch_vec<DT, true>(q, scales, out, M, K, ldq, ldo, block, st) : launch_vec<DT, false>(q, scales, out, M, K, ldq, ldo, block, st);
     }
     int64_t grid = M * ((K + 2047) / 2048);
     if (grid > (1 << 20)) grid = 1 << 20;
