@@ -107,6 +107,39 @@ template <int L> __device__ __forceinline__ float bi8_group_max(float m) {
     return m;
 }
 
+// ---- the same maximum on the elements' bits -----------------------------------------------------------
+// The largest magnitude of a lane's 16 bytes, as bits: magnitudes order like their bits, and a NaN lies above infinity.  16-bit
+// types: the maxima of the low and of the high halves, which bi8_magnitude_of() joins.
+template <int DT> __device__ __forceinline__ uint32_t bi8_larger_bits(uint32_t a, uint32_t b) {
+    if constexpr (DT == BI8_F32) return max(a, b);
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+template <int DT> __device__ __forceinline__ uint32_t bi8_abs_bits(uint32_t w) { return w & (DT == BI8_F32 ? 0x7fffffffu : 0x7fff7fffu); }
+template <int DT> __device__ __forceinline__ uint32_t bi8_magnitude_bits(const bi8_v4u &raw) {
+    uint32_t m = bi8_abs_bits<DT>(raw[0]);
+#pragma unroll
+    for (int e = 1; e < 4; ++e) m = bi8_larger_bits<DT>(m, bi8_abs_bits<DT>(raw[e]));
+    return m;
+}
+template <int CTRL> __device__ __forceinline__ uint32_t bi8_dpp_bits(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true); }
+// over aligned groups of L lanes (the steps of bi8_group_max)
+template <int DT, int L> __device__ __forceinline__ uint32_t bi8_group_bits(uint32_t m) {
+    if constexpr (L >= 2) m = bi8_larger_bits<DT>(m, bi8_dpp_bits<0xB1>(m));
+    if constexpr (L >= 4) m = bi8_larger_bits<DT>(m, bi8_dpp_bits<0x4E>(m));
+    if constexpr (L >= 8) m = bi8_larger_bits<DT>(m, bi8_dpp_bits<0x141>(m));
+    if constexpr (L >= 16) m = bi8_larger_bits<DT>(m, bi8_dpp_bits<0x140>(m));
+    if constexpr (L >= 32) m = bi8_larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 16, 64));
+    if constexpr (L >= 64) m = bi8_larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+    return m;
+}
+// the magnitude itself; a NaN stays one
+template <int DT> __device__ __forceinline__ float bi8_magnitude_of(uint32_t m) {
+    if constexpr (DT == BI8_F32) return bi8_u2f(m);
+    const uint32_t h = max(m & 0xffffu, m >> 16);
+    return DT == BI8_BF16 ? bi8_from_bf16_bits(h) : bi8_from_f16_bits(h);
+}
+
 // ---- exact block quantization of one element ----------------------------------------------------
 // code = rint_even( fl32( 127 * fl32( v / s ) ) ), the reference's llrint(127. * (x / max_val))
 // (triton_functions.py:212).  Built with -ffp-contract=off, so the product and the magic add below
@@ -120,6 +153,10 @@ template <int L> __device__ __forceinline__ float bi8_group_max(float m) {
 __device__ __forceinline__ bool bi8_scale_is_ordinary(float s) {
     return s >= 8.6736173798840355e-19f && s <= 1.2676506002282294e+30f;
 }
+
+// ... and a scale of 0, whose elements are zeros: with y = 0 for its reciprocal their codes come out as 0.
+__device__ __forceinline__ bool bi8_scale_is_fast(float s) { return bi8_scale_is_ordinary(s) || s == 0.0f; }
+__device__ __forceinline__ float bi8_recip_of_scale(float s) { return s > 0.0f ? 1.0f / s : 0.0f; }       // correctly rounded
 
 // Correctly rounded v / s from y = fl32(1/s), for |v| <= s and s ordinary: a rounded product and
 // NCORR FMA corrections.  Two corrections are exact for any binary32 operands (Markstein: the first
@@ -143,12 +180,11 @@ template <int NCORR> __device__ __forceinline__ uint32_t bi8_code_fast(float v, 
 }
 
 // any scale, any element: IEEE division; zero blocks and NaN elements give code 0
+// (no branches: kernels hold many copies of this)
 __device__ __forceinline__ uint32_t bi8_code_slow(float v, float s) {
-    if (!(s > 0.0f) || v != v) return 0u;
-    float t = 127.0f * (v / s);
-    if (t != t) return 0u;                       // inf / inf
-    t = __builtin_fminf(__builtin_fmaxf(t, -127.0f), 127.0f);
-    return bi8_f2u(t + BI8_MAGIC);
+    const float t = 127.0f * (v / s);                // NaN: of inf / inf, 0 / 0
+    const float c = __builtin_fminf(__builtin_fmaxf(t, -127.0f), 127.0f);
+    return s > 0.0f && t == t ? bi8_f2u(c + BI8_MAGIC) : 0u;
 }
 
 __device__ __forceinline__ uint32_t bi8_pack4(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3) {

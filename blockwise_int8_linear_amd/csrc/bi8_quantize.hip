@@ -21,45 +21,6 @@ constexpr int kThreads = 256;
 // 116.8 -> 117.3.
 constexpr int64_t kKeepCodes = 32 << 20;
 
-// The largest magnitude of a lane's 16 bytes, as bits: magnitudes order like their bits, and a NaN lies above infinity.  16-bit
-// types: the maxima of the low and of the high halves, which magnitude_of() joins.
-template <int DT> __device__ __forceinline__ uint32_t magnitude_bits(const bi8_v4u &raw) {
-    if constexpr (DT == BI8_F32) {
-        uint32_t m = raw[0] & 0x7fffffffu;
-#pragma unroll
-        for (int e = 1; e < 4; ++e) m = max(m, raw[e] & 0x7fffffffu);
-        return m;
-    } else {
-        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-        u16x2 m = __builtin_bit_cast(u16x2, raw[0] & 0x7fff7fffu);
-#pragma unroll
-        for (int e = 1; e < 4; ++e) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, raw[e] & 0x7fff7fffu));
-        return __builtin_bit_cast(uint32_t, m);
-    }
-}
-template <int DT> __device__ __forceinline__ uint32_t larger_bits(uint32_t a, uint32_t b) {
-    if constexpr (DT == BI8_F32) return max(a, b);
-    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
-}
-template <int CTRL> __device__ __forceinline__ uint32_t dpp_bits(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true); }
-// over aligned groups of L lanes (the steps of bi8_group_max)
-template <int DT, int L> __device__ __forceinline__ uint32_t group_bits(uint32_t m) {
-    if constexpr (L >= 2) m = larger_bits<DT>(m, dpp_bits<0xB1>(m));
-    if constexpr (L >= 4) m = larger_bits<DT>(m, dpp_bits<0x4E>(m));
-    if constexpr (L >= 8) m = larger_bits<DT>(m, dpp_bits<0x141>(m));
-    if constexpr (L >= 16) m = larger_bits<DT>(m, dpp_bits<0x140>(m));
-    if constexpr (L >= 32) m = larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 16, 64));
-    if constexpr (L >= 64) m = larger_bits<DT>(m, (uint32_t)__shfl_xor((int)m, 32, 64));
-    return m;
-}
-// the magnitude itself; a NaN stays one
-template <int DT> __device__ __forceinline__ float magnitude_of(uint32_t m) {
-    if constexpr (DT == BI8_F32) return bi8_u2f(m);
-    const uint32_t h = max(m & 0xffffu, m >> 16);
-    return DT == BI8_BF16 ? bi8_from_bf16_bits(h) : bi8_from_f16_bits(h);
-}
-
 // One wave = RPW rows x 1 KiB, one workgroup = four of them, one below the other.
 // ALIGNED: rows of x on 16-byte boundaries, K a multiple of the elements per 16 bytes, rows of q aligned to their
 // 4- or 8-byte stores.  Otherwise (odd row length or leading dimension, e.g. the GPT-2 vocabulary 50257) whole chunks
@@ -67,7 +28,7 @@ template <int DT> __device__ __forceinline__ float magnitude_of(uint32_t m) {
 // keep: the codes' stores of aligned rows are not marked non-temporal (see kKeepCodes).
 // Kp: columns written, K or more: zero codes and zero scales past the row's end (the padding that a GEMM contracted over K wants).
 // A row past the end reads the last one and is not stored: the rows' loads do not branch, nor does their arithmetic, so that the rows' chains of dependent instructions run side by side: a block that needs the IEEE division (a
-// scale of 0, subnormal, huge or infinite, a NaN) is done over in one place behind them.
+// subnormal, huge or infinite scale, a NaN) is done over in one place behind them.
 template <int DT, int L, bool ALIGNED, int RPW>
 __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const void *__restrict__ x, int8_t *__restrict__ q,
                                                               float *__restrict__ scales, int64_t M, int64_t K, int64_t Kp,
@@ -120,29 +81,23 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const void *__rest
     uint32_t w[RPW][VEC / 4];
     bool slow = false;
 #pragma unroll
-    for (int i = 0; i < RPW; ++i) m[i] = magnitude_of<DT>(group_bits<DT, L>(magnitude_bits<DT>(raw[i])));
+    for (int i = 0; i < RPW; ++i) m[i] = bi8_magnitude_of<DT>(bi8_group_bits<DT, L>(bi8_magnitude_bits<DT>(raw[i])));
 #pragma unroll
     for (int i = 0; i < RPW; ++i) {
         float f[VEC];
         bi8_unpack<DT>(raw[i], f);
-        slow |= mine > 0 && !bi8_scale_is_ordinary(m[i]);
-        const float y = 1.0f / m[i];                                    // correctly rounded reciprocal
+        slow |= !bi8_scale_is_fast(m[i]);
+        const float y = bi8_recip_of_scale(m[i]);
         uint32_t code[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) code[e] = bi8_code_fast<NCORR>(f[e], m[i], y);
 #pragma unroll
         for (int e = 0; e < VEC; e += 4) w[i][e / 4] = bi8_pack4(code[e], code[e + 1], code[e + 2], code[e + 3]);
     }
-    if (left < TE) {                                 // past the row's end: codes of zero
-#pragma unroll
-        for (int i = 0; i < RPW; ++i)
-#pragma unroll
-            for (int e = 0; e < VEC / 4; ++e) w[i][e] = mine > 0 ? w[i][e] : 0u;
-    }
     if (__builtin_expect(__any(slow), 0)) {
 #pragma unroll
         for (int i = 0; i < RPW; ++i) {
-            if (!bi8_scale_is_ordinary(m[i])) {                         // (the same for all lanes of a block)
+            if (!bi8_scale_is_fast(m[i])) {                             // (the same for all lanes of a block)
                 float f[VEC], s = 0.0f;
                 bi8_unpack<DT>(raw[i], f);
 #pragma unroll

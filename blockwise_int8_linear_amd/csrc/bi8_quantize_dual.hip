@@ -4,6 +4,11 @@
 // quantizes each of X, W and G twice, once per direction (block_linear.py:77-78, :92-94, :100-103): with this kernel
 // every one of them is read from HBM once.
 //
+// What bounds it: memory, at 5.0 TB/s of the 272 MB of bf16 [8192,8192], block 128 (a copy with these access widths: 6.2), behind it ~20
+// vector instructions per element.  us, a branch around every load and store, per-element NaN tests and the IEEE path inside each
+// row -> this: bf16 block 128 [8192,8192] 57.9 -> 54.2, [4096,11008] 44.4 -> 41.8, [11008,4096] 40.8 -> 39.0; block 64 [8192,3072] with
+// column sums 29.0 -> 23.2, [8192,50257] 414 -> 380 ([8192,50304]: 360 -> 345); fp32 [8192,8192] 114 -> 85 (three workgroups per CU for two).
+//
 // A workgroup owns a 128 x 128 tile, held in registers as two 64-column halves (16 bytes per lane per row pass; the
 // next tile's loads are issued while this one is processed).  The row direction is finished straight from the
 // registers: the lanes of one row reduce their absmax with DPP, quantize and store their codes.  The column direction
@@ -28,81 +33,111 @@ constexpr int kThreads = 256;
 // are all long runs in memory.
 // Measured on bf16 [8192,8192]: 16 x 16 tiles 64.0 us, row by row 65.4, 8 x 32 64.6, 32 x 8 69.
 constexpr int kSBR = 16, kSBC = 16;
-__device__ __forceinline__ void tile_coords(int64_t t, int64_t tiles_r, int64_t tiles_c, int64_t &tr, int64_t &tc) {
-    const int64_t band = t / (kSBR * tiles_c);
-    const int64_t rows_b = (tiles_r - band * kSBR < kSBR) ? (tiles_r - band * kSBR) : kSBR;
-    const int64_t in = t - band * kSBR * tiles_c;
-    const int64_t chunk = in / (rows_b * kSBC);
-    const int64_t wc = (tiles_c - chunk * kSBC < kSBC) ? (tiles_c - chunk * kSBC) : kSBC;
-    const int64_t in2 = in - chunk * rows_b * kSBC;
-    tr = band * kSBR + in2 / wc;
-    tc = chunk * kSBC + in2 % wc;
+// DOWN: inside a chunk column by column instead of row by row.  Two tiles side by side are then kSBR apart in the order, a multiple of
+// the eight XCDs: where rows of x start off 128-byte lines, both read the line that their border cuts, and it is in their L2.
+template <bool DOWN> __device__ __forceinline__ void tile_coords(int t, int tiles_r, int tiles_c, int &tr, int &tc) {
+    const int band = t / (kSBR * tiles_c);
+    const int rows_b = (tiles_r - band * kSBR < kSBR) ? (tiles_r - band * kSBR) : kSBR;
+    const int in = t - band * kSBR * tiles_c;
+    const int chunk = in / (rows_b * kSBC);
+    const int wc = (tiles_c - chunk * kSBC < kSBC) ? (tiles_c - chunk * kSBC) : kSBC;
+    const int in2 = in - chunk * rows_b * kSBC;
+    tr = band * kSBR + (DOWN ? in2 % rows_b : in2 / wc);
+    tc = chunk * kSBC + (DOWN ? in2 / rows_b : in2 % wc);
 }
 constexpr int kQPitch = kTR + 16;  // code tile pitch in bytes: rows stay 16-byte aligned
 
-// ALIGNED: rows of x start on 16-byte boundaries and C is a multiple of the elements per 16 bytes, rows of q on 8-byte
-// boundaries.  Otherwise whole 16-byte chunks move with unaligned accesses and the last, partial chunk of a row
-// element by element.
+// element k (of one or two) of a 32-bit word of x
+template <int DT> __device__ __forceinline__ float word_elem(uint32_t d, int k) {
+    if constexpr (DT == BI8_F32) return bi8_u2f(d);
+    else if constexpr (DT == BI8_BF16) return k == 0 ? bi8_u2f(d << 16) : bi8_u2f(d & 0xffff0000u);
+    else return bi8_from_f16_bits(k == 0 ? d & 0xffffu : d >> 16);
+}
+
+template <int DT, int B, bool SUM, int NH> struct DualLds {
+    static constexpr int kES = DT == BI8_F32 ? 4 : 2;              // bytes per element
+    static constexpr int kCPT = 4 / kES;                           // columns per thread in the column walk: one 32-bit word
+    static constexpr int kG = kThreads / (kTC / kCPT);             // row groups: 4 (fp32) or 8
+    static constexpr int kXPitch = kTC * kES + (kES == 4 ? 0 : 16);      // bytes, 16-byte aligned (as in bi8_quantize_transposed)
+    // the tile's row-direction scales, [block along the row][tile row]: stored from here as runs of kTR consecutive rows
+    // (single 4-byte stores from the lanes that hold them cost the fabric a 32-byte write each)
+    static constexpr int kNRB = (NH * kTC + B - 1) / B;
+    __attribute__((aligned(16))) uint8_t x[kTR * kXPitch];
+    __attribute__((aligned(16))) uint8_t q[kTC * kQPitch];
+    uint32_t max[kG][kTC / kCPT];
+    float sum[SUM ? kG : 1][kTC];
+    float rs[kNRB][kTR];
+};
+
+// ALIGNED: rows of x start on 16-byte boundaries and C is a multiple of the elements per 16 bytes.  Otherwise whole 16-byte chunks move
+// with unaligned accesses and the last, partial chunk of a row element by element.
 // NH: halves per tile.  2 is the tile described above; 1 (a 128 x 64 tile, blocks of at most 64) doubles the number of
 // workgroups for inputs too small to occupy the chip with full tiles.
-// Rp, Cp: rows and columns written, the matrix' own or more: zeros past its end.  The workgroup's tiles: first_tile, first_tile +
-// tile_step, ... of ntiles, tiles_c in a row of tiles.
-template <int DT, int B, bool ALIGNED, bool SUM, int NH>
-__device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales, int8_t *__restrict__ qT,
-                                           float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx, int64_t ldq,
-                                           int64_t ldqt, int64_t Rp, int64_t Cp, int64_t tiles_c, int64_t ntiles, int64_t first_tile, int64_t tile_step) {
+// Rp, Cp: rows and columns written, the matrix' own or more: zeros past its end.
+// FULL: the tiles that lie inside the matrix, otherwise those at its right and lower end.  Every load and store of a full tile is
+// unconditional, so that the wait for the next tile's loads is for those, and not for the stores issued behind them: with a branch
+// around either the compiler cannot count them and waits for everything, a tile's codes on their way to memory included.
+// The workgroup's tiles: first_tile, first_tile + tile_step, ...
+template <int DT, int B, bool ALIGNED, bool SUM, int NH, bool FULL>
+__device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales,
+                                           int8_t *__restrict__ qT, float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx,
+                                           int64_t ldq, int64_t ldqt, int64_t Rp, int64_t Cp, int first_tile, int tile_step) {
+    using L = DualLds<DT, B, SUM, NH>;
     constexpr int VEC = Bi8Vec<DT>::kElems;
-    constexpr int64_t ES = 16 / VEC;
+    constexpr int ES = L::kES, CPT = L::kCPT, G = L::kG;
     constexpr int LPR = kTC / VEC;                 // lanes per half row: 8 (16-bit) or 16 (fp32)
     constexpr int RPP = kThreads / LPR;            // rows per load pass
     constexpr int NP = kTR / RPP;                  // load passes per half
     constexpr int NCORR = (DT == BI8_F32) ? 2 : 1;
-    constexpr int ESZ = (int)ES;                   // bytes per element
-    constexpr int CPT = 4 / ESZ;                   // columns per thread in the column walk: one 32-bit word
-    constexpr int G = kThreads / (kTC / CPT);      // row groups: 4 (fp32) or 8
-    constexpr int RPT = kTR / G;                   // rows per thread: 32 (fp32) or 16
+    constexpr int RPT = kTR / G;                   // rows per thread in the column walk: 32 (fp32) or 16
     constexpr int GPW = B / RPT;                   // row groups per column block
-    constexpr int kXPitch = kTC * ESZ + (ESZ == 4 ? 0 : 16);   // bytes, 16-byte aligned (as in bi8_quantize_transposed)
     constexpr int LB = (B < kTC ? B : kTC) / VEC;  // lanes of one half row that share a row block
+    constexpr int TC = NH * kTC;                   // columns of a tile
     static_assert(B == 32 || B == 64 || B == 128, "tile = one or more whole blocks in both directions");
     static_assert(NH == 2 || (NH == 1 && B <= kTC), "a row block lies inside the tile");
-    __shared__ __attribute__((aligned(16))) uint8_t s_x[kTR * kXPitch];
-    __shared__ float s_max[G][kTC];
-    __shared__ float s_sum[SUM ? G : 1][kTC];
-    __shared__ __attribute__((aligned(16))) uint8_t s_q[kTC * kQPitch];
-    // the tile's row-direction scales, [block along the row][tile row]: stored from here as runs of kTR consecutive rows
-    // (single 4-byte stores from the lanes that hold them cost the fabric a 32-byte write each)
-    constexpr int NRB = (NH * kTC + B - 1) / B;
-    __shared__ float s_rs[NRB][kTR];
+    static_assert(GPW > 1 || B == RPT, "a thread's rows are inside one block");
 
     const int tid = threadIdx.x;
-    const char *xb = (const char *)x;
     const bool wide_q = (((uintptr_t)q | (uintptr_t)ldq) & 15) == 0;     // rows of q on 16-byte boundaries: 16-byte code stores
     const int lr = tid / LPR;                      // row inside a pass
     const int cc = (tid % LPR) * VEC;              // first column of this lane inside a half
 
-    const int64_t tiles_r = (Rp + kTR - 1) / kTR;
-    auto load_half = [&](int64_t tile, int h, bi8_v4u *raw) {
-        int64_t tr = 0, tc = 0;
-        if (tile < ntiles) tile_coords(tile, tiles_r, tiles_c, tr, tc);
-        const int64_t r0 = tr * kTR;
-        const int64_t c0 = tc * (NH * kTC) + h * kTC;
+    const int full_r = (int)(R / kTR), full_c = (int)(C / TC);
+    const int all_r = (int)((Rp + kTR - 1) / kTR), all_c = (int)((Cp + TC - 1) / TC);
+    const int right = all_r * (all_c - full_c);    // tiles in the columns behind the full ones; then those below them
+    const int ntiles = FULL ? full_r * full_c : right + (all_r - full_r) * full_c;
+    auto coords = [&](int t, int &tr, int &tc) {
+        if constexpr (FULL) {
+            tile_coords<!ALIGNED>(t, full_r, full_c, tr, tc);
+        } else if (t < right) {
+            tr = t / (all_c - full_c);
+            tc = full_c + t % (all_c - full_c);
+        } else {
+            tr = full_r + (t - right) / full_c;
+            tc = (t - right) % full_c;
+        }
+    };
+    const char *x_lane = (const char *)x + ((int64_t)lr * ldx + cc) * ES;
+    auto load_half = [&](int tr, int tc, int h, bi8_v4u *raw) {
+        const int64_t r0 = (int64_t)tr * kTR, c0 = (int64_t)tc * TC + h * kTC;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const int r = p * RPP + lr;
-            raw[p] = bi8_v4u{0u, 0u, 0u, 0u};
-            if (tile < ntiles && r0 + r < R && c0 + cc < C) {
-                const char *src = xb + ((r0 + r) * ldx + c0 + cc) * ES;
-                if constexpr (ALIGNED) {
-                    raw[p] = __builtin_nontemporal_load((const bi8_v4u *)src);
-                } else if (c0 + cc + VEC <= C) {
-                    raw[p] = *(const bi8_v4u_unaligned *)src;
-                } else {                           // the row ends inside this chunk
+            const char *src = x_lane + ((r0 + p * RPP) * ldx + c0) * ES;
+            if constexpr (FULL) {
+                if constexpr (ALIGNED) raw[p] = __builtin_nontemporal_load((const bi8_v4u *)src);
+                else raw[p] = *(const bi8_v4u_unaligned *)src;
+            } else {
+                raw[p] = bi8_v4u{0u, 0u, 0u, 0u};
+                if (r0 + p * RPP + lr < R && c0 + cc < C) {
+                    if (c0 + cc + VEC <= C) {
+                        raw[p] = *(const bi8_v4u_unaligned *)src;
+                    } else {                       // the row ends inside this chunk
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        if (c0 + cc + e < C) {
-                            if constexpr (DT == BI8_F32) raw[p][e] = ((const uint32_t *)src)[e];
-                            else raw[p][e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
+                        for (int e = 0; e < VEC; ++e) {
+                            if (c0 + cc + e < C) {
+                                if constexpr (DT == BI8_F32) raw[p][e] = ((const uint32_t *)src)[e];
+                                else raw[p][e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
+                            }
                         }
                     }
                 }
@@ -110,94 +145,117 @@ __device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *_
         }
     };
 
+    if (first_tile >= ntiles) return;
+    int tr, tc;
+    coords(first_tile, tr, tc);
     bi8_v4u raw[NH][NP];
 #pragma unroll
-    for (int h = 0; h < NH; ++h) load_half(first_tile, h, raw[h]);
-    for (int64_t tile = first_tile; tile < ntiles; tile += tile_step) {
-        int64_t tr, tc;
-        tile_coords(tile, tiles_r, tiles_c, tr, tc);
-        const int64_t r0 = tr * kTR;
-        const int64_t cbase = tc * (NH * kTC);
+    for (int h = 0; h < NH; ++h) load_half(tr, tc, h, raw[h]);
+    for (int tile = first_tile;;) {
+        const int64_t r0 = (int64_t)tr * kTR, cbase = (int64_t)tc * TC;
+        const int next = tile + tile_step;
+        int tr_n = 0, tc_n = 0;
+        if (next < ntiles) coords(next, tr_n, tc_n);
 
         // ---- along the rows, from the registers ----------------------------------------------------------------
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
             const int64_t row = r0 + p * RPP + lr;
-            float f[NH][VEC];
+            uint32_t bits[NH];
             float m[NH];
-            bool special[NH];
+            bi8_v2u wq[NH];                        // (fp32: four codes, the first word)
+            bool slow = false;
 #pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                bi8_unpack<DT>(raw[h][p], f[h]);
-                m[h] = 0.0f;
-                special[h] = false;
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    m[h] = __builtin_fmaxf(m[h], __builtin_fabsf(f[h][e]));
-                    special[h] |= (f[h][e] != f[h][e]);
-                }
-            }
+            for (int h = 0; h < NH; ++h) bits[h] = bi8_magnitude_bits<DT>(raw[h][p]);
             if constexpr (B == 2 * kTC) {
-                m[0] = m[NH - 1] = bi8_group_max<LPR>(__builtin_fmaxf(m[0], m[NH - 1]));
+                m[0] = m[NH - 1] = bi8_magnitude_of<DT>(bi8_group_bits<DT, LPR>(bi8_larger_bits<DT>(bits[0], bits[NH - 1])));
             } else {
 #pragma unroll
-                for (int h = 0; h < NH; ++h) m[h] = bi8_group_max<LB>(m[h]);
+                for (int h = 0; h < NH; ++h) m[h] = bi8_magnitude_of<DT>(bi8_group_bits<DT, LB>(bits[h]));
             }
-            // (16-bit inputs, two halves, aligned: a lane's 8 codes of each half are exchanged with its neighbour's so that the
-            // even lane stores 16 consecutive codes of the left half and the odd lane 16 of the right half -- the eight lanes of
-            // a row then write the row's whole 128-byte line in one instruction instead of two halves in two)
-            constexpr bool kPairStores = ALIGNED && VEC == 8 && NH == 2;
-            bi8_v2u wq[NH];
 #pragma unroll
             for (int h = 0; h < NH; ++h) {
-                const int64_t col = cbase + h * kTC + cc;
-                const bool live = row < R && col < Cp;
-                if ((tid % LB) == 0 && (B != 2 * kTC || h == 0)) s_rs[(h * kTC + cc) / B][p * RPP + lr] = m[h];
-                const bool slow = special[h] | !bi8_scale_is_ordinary(m[h]);
+                float f[VEC];
+                bi8_unpack<DT>(raw[h][p], f);
+                slow |= !bi8_scale_is_fast(m[h]);
+                const float y = bi8_recip_of_scale(m[h]);
                 uint32_t code[VEC];
-                if (__builtin_expect(slow, 0)) {
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) code[e] = bi8_code_slow(f[h][e], m[h]);
-                } else {
-                    const float y = 1.0f / m[h];
+                for (int e = 0; e < VEC; ++e) code[e] = bi8_code_fast<NCORR>(f[e], m[h], y);
+                wq[h][0] = bi8_pack4(code[0], code[1], code[2], code[3]);
+                if constexpr (VEC == 8) wq[h][1] = bi8_pack4(code[4], code[5], code[6], code[7]);
+            }
+            if (__builtin_expect(__any(slow), 0)) {          // (the lanes of a block agree on it)
+                float s[NH];
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) code[e] = bi8_code_fast<NCORR>(f[h][e], m[h], y);
+                for (int h = 0; h < NH; ++h) {
+                    float f[VEC];
+                    bi8_unpack<DT>(raw[h][p], f);
+                    s[h] = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) s[h] = __builtin_fmaxf(s[h], __builtin_fabsf(f[e]));     // ignores NaN
                 }
-                if constexpr (kPairStores) {
-                    wq[h] = bi8_v2u{bi8_pack4(code[0], code[1], code[2], code[3]), bi8_pack4(code[4], code[5], code[6], code[7])};
-                    if (!wide_q && live) __builtin_nontemporal_store(wq[h], (bi8_v2u *)(q + row * ldq + col));
-                } else if (live) {
-                    int8_t *dst = q + row * ldq + col;
-                    if (ALIGNED || col + VEC <= Cp) {
-                        if constexpr (VEC == 4) {
-                            const uint32_t w = bi8_pack4(code[0], code[1], code[2], code[3]);
-                            if constexpr (ALIGNED) __builtin_nontemporal_store(w, (uint32_t *)dst);
-                            else *(bi8_u32_unaligned *)dst = w;
-                        } else {
-                            const bi8_v2u w = {bi8_pack4(code[0], code[1], code[2], code[3]), bi8_pack4(code[4], code[5], code[6], code[7])};
-                            if constexpr (ALIGNED) __builtin_nontemporal_store(w, (bi8_v2u *)dst);
-                            else *(bi8_v2u_unaligned *)dst = w;
-                        }
-                    } else {
+                if constexpr (B == 2 * kTC) {
+                    s[0] = s[NH - 1] = bi8_group_max<LPR>(__builtin_fmaxf(s[0], s[NH - 1]));
+                } else {
 #pragma unroll
-                        for (int e = 0; e < VEC; ++e)
-                            if (col + e < Cp) dst[e] = (int8_t)(code[e] & 0xffu);
-                    }
+                    for (int h = 0; h < NH; ++h) s[h] = bi8_group_max<LB>(s[h]);
+                }
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+                    if (bi8_scale_is_fast(m[h])) continue;
+                    float f[VEC];
+                    bi8_unpack<DT>(raw[h][p], f);
+                    m[h] = s[h];
+                    uint32_t code[VEC];
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) code[e] = bi8_code_slow(f[e], s[h]);
+                    wq[h][0] = bi8_pack4(code[0], code[1], code[2], code[3]);
+                    if constexpr (VEC == 8) wq[h][1] = bi8_pack4(code[4], code[5], code[6], code[7]);
                 }
             }
-            if constexpr (kPairStores) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+                if ((tid % LB) == 0 && (B != 2 * kTC || h == 0)) lds.rs[(h * kTC + cc) / B][p * RPP + lr] = m[h];
+            if constexpr (FULL) {
+                // (16-bit inputs, two halves: a lane's 8 codes of each half are exchanged with its neighbour's so that the
+                // even lane stores 16 consecutive codes of the left half and the odd lane 16 of the right half -- the eight lanes of
+                // a row then write the row's whole 128-byte line in one instruction instead of two halves in two)
                 if (wide_q) {
-                    const bool odd = (tid & 1) != 0;
-                    const bi8_v2u send = odd ? wq[0] : wq[1];              // what the neighbour stores of this lane's codes
-                    bi8_v2u recv;
-                    recv[0] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send[0], 0xB1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
-                    recv[1] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send[1], 0xB1, 0xf, 0xf, false);
-                    const bi8_v4u w = odd ? bi8_v4u{recv[0], recv[1], wq[1][0], wq[1][1]} : bi8_v4u{wq[0][0], wq[0][1], recv[0], recv[1]};
-                    const int64_t col = cbase + (odd ? kTC + cc - VEC : cc);       // 16 consecutive codes from here
-                    if (row < R && col < Cp) {
-                        int8_t *dst = q + row * ldq + col;
-                        if (col + 2 * VEC <= Cp) __builtin_nontemporal_store(w, (bi8_v4u *)dst);
-                        else __builtin_nontemporal_store(bi8_v2u{w[0], w[1]}, (bi8_v2u *)dst);      // (Cp is a multiple of 8: the row ends after the first 8)
+                    if constexpr (VEC == 8 && NH == 2) {
+                        const bool odd = (tid & 1) != 0;
+                        const bi8_v2u send = odd ? wq[0] : wq[NH - 1];        // what the neighbour stores of this lane's codes
+                        const bi8_v2u recv = {bi8_dpp_bits<0xB1>(send[0]), bi8_dpp_bits<0xB1>(send[1])};     // quad_perm [1,0,3,2]
+                        const bi8_v4u w = odd ? bi8_v4u{recv[0], recv[1], wq[NH - 1][0], wq[NH - 1][1]} : bi8_v4u{wq[0][0], wq[0][1], recv[0], recv[1]};
+                        __builtin_nontemporal_store(w, (bi8_v4u *)(q + row * ldq + cbase + (odd ? kTC + cc - VEC : cc)));
+                    } else {
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            int8_t *dst = q + row * ldq + cbase + h * kTC + cc;
+                            if constexpr (VEC == 8) __builtin_nontemporal_store(wq[h], (bi8_v2u *)dst);
+                            else __builtin_nontemporal_store(wq[h][0], (uint32_t *)dst);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+                        int8_t *dst = q + row * ldq + cbase + h * kTC + cc;
+                        if constexpr (VEC == 8) *(bi8_v2u_unaligned *)dst = wq[h];
+                        else *(bi8_u32_unaligned *)dst = wq[h][0];
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int h = 0; h < NH; ++h) {
+                    const int64_t col = cbase + h * kTC + cc;
+                    int8_t *dst = q + row * ldq + col;
+                    if (row < R && col + VEC <= Cp) {
+                        if constexpr (VEC == 8) *(bi8_v2u_unaligned *)dst = wq[h];
+                        else *(bi8_u32_unaligned *)dst = wq[h][0];
+                    } else if (row < R) {
+#pragma unroll
+                        for (int e = 0; e < VEC - 1; ++e)
+                            if (col + e < Cp) dst[e] = (int8_t)((wq[h][e / 4] >> (8 * (e & 3))) & 0xffu);
                     }
                 }
             }
@@ -210,13 +268,14 @@ __device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *_
             // phase 1: this half -> LDS as it is (the previous half's column reads ended before the barrier that
             // precedes its phase 4); then start the next tile's loads of this half
 #pragma unroll
-            for (int p = 0; p < NP; ++p) *(bi8_v4u *)&s_x[(p * RPP + lr) * kXPitch + (tid % LPR) * 16] = raw[h][p];
-            load_half(tile + tile_step, h, raw[h]);
+            for (int p = 0; p < NP; ++p) *(bi8_v4u *)&lds.x[(p * RPP + lr) * L::kXPitch + (tid % LPR) * 16] = raw[h][p];
+            if (next < ntiles) load_half(tr_n, tc_n, h, raw[h]);
             __syncthreads();
             if (h == 0) {
-                for (int i = tid; i < NRB * kTR; i += kThreads) {
+#pragma unroll
+                for (int i = tid; i < L::kNRB * kTR; i += kThreads) {
                     const int b = i / kTR, r = i % kTR;
-                    if (r0 + r < R && cbase + b * B < Cp) scales[(cbase / B + b) * R + r0 + r] = s_rs[b][r];
+                    if (FULL || (r0 + r < R && cbase + b * B < Cp)) scales[(cbase / B + b) * R + r0 + r] = lds.rs[b][r];
                 }
             }
 
@@ -224,42 +283,27 @@ __device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *_
             // columns), then over the block's row groups
             const int cw = tid % (kTC / CPT);
             const int g = tid / (kTC / CPT);
-            float v[CPT][RPT];
-            float m[CPT];
-            bool special = false;
+            uint32_t d[RPT];
 #pragma unroll
-            for (int k = 0; k < CPT; ++k) m[k] = 0.0f;
+            for (int i = 0; i < RPT; ++i) d[i] = *(const uint32_t *)&lds.x[(g * RPT + i) * L::kXPitch + cw * 4];
+            uint32_t bits = bi8_abs_bits<DT>(d[0]);
 #pragma unroll
-            for (int i = 0; i < RPT; ++i) {
-                const uint32_t d = *(const uint32_t *)&s_x[(g * RPT + i) * kXPitch + cw * 4];
-                if constexpr (DT == BI8_F32) {
-                    v[0][i] = bi8_u2f(d);
-                } else if constexpr (DT == BI8_BF16) {
-                    v[0][i] = bi8_u2f(d << 16);
-                    v[1][i] = bi8_u2f(d & 0xffff0000u);
-                } else {
-                    v[0][i] = bi8_from_f16_bits(d & 0xffffu);
-                    v[1][i] = bi8_from_f16_bits(d >> 16);
-                }
-#pragma unroll
-                for (int k = 0; k < CPT; ++k) {
-                    m[k] = __builtin_fmaxf(m[k], __builtin_fabsf(v[k][i]));
-                    special |= (v[k][i] != v[k][i]);
-                }
-            }
+            for (int i = 1; i < RPT; ++i) bits = bi8_larger_bits<DT>(bits, bi8_abs_bits<DT>(d[i]));
             if constexpr (SUM) {
                 // this thread's rows of its columns, top to bottom (rows past R were loaded as zeros)
 #pragma unroll
                 for (int k = 0; k < CPT; ++k) {
-                    float t = v[k][0];
+                    float t = word_elem<DT>(d[0], k);
 #pragma unroll
-                    for (int i = 1; i < RPT; ++i) t += v[k][i];
-                    s_sum[g][cw * CPT + k] = t;
+                    for (int i = 1; i < RPT; ++i) t += word_elem<DT>(d[i], k);
+                    lds.sum[g][cw * CPT + k] = t;
                 }
+                // (the codes unpack the words again: kept from here they would be twice the registers)
+#pragma unroll
+                for (int i = 0; i < RPT; ++i) asm volatile("" : "+v"(d[i]));
             }
             if constexpr (GPW > 1 || SUM) {
-#pragma unroll
-                for (int k = 0; k < CPT; ++k) s_max[g][cw * CPT + k] = m[k];
+                if constexpr (GPW > 1) lds.max[g][cw] = bits;
                 __syncthreads();
                 if constexpr (SUM) {
                     // the tile's row groups in ascending order; read before the barrier that follows phase 3, written
@@ -267,51 +311,71 @@ __device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *_
                     if (g == 0) {
 #pragma unroll
                         for (int k = 0; k < CPT; ++k) {
-                            float t = s_sum[0][cw * CPT + k];
+                            float t = lds.sum[0][cw * CPT + k];
 #pragma unroll
-                            for (int qg = 1; qg < G; ++qg) t += s_sum[qg][cw * CPT + k];
-                            if (c0 + cw * CPT + k < C) colsum_part[tr * C + c0 + cw * CPT + k] = t;
+                            for (int qg = 1; qg < G; ++qg) t += lds.sum[qg][cw * CPT + k];
+                            if (FULL || c0 + cw * CPT + k < C) colsum_part[tr * C + c0 + cw * CPT + k] = t;
                         }
                     }
                 }
-                const int gb = g & ~(GPW - 1);
+                if constexpr (GPW > 1) {
+                    const int gb = g & ~(GPW - 1);
+                    bits = lds.max[gb][cw];
 #pragma unroll
-                for (int qg = 0; qg < GPW; ++qg)
+                    for (int qg = 1; qg < GPW; ++qg) bits = bi8_larger_bits<DT>(bits, lds.max[gb + qg][cw]);
+                }
+            }
+            float mc[CPT];
+            bool slow_c = false;
 #pragma unroll
-                    for (int k = 0; k < CPT; ++k) m[k] = __builtin_fmaxf(m[k], s_max[gb + qg][cw * CPT + k]);
+            for (int k = 0; k < CPT; ++k) mc[k] = word_elem<DT>(bits, k);
+
+            // phase 3: codes of this thread's rows -> byte tile [column][row], 16 bytes per store
+            bi8_v4u w[CPT][RPT / 16];
+#pragma unroll
+            for (int k = 0; k < CPT; ++k) {
+                slow_c |= !bi8_scale_is_fast(mc[k]);
+                const float y = bi8_recip_of_scale(mc[k]);
+#pragma unroll
+                for (int i = 0; i < RPT; i += 4) {
+                    uint32_t code[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) code[e] = bi8_code_fast<NCORR>(word_elem<DT>(d[i + e], k), mc[k], y);
+                    w[k][i / 16][(i % 16) / 4] = bi8_pack4(code[0], code[1], code[2], code[3]);
+                }
+            }
+            if (__builtin_expect(__any(slow_c), 0)) {
+#pragma unroll
+                for (int k = 0; k < CPT; ++k) {
+                    if (bi8_scale_is_fast(mc[k])) continue;
+                    float s = 0.0f;                // of the block's rows, from the tile (the other groups' maxima hold its NaNs)
+#pragma nounroll
+                    for (int r = g * RPT / B * B; r < g * RPT / B * B + B; ++r)
+                        s = __builtin_fmaxf(s, __builtin_fabsf(word_elem<DT>(*(const uint32_t *)&lds.x[r * L::kXPitch + cw * 4], k)));
+                    mc[k] = s;
+#pragma unroll
+                    for (int i = 0; i < RPT; i += 4) {
+                        uint32_t code[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) code[e] = bi8_code_slow(word_elem<DT>(d[i + e], k), s);
+                        w[k][i / 16][(i % 16) / 4] = bi8_pack4(code[0], code[1], code[2], code[3]);
+                    }
+                }
             }
             if ((g & (GPW - 1)) == 0) {
                 const int64_t jb = (r0 + g * RPT) / B;
 #pragma unroll
                 for (int k = 0; k < CPT; ++k)
-                    if (r0 + g * RPT < Rp && c0 + cw * CPT + k < C) scalesT[jb * C + c0 + cw * CPT + k] = m[k];
+                    if (FULL || (r0 + g * RPT < Rp && c0 + cw * CPT + k < C)) scalesT[jb * C + c0 + cw * CPT + k] = mc[k];
             }
-
-            // phase 3: codes of this thread's rows -> byte tile [column][row], 16 bytes per store
 #pragma unroll
-            for (int k = 0; k < CPT; ++k) {
-                uint32_t code[RPT];
-                if (__builtin_expect(special || !bi8_scale_is_ordinary(m[k]), 0)) {
+            for (int k = 0; k < CPT; ++k)
 #pragma unroll
-                    for (int i = 0; i < RPT; ++i) code[i] = bi8_code_slow(v[k][i], m[k]);
-                } else {
-                    const float y = 1.0f / m[k];
-#pragma unroll
-                    for (int i = 0; i < RPT; ++i) code[i] = bi8_code_fast<NCORR>(v[k][i], m[k], y);
-                }
-#pragma unroll
-                for (int i = 0; i < RPT / 16; ++i) {
-                    bi8_v4u w;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        w[e] = bi8_pack4(code[16 * i + 4 * e], code[16 * i + 4 * e + 1], code[16 * i + 4 * e + 2], code[16 * i + 4 * e + 3]);
-                    *(bi8_v4u *)&s_q[(cw * CPT + k) * kQPitch + g * RPT + 16 * i] = w;
-                }
-            }
+                for (int i = 0; i < RPT / 16; ++i) *(bi8_v4u *)&lds.q[(cw * CPT + k) * kQPitch + g * RPT + 16 * i] = w[k][i];
             __syncthreads();
 
-            // phase 4: 16 codes per lane, 8 lanes per output row.  The next writes to s_x come after this barrier, the
-            // next writes to s_q after the next phase-1 barrier.
+            // phase 4: 16 codes per lane, 8 lanes per output row.  The next writes to the tile come after this barrier, the
+            // next writes to the code tile after the next phase-1 barrier.
 #pragma unroll
             for (int p = 0; p < (kTC * kTR / 16) / kThreads; ++p) {
                 const int idx = p * kThreads + tid;
@@ -319,55 +383,64 @@ __device__ __forceinline__ void dual_tiles(const void *__restrict__ x, int8_t *_
                 const int seg = idx % (kTR / 16);
                 const int64_t orow = c0 + oc;
                 const int64_t ocol = r0 + seg * 16;
-                if (orow < C && ocol < Rp) {
-                    const bi8_v4u w = *(const bi8_v4u *)&s_q[oc * kQPitch + seg * 16];
+                if (FULL || (orow < C && ocol < Rp)) {
+                    const bi8_v4u v = *(const bi8_v4u *)&lds.q[oc * kQPitch + seg * 16];
                     int8_t *dst = qT + orow * ldqt + ocol;
-                    if (ocol + 16 <= Rp) {
-                        __builtin_nontemporal_store(w, (bi8_v4u *)dst);
+                    if (FULL || ocol + 16 <= Rp) {
+                        __builtin_nontemporal_store(v, (bi8_v4u *)dst);
                     } else {
-                        for (int e = 0; e < (int)(Rp - ocol); ++e) dst[e] = (int8_t)((w[e >> 2] >> (8 * (e & 3))) & 0xffu);
+                        for (int e = 0; e < (int)(Rp - ocol); ++e) dst[e] = (int8_t)((v[e >> 2] >> (8 * (e & 3))) & 0xffu);
                     }
                 }
             }
         }
+        if (next >= ntiles) break;
+        tile = next;
+        tr = tr_n;
+        tc = tc_n;
     }
 }
 
-#define BI8_DUAL_KERNEL __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DT == BI8_F32 ? 2 : 3)))
+// All of a matrix' tiles: workgroup `first` of `step` takes every step-th of the full ones, then of the others, counted on from there.
 template <int DT, int B, bool ALIGNED, bool SUM, int NH>
-BI8_DUAL_KERNEL void quantize_dual_tile(const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales, int8_t *__restrict__ qT,
-                                        float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx, int64_t ldq, int64_t ldqt,
-                                        int64_t Rp, int64_t Cp, int64_t tiles_c, int64_t ntiles) {
-    dual_tiles<DT, B, ALIGNED, SUM, NH>(x, q, scales, qT, scalesT, colsum_part, R, C, ldx, ldq, ldqt, Rp, Cp, tiles_c, ntiles, blockIdx.x, gridDim.x);
+__device__ __forceinline__ void dual_matrix(const Bi8DualTask &t, float *colsum_part, int first, int step) {
+    __shared__ DualLds<DT, B, SUM, NH> lds;
+    dual_tiles<DT, B, ALIGNED, SUM, NH, true>(lds, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx, t.ldq, t.ldqt, t.Rp, t.Cp, first, step);
+    if (t.Rp % kTR == 0 && t.Cp % (NH * kTC) == 0 && t.Rp == t.R && t.Cp == t.C) return;
+    const int full = (int)(t.R / kTR) * (int)(t.C / (NH * kTC));
+    const int offset = (first - full % step + step) % step;
+    __syncthreads();                               // the last full tile has been read
+    dual_tiles<DT, B, ALIGNED, SUM, NH, false>(lds, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx, t.ldq, t.ldqt, t.Rp, t.Cp, offset, step);
+}
+
+#define BI8_DUAL_KERNEL __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DT == BI8_F32 ? 3 : 4)))
+template <int DT, int B, bool ALIGNED, bool SUM, int NH>
+BI8_DUAL_KERNEL void quantize_dual_tile(const Bi8DualTask task, float *__restrict__ colsum_part) {
+    dual_matrix<DT, B, ALIGNED, SUM, NH>(task, colsum_part, blockIdx.x, gridDim.x);
 }
 
 // Two matrices: the grid's first blocks0 workgroups work on the first, the others on the second (a layer's X and W: one launch, and
 // the smaller of the two does not have the chip to itself half empty).
 struct DualPair {
     Bi8DualTask task[2];
-    int64_t tiles_c[2], ntiles[2];
     unsigned blocks0;
 };
 template <int DT, int B, bool ALIGNED, int NH> BI8_DUAL_KERNEL void quantize_dual_pair(const DualPair pair) {
     const bool second = blockIdx.x >= pair.blocks0;
     const Bi8DualTask &t0 = pair.task[0], &t1 = pair.task[1];
 #define BI8_OF_TASK(f) (second ? t1.f : t0.f)
-    dual_tiles<DT, B, ALIGNED, false, NH>(BI8_OF_TASK(x), BI8_OF_TASK(q), BI8_OF_TASK(scales), BI8_OF_TASK(qT), BI8_OF_TASK(scalesT), nullptr, BI8_OF_TASK(R),
-                                          BI8_OF_TASK(C), BI8_OF_TASK(ldx), BI8_OF_TASK(ldq), BI8_OF_TASK(ldqt), BI8_OF_TASK(Rp), BI8_OF_TASK(Cp),
-                                          second ? pair.tiles_c[1] : pair.tiles_c[0], second ? pair.ntiles[1] : pair.ntiles[0],
-                                          second ? blockIdx.x - pair.blocks0 : blockIdx.x, second ? gridDim.x - pair.blocks0 : pair.blocks0);
+    const Bi8DualTask task{BI8_OF_TASK(x), BI8_OF_TASK(q), BI8_OF_TASK(qT), BI8_OF_TASK(scales), BI8_OF_TASK(scalesT), BI8_OF_TASK(R), BI8_OF_TASK(C),
+                           BI8_OF_TASK(ldx), BI8_OF_TASK(ldq), BI8_OF_TASK(ldqt), BI8_OF_TASK(Rp), BI8_OF_TASK(Cp)};
 #undef BI8_OF_TASK
+    dual_matrix<DT, B, ALIGNED, false, NH>(task, nullptr, (int)(second ? blockIdx.x - pair.blocks0 : blockIdx.x), (int)(second ? gridDim.x - pair.blocks0 : pair.blocks0));
 }
 
 template <int DT, int B, bool ALIGNED, int NH> int launch_one(const Bi8DualTask &t, float *colsum_part, int64_t resident, hipStream_t st) {
-    const int64_t tiles_c = (t.Cp + NH * kTC - 1) / (NH * kTC), ntiles = tiles_c * ((t.Rp + kTR - 1) / kTR);
+    const int64_t ntiles = ((t.Cp + NH * kTC - 1) / (NH * kTC)) * ((t.Rp + kTR - 1) / kTR);
+    if (ntiles + resident > 0x7fffffffLL) return BI8_ERR_TOO_LARGE;
     const dim3 grid((unsigned)(ntiles < resident ? ntiles : resident));
-    if (colsum_part)
-        hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, true, NH>), grid, dim3(kThreads), 0, st, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx,
-                           t.ldq, t.ldqt, t.Rp, t.Cp, tiles_c, ntiles);
-    else
-        hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH>), grid, dim3(kThreads), 0, st, t.x, t.q, t.scales, t.qT, t.scalesT, colsum_part, t.R, t.C, t.ldx,
-                           t.ldq, t.ldqt, t.Rp, t.Cp, tiles_c, ntiles);
+    if (colsum_part) hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, true, NH>), grid, dim3(kThreads), 0, st, t, colsum_part);
+    else hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH>), grid, dim3(kThreads), 0, st, t, colsum_part);
     return bi8_launch_rc();
 }
 
@@ -378,12 +451,11 @@ template <int DT, int B, bool ALIGNED, int NH> int launch_one(const Bi8DualTask 
 // 30.3; at fp32 (768 workgroups) 1710 + 665 (4 -> 4) 67.7 -> 67.7, 672 + 1120 (3 -> 3) 50.1 -> 49.6; 1836 + 4104 (7 -> 6) 92.1 -> 84.4.
 constexpr int64_t kPairRounds = 4;
 template <int DT, int B, bool ALIGNED, int NH> int launch_pair(const Bi8DualTask *task, int64_t resident, hipStream_t st) {
-    DualPair pair{{task[0], task[1]}, {}, {}, 0};
-    for (int i = 0; i < 2; ++i) {
-        pair.tiles_c[i] = (task[i].Cp + NH * kTC - 1) / (NH * kTC);
-        pair.ntiles[i] = pair.tiles_c[i] * ((task[i].Rp + kTR - 1) / kTR);
-    }
-    const int64_t *tiles = pair.ntiles, all = tiles[0] + tiles[1], grid = all < resident ? all : resident;
+    DualPair pair{{task[0], task[1]}, 0};
+    int64_t tiles[2];
+    for (int i = 0; i < 2; ++i) tiles[i] = ((task[i].Cp + NH * kTC - 1) / (NH * kTC)) * ((task[i].Rp + kTR - 1) / kTR);
+    const int64_t all = tiles[0] + tiles[1], grid = all < resident ? all : resident;
+    if (all + resident > 0x7fffffffLL) return BI8_ERR_TOO_LARGE;
     int64_t first = all <= resident ? tiles[0] : (grid * tiles[0] + all / 2) / all;
     first = first < 1 ? 1 : first > grid - 1 ? grid - 1 : first;
     const int64_t apart = (tiles[0] + resident - 1) / resident + (tiles[1] + resident - 1) / resident;
@@ -395,8 +467,8 @@ template <int DT, int B, bool ALIGNED, int NH> int launch_pair(const Bi8DualTask
 }
 
 template <int DT, int B, bool ALIGNED> int launch_dual(const Bi8DualTask *task, int count, float *colsum_part, hipStream_t st) {
-    // workgroups per CU: four with 16-bit inputs (29 KiB of LDS, under 128 registers: 62.7 us against 65.9 with three at
-    // bf16 [8192,8192]), three with fp32 (42 KiB)
+    // workgroups per CU: four with 16-bit inputs (30 KiB of LDS, at most 128 registers), three with fp32 (43 KiB, 168).  us with three
+    // / four: bf16 [8192,4096] 29.5 / 28.6, [8192,3072] 22.7 / 22.7, fp32 [4096,4096] 23.5 / 27.9
     const int64_t resident = (DT == BI8_F32 ? 3 : 4) * 256;
     // inputs of fewer full tiles than the chip holds workgroups: half tiles, twice as many workgroups
     int64_t full = 0;
@@ -418,6 +490,25 @@ template <int DT, bool ALIGNED> int dispatch(const Bi8DualTask *task, int count,
     default: return launch_dual<DT, 128, ALIGNED>(task, count, colsum_part, st);
     }
 }
+
+}  // namespace
+
+// This file is compiled once per input type with -DBI8_DUAL_DT=d, which gives the one function below with that type's kernels, and once
+// without for everything else: one translation unit with all of them takes two minutes.
+#define BI8_DUAL_RUN_PASTE(d) bi8_dual_run_##d
+#define BI8_DUAL_RUN_NAME(d) BI8_DUAL_RUN_PASTE(d)
+#define BI8_DUAL_RUN(d) int BI8_DUAL_RUN_NAME(d)(const Bi8DualTask *task, int count, bool aligned, float *colsum_part, int block, hipStream_t st)
+#ifdef BI8_DUAL_DT
+__attribute__((visibility("hidden"))) BI8_DUAL_RUN(BI8_DUAL_DT) {
+    return aligned ? dispatch<BI8_DUAL_DT, true>(task, count, colsum_part, block, st) : dispatch<BI8_DUAL_DT, false>(task, count, colsum_part, block, st);
+}
+#else
+BI8_DUAL_RUN(0);
+BI8_DUAL_RUN(1);
+BI8_DUAL_RUN(2);
+static_assert(BI8_F32 == 0 && BI8_BF16 == 1 && BI8_F16 == 2, "the names of the functions");
+
+namespace {
 
 // Column sums without the quantizer (the shapes that the one-pass kernel does not take): the same grouping of the
 // rows -- groups of kTR / G rows top to bottom, the groups of a 128-row tile in ascending order -- so that the sums
@@ -485,13 +576,13 @@ extern "C" int bi8x_quantize_dual(const Bi8DualTask *task, int count, int x_dtyp
         const Bi8DualTask &t = task[i];
         if (!one_pass(t, x_dtype, block)) return BI8_ERR_UNSUPPORTED;
         if (t.R < 1 || t.C < 1 || t.ldx < t.C || t.Cp < t.C || t.Rp < t.R || t.ldq < t.Cp || t.ldqt < t.Rp) return BI8_ERR_BAD_SHAPE;
-        aligned = aligned && t.C % vec == 0 && t.ldx % vec == 0 && bi8_aligned(t.x, 16) && t.ldq % 8 == 0 && bi8_aligned(t.q, 8);
+        aligned = aligned && t.C % vec == 0 && t.ldx % vec == 0 && bi8_aligned(t.x, 16);
     }
     hipStream_t st = (hipStream_t)stream;
     switch (x_dtype) {
-    case BI8_F32: return aligned ? dispatch<BI8_F32, true>(task, count, colsum_part, block, st) : dispatch<BI8_F32, false>(task, count, colsum_part, block, st);
-    case BI8_BF16: return aligned ? dispatch<BI8_BF16, true>(task, count, colsum_part, block, st) : dispatch<BI8_BF16, false>(task, count, colsum_part, block, st);
-    default: return aligned ? dispatch<BI8_F16, true>(task, count, colsum_part, block, st) : dispatch<BI8_F16, false>(task, count, colsum_part, block, st);
+    case BI8_F32: return BI8_DUAL_RUN_NAME(0)(task, count, aligned, colsum_part, block, st);
+    case BI8_BF16: return BI8_DUAL_RUN_NAME(1)(task, count, aligned, colsum_part, block, st);
+    default: return BI8_DUAL_RUN_NAME(2)(task, count, aligned, colsum_part, block, st);
     }
 }
 
@@ -550,3 +641,4 @@ extern "C" int bi8_quantize_dual_colsum(const void *x, int x_dtype, int8_t *q, f
     const int rc = quantize_dual(x, x_dtype, q, scales, qT, scalesT, (float *)workspace, R, C, ldx, ldq, ldqt, block, stream);
     return rc != BI8_OK ? rc : bi8x_colsum_finish((const float *)workspace, colsum, x_dtype, R, C, stream);
 }
+#endif  // BI8_DUAL_DT
