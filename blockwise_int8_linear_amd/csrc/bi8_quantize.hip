@@ -206,16 +206,21 @@ int launch_rows(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, i
 // two up to 72, four beyond, where more loads in flight per wave pay.  us with 1 / 2 / 4 (before: four, 1 KiB loads that waited for
 // one another, and the IEEE path inside each row): bf16, block 128 16 x 4096 1.8 / 2.1 / 2.5 (2.8), 512 x 4096 2.6 / 2.7 / 2.9 (3.2), 2048 x
 // 4096 7.2 / 6.6 / 6.9 (7.4), 3000 x 4096 9.4 / 9.0 / 8.8 (9.3), 4096 x 4096 11.9 / 11.5 / 10.8 (11.5), 8192 x 8192 37.2 / 34.8 / 35.3 (35.4);
-// fp16 100 x 11008 2.3 / 2.7 / 3.0 (3.9), 300 x 16384 4.9 / 4.8 / 5.3 (5.4); fp32, block 32 1000 x 5004 7.6 / 7.5 / 7.0 (7.2).  Rows off 16-byte
-// boundaries run with one whatever the size: bf16 1000 x 5003 5.6 / 5.6 / 7.2 (9.1), 8192 x 50257 267 / 293 / 287 (283).
+// fp16 100 x 11008 2.3 / 2.7 / 3.0 (3.9), 300 x 16384 4.9 / 4.8 / 5.3 (5.4); fp32, block 32 1000 x 5004 7.6 / 7.5 / 7.0 (7.2).
+// Rows off 16-byte boundaries run with one whatever the size where a KiB of row holds at most eight blocks: bf16, block 128 1000 x 5003
+// 5.6 / 5.6 / 7.2 (9.1), 8192 x 50257 250 / 279 / 280 (278), block 64 267 / 290 / 287 (282); fp32, block 32 8192 x 50257 472 / 514 / 516 (505).
+// With one row per wave every scale is a 4-byte store by itself; smaller blocks, sixteen stores and more per KiB, go by the size: bf16,
+// block 32 8192 x 50257 320 / 317 / 297 (293), 8192 x 5001 32.4 / 30.2 / 30.5 (32.0); block 8 672 / 473 / 352 (343), 53.4 / 40.6 / 34.3 (35.9); fp32,
+// block 16 8192 x 50257 571 / 570 / 531 (530); with two at most where a row is short: block 32, fp16 20000 x 1001 18.7 / 20.4 / 22.4 (20.3), 65536 x 251
+// 28.7 / 25.5 / 29.0 (28.3).
 constexpr int64_t kOneRowWaves = 24 * 256, kTwoRowWaves = 72 * 256;
 template <int DT, int L, bool ALIGNED>
 int launch_vec(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, int64_t Kp, int64_t ldx, int64_t ldq, hipStream_t st) {
     constexpr int TE = BI8_WAVE * Bi8Vec<DT>::kElems;
-    const int64_t waves = M * ((Kp + TE - 1) / TE);
-    if constexpr (ALIGNED) {
-        if (waves > kTwoRowWaves) return launch_rows<DT, L, true, 4>(x, q, scales, M, K, Kp, ldx, ldq, st);
-        if (waves > kOneRowWaves) return launch_rows<DT, L, true, 2>(x, q, scales, M, K, Kp, ldx, ldq, st);
+    const int64_t runs = (Kp + TE - 1) / TE, waves = M * runs;
+    if constexpr (ALIGNED || L <= 4) {
+        if (waves > kTwoRowWaves && (ALIGNED || runs > 4)) return launch_rows<DT, L, ALIGNED, 4>(x, q, scales, M, K, Kp, ldx, ldq, st);
+        if (waves > kOneRowWaves) return launch_rows<DT, L, ALIGNED, 2>(x, q, scales, M, K, Kp, ldx, ldq, st);
     }
     return launch_rows<DT, L, ALIGNED, 1>(x, q, scales, M, K, Kp, ldx, ldq, st);
 }
