@@ -1,8 +1,9 @@
 // Block dequantize (bi8_dequantize_rowwise): out = (scale * float(code)) * fp32(1/127), cast on store.
 // Replaces _dequantize_block_rowwise, triton_functions.py:468-490.  HBM-bound: one lane = one 128-bit store
 // of outputs (8 bf16/f16 or 4 fp32) per step, so every wave store covers 1 KiB of contiguous output.  Same
-// tiling as the quantizer: a workgroup owns 8 rows x 2 KiB of output row (small calls: 4 x 1 KiB, short rows 16 x 1 KiB) and, with more
-// than a row per wave, first pulls its scales in through LDS, so the block-major / row-minor scale array is read as runs of 8 or 16 rows.
+// tiling as the quantizer: a workgroup owns 8 rows x 2 KiB of output row (small calls: 4 x 1 KiB, short rows 8 or 16 x 1 KiB, ragged ones of
+// middling calls 4 x 4 KiB) and, with more than a row per wave, first pulls its scales in through LDS, so the block-major / row-minor
+// scale array is read as runs of 8 or 16 rows.
 #include "bi8_common.h"
 
 namespace {
@@ -106,9 +107,13 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_vec(const int8_t *__
     // one row per wave: its scales straight from memory; otherwise through LDS, read as runs of the workgroup's rows
     constexpr int kMaxBlocks = R == 1 ? 1 : TE / 8;                       // block size >= 8 on this path
     __shared__ float s_tile[kMaxBlocks][kRows + 1];
-    float s_lane = 0.0f;
+    float s_lane[NC];
     if constexpr (R == 1) {
-        if (lane * VEC < left) s_lane = scales[(jb0 + ((lane * VEC) >> log2b)) * M + row0];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int incol = (c * BI8_WAVE + lane) * VEC;
+            s_lane[c] = incol < left ? scales[(jb0 + (incol >> log2b)) * M + row0] : 0.0f;
+        }
     } else {
         const int nb = (TE >> log2b) > 0 ? (TE >> log2b) : 1;             // blocks per tile row
         for (int t = tid; t < nb * kRows; t += kThreads) {
@@ -128,7 +133,7 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_vec(const int8_t *__
         for (int c = 0; c < NC; ++c) {
             const int incol = (c * BI8_WAVE + lane) * VEC, mine = left - incol;
             if (mine <= 0) continue;
-            const float s = R == 1 ? s_lane : s_tile[R == 1 ? 0 : incol >> log2b][wave * R + i];
+            const float s = R == 1 ? s_lane[c] : s_tile[R == 1 ? 0 : incol >> log2b][wave * R + i];
             float v[VEC];
 #pragma unroll
             for (int e = 0; e < VEC / 4; ++e) {
@@ -183,17 +188,34 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_generic(const int8_t
     }
 }
 
-// One row and one chunk per wave where that is few waves (a call of few rows is latency; rows off 16-byte boundaries: up to more of
-// them), else two rows of two chunks, or four rows where a row is one chunk.  us with one / two rows (before: two, loads that waited for
-// one another): bf16, block 128 16 x 4096 1.7 / 2.4 (2.7), 512 x 4096 2.6 / 3.1 (3.2), 2048 x 4096 6.3 / 5.2 (5.1), 8192 x 8192 37.3 / 32.6
-// (33.6); fp16 100 x 11008 2.1 / 2.8 (2.9), 300 x 16384 4.3 / 3.9 (4.1); odd rows fp32 1000 x 5003 6.4 / 6.8 (6.9), bf16 8192 x 5001 34.5 / 31.0
-// (31.1).
-constexpr int64_t kOneRowWaves = 24 * 256, kOneRowWavesRagged = 96 * 256;
+// One row and one chunk per wave where that is few waves (a call of few rows is latency), else two rows of two chunks.  us with one / two
+// rows (before: two, loads that waited for one another), codes in the caches: bf16, block 128 16 x 4096 1.7 / 2.4 (2.7), 512 x 4096 2.6 /
+// 3.1 (3.2), 2048 x 4096 6.3 / 5.2 (5.1), 8192 x 8192 37.3 / 32.6 (33.6); fp16 100 x 11008 2.1 / 2.8 (2.9), 300 x 16384 4.3 / 3.9 (4.1).
+// Rows of one chunk: two or four of them.  Codes from memory, block 32, one / two / four: bf16 12000 x 256 4.8 / 3.6 / 3.8 (3.6), 24000 x 256 7.4 /
+// 6.0 / 5.4 (6.0), 65536 x 256 17.4 / 13.6 / 12.7 (13.6), 24000 x 512 9.9 / 9.0 / 7.6 (9.0), 36000 x 512 13.9 / 12.6 / 13.0 (12.6); fp32 12000 x 256 4.9 / 3.8 /
+// 3.8 (4.0), 24000 x 256 8.9 / 7.2 / 6.0 (7.2), 65536 x 256 21.0 / 16.5 / 17.4 (16.6).  Off 16-byte boundaries one or four: bf16 12000 x 251 6.2 for one, 7.2
+// for four (6.2), 65536 x 251 31.2 / 25.6 (26.5), fp32 33.0 / 28.6 (28.0).
+// Rows off 16-byte boundaries: one chunk per wave in larger calls too (fp32 larger than 16-bit ones), then, where a row has more than
+// two, one row of four chunks (a wave's run cuts lines at its two ends only).  Codes from memory / quantizer and this with all in the caches,
+// 1 x 1, 1 x 4, 2 x 2 (before): block 32 fp32 700 x 5003 8.0 / 10.9, 7.2 / 11.5, 8.0 / 11.6 (8.0 / 11.7), 1000 x 5003 10.3 / 13.5, 9.0 / 13.9, 9.6 / 13.9 (9.8 /
+// 14.1), 8192 x 5001 50.9 / 94.7, 46.3 / 94.7, 47.7 / 94.4 (50.0 / 94.7); bf16 1000 x 5003 8.0 / 11.6, 7.3 / 11.6, 8.6 / 12.7 (8.8 / 12.8), 2048 x 5001 11.8 /
+// 16.9, 10.2 / 17.0, 11.0 / 16.9 (10.6 / 16.9), 3000 x 5001 15.7 / 22.2, 15.1 / 22.0, 14.8 / 21.1 (14.7 / 21.4).
+constexpr int64_t kOneRunWaves = 24 * 256, kOneShortRowWavesRagged = 96 * 256;
+template <int DT> constexpr int64_t kOneRunWavesRagged = (DT == BI8_F32 ? 88 : 56) * 256, kOneRowWavesRagged = (DT == BI8_F32 ? 144 : 112) * 256;
+constexpr int64_t kTwoShortRowsWaves = 64 * 256, kFourLongerRowsWaves = 128 * 256;
 template <int DT, bool ALIGNED>
 int launch_vec(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block, hipStream_t st) {
     constexpr int kChunk = BI8_WAVE * Out<DT>::kElems;
-    if (M * ((K + kChunk - 1) / kChunk) <= (ALIGNED ? kOneRowWaves : kOneRowWavesRagged)) return launch_rows<DT, ALIGNED, 1, 1>(q, scales, out, M, K, ldq, ldo, block, st);
-    if (K <= kChunk) return launch_rows<DT, ALIGNED, 4, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+    const int64_t waves = M * ((K + kChunk - 1) / kChunk);
+    if (waves <= (ALIGNED ? kOneRunWaves : K <= kChunk ? kOneShortRowWavesRagged : kOneRunWavesRagged<DT>))
+        return launch_rows<DT, ALIGNED, 1, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+    if (K <= kChunk) {
+        if constexpr (ALIGNED)
+            if (waves <= kTwoShortRowsWaves || (2 * K > kChunk && waves > kFourLongerRowsWaves)) return launch_rows<DT, ALIGNED, 2, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+        return launch_rows<DT, ALIGNED, 4, 1>(q, scales, out, M, K, ldq, ldo, block, st);
+    }
+    if constexpr (!ALIGNED)
+        if (K > 2 * kChunk && waves <= kOneRowWavesRagged<DT>) return launch_rows<DT, ALIGNED, 1, 4>(q, scales, out, M, K, ldq, ldo, block, st);
     return launch_rows<DT, ALIGNED, 2, 2>(q, scales, out, M, K, ldq, ldo, block, st);
 }
 
