@@ -201,7 +201,8 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_generic(const int8_t
 // 14.1), 8192 x 5001 50.9 / 94.7, 46.3 / 94.7, 47.7 / 94.4 (50.0 / 94.7); bf16 1000 x 5003 8.0 / 11.6, 7.3 / 11.6, 8.6 / 12.7 (8.8 / 12.8), 2048 x 5001 11.8 /
 // 16.9, 10.2 / 17.0, 11.0 / 16.9 (10.6 / 16.9), 3000 x 5001 15.7 / 22.2, 15.1 / 22.0, 14.8 / 21.1 (14.7 / 21.4).
 constexpr int64_t kOneRunWaves = 24 * 256, kOneShortRowWavesRagged = 96 * 256;
-template <int DT> constexpr int64_t kOneRunWavesRagged = (DT == BI8_F32 ? 88 : 56) * 256, kOneRowWavesRagged = (DT == BI8_F32 ? 144 : 112) * 256;
+template <int DT> constexpr int64_t kOneRunWavesRagged = (DT == BI8_F32 ? 88 : 56) * 256;
+template <int DT> constexpr int64_t kOneRowWavesRagged = (DT == BI8_F32 ? 144 : 112) * 256;
 constexpr int64_t kTwoShortRowsWaves = 64 * 256, kFourLongerRowsWaves = 128 * 256;
 template <int DT, bool ALIGNED>
 int launch_vec(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block, hipStream_t st) {
