@@ -12,27 +12,23 @@
 namespace {
 
 constexpr int kThreads = 256;
-// Codes of more than this (the eight 4 MiB L2s together) leave with ordinary stores, others non-temporal.  Marked non-temporal, a large
-// tensor's codes come back slower to the kernel that reads them next.  us, non-temporal -> ordinary, quantize + dequantize: bf16
-// [8192,8192] 68.2 -> 65.1 (5.2 TB/s of the 338 MB that input, codes and output take once; 69.5 -> 69.2 on another machine), fp32
-// [8192,8192] 109 -> 102, bf16 [8320,4096] 37.9 -> 36.3, [8192,12288] 102.4 -> 96.1; quantize + GEMM: 8192 x 11008 -> 1024 158 -> 148,
-// fp32 4096 x 12288 -> 4096 271 -> 252, 8192 x 4224 -> 2048 95.2 -> 95.4.  The quantizer by itself pays for a part of that: bf16
-// [8192,8192] 31.9 -> 34.4, [8320,4096] 17.1 -> 19.5, fp32 [8192,8192] 53.7 -> 52.3.  Below, they gain nothing: 2048 x 4096 -> 11008 (8 MiB)
-// 116.8 -> 117.3.
-constexpr int64_t kKeepCodes = 32 << 20;
+// Codes leave with ordinary stores.  Marked non-temporal the quantizer by itself is 3-8 % faster, but its codes come back slower to the
+// kernel that reads them next.  us, ordinary / non-temporal, the quantizer and quantize + dequantize: bf16, block 128 512 x 4096 3.2 / 2.9, 5.7 /
+// 5.6, 3000 x 4096 8.9 / 8.4, 15.7 / 15.8, 8192 x 4096 18.9 / 18.2, 34.9 / 36.6; fp32 1400 x 4096 7.3 / 7.1, 12.7 / 13.1, 8192 x 4096 27.0 / 26.6, 51.8 /
+// 55.9; quantize + GEMM bf16 8192 x 11008 -> 1024 148 / 158, fp32 4096 x 12288 -> 4096 252 / 271, 8192 x 4224 -> 2048 95.4 / 95.2.
 
 // One wave = RPW rows x 1 KiB, one workgroup = four of them, one below the other.
 // ALIGNED: rows of x on 16-byte boundaries, K a multiple of the elements per 16 bytes, rows of q aligned to their
 // 4- or 8-byte stores.  Otherwise (odd row length or leading dimension, e.g. the GPT-2 vocabulary 50257) whole chunks
 // move with unaligned 16-byte loads and 4- or 8-byte stores, the last, partial chunk of a row element by element.
-// keep: the codes' stores of aligned rows are not marked non-temporal (see kKeepCodes).
 // Kp: columns written, K or more: zero codes and zero scales past the row's end (the padding that a GEMM contracted over K wants).
-// A row past the end reads the last one and is not stored: the rows' loads do not branch, nor does their arithmetic, so that the rows' chains of dependent instructions run side by side: a block that needs the IEEE division (a
-// subnormal, huge or infinite scale, a NaN) is done over in one place behind them.
+// A row past the end reads the last one and is not stored: the rows' loads do not branch, nor does their arithmetic, so that the rows'
+// chains of dependent instructions run side by side: a block that needs the IEEE division (a subnormal, huge or infinite scale, a NaN)
+// is done over in one place behind them.
 template <int DT, int L, bool ALIGNED, int RPW>
 __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const void *__restrict__ x, int8_t *__restrict__ q,
                                                               float *__restrict__ scales, int64_t M, int64_t K, int64_t Kp,
-                                                              int64_t ldx, int64_t ldq, int64_t nblk, bool keep) {
+                                                              int64_t ldx, int64_t ldq, int64_t nblk) {
     constexpr int VEC = Bi8Vec<DT>::kElems;
     constexpr int B = L * VEC;                       // block size in elements
     constexpr int TE = BI8_WAVE * VEC;               // elements of one row covered by a tile
@@ -121,20 +117,12 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const void *__rest
         int8_t *dst = q + (row0 + i) * ldq + col0 + lane * VEC;
         if (room >= VEC) {
             if constexpr (VEC == 4) {
-                if constexpr (ALIGNED) {
-                    if (keep) *(uint32_t *)dst = w[i][0];
-                    else __builtin_nontemporal_store(w[i][0], (uint32_t *)dst);
-                } else {
-                    *(bi8_u32_unaligned *)dst = w[i][0];
-                }
+                if constexpr (ALIGNED) *(uint32_t *)dst = w[i][0];
+                else *(bi8_u32_unaligned *)dst = w[i][0];
             } else {
                 const bi8_v2u c = {w[i][0], w[i][1]};
-                if constexpr (ALIGNED) {
-                    if (keep) *(bi8_v2u *)dst = c;
-                    else __builtin_nontemporal_store(c, (bi8_v2u *)dst);
-                } else {
-                    *(bi8_v2u_unaligned *)dst = c;
-                }
+                if constexpr (ALIGNED) *(bi8_v2u *)dst = c;
+                else *(bi8_v2u_unaligned *)dst = c;
             }
         } else if constexpr (!ALIGNED) {
 #pragma unroll
@@ -199,7 +187,7 @@ int launch_rows(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, i
     if (tiles_k * gy * gz > 0x7fffffffLL || gz > 65535) return BI8_ERR_TOO_LARGE;
     const int64_t nblk = (Kp + B - 1) / B;
     hipLaunchKernelGGL((quantize_rows_vec<DT, L, ALIGNED, RPW>), dim3((unsigned)tiles_k, (unsigned)gy, (unsigned)gz), dim3(kThreads), 0, st, x, q, scales, M, K, Kp,
-                       ldx, ldq, nblk, M * Kp > kKeepCodes);
+                       ldx, ldq, nblk);
     return bi8_launch_rc();
 }
 // Rows per wave: one where that leaves every CU at most 24 waves (a call of few rows is latency, and a wave's rows follow one another),

@@ -1,4 +1,4 @@
-"""quantize_rowwise on both sides of the size from which its codes leave with ordinary stores: the same codes and scales as row by row."""
+"""quantize_rowwise on codes as large as the L2s together and larger: the same codes and scales as row by row."""
 import pytest
 import torch
 
