@@ -69,14 +69,19 @@ template <int DT, int B, bool SUM, int NH> struct DualLds {
     float rs[kNRB][kTR];
 };
 
-// ALIGNED: rows of x start on 16-byte boundaries and C is a multiple of the elements per 16 bytes.  Otherwise whole 16-byte chunks move
-// with unaligned accesses and the last, partial chunk of a row element by element.
+// ALIGNED: rows of x start on 16-byte boundaries and C is a multiple of the elements per 16 bytes.  Otherwise 16-byte chunks move
+// with unaligned accesses, the last, partial chunk of a row as the row's last 16 bytes.
 // NH: halves per tile.  2 is the tile described above; 1 (a 128 x 64 tile, blocks of at most 64) doubles the number of
 // workgroups for inputs too small to occupy the chip with full tiles.
 // Rp, Cp: rows and columns written, the matrix' own or more: zeros past its end.
 // FULL: the tiles that lie inside the matrix, otherwise those at its right and lower end.  Every load and store of a full tile is
 // unconditional, so that the wait for the next tile's loads is for those, and not for the stores issued behind them: with a branch
-// around either the compiler cannot count them and waits for everything, a tile's codes on their way to memory included.
+// around either the compiler cannot count them and waits for everything, a tile's codes on their way to memory included.  Tiles at the
+// ends: a call of few rows is little else, and what bounds it is the chain load, rows, columns, store and the length of the code, run
+// once; so no loads element by element, none of rows and passes that lie past the end, loops where single codes are stored.  us,
+// with all these -> this (before the two kinds of tiles): block 64 fp32 100 x 11008 7.7 -> 6.0 (6.6), 500 x 4096 8.2 -> 6.6 (7.0), 11008 x 100 9.1 ->
+// 6.7 (7.6), bf16 300 x 5003 7.2 -> 6.2 (9.0), 300 x 32768 14.4 -> 14.0 (12.8); block 128 bf16 1000 x 5003 11.3 -> 9.8 (15.3), fp32 12.7 -> 10.7 (16.5)
+// at 4097 x 1023.
 // The workgroup's tiles: first_tile, first_tile + tile_step, ...
 template <int DT, int B, bool ALIGNED, bool SUM, int NH, bool FULL>
 __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales,
@@ -117,32 +122,44 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
             tc = (t - right) % full_c;
         }
     };
+    constexpr bool kShift = !FULL && !ALIGNED;
     const char *x_lane = (const char *)x + ((int64_t)lr * ldx + cc) * ES;
     auto load_half = [&](int tr, int tc, int h, bi8_v4u *raw) {
         const int64_t r0 = (int64_t)tr * kTR, c0 = (int64_t)tc * TC + h * kTC;
+        // a chunk that ends past a row's end is the row's last 16 bytes (see settle)
+        const int64_t ahead = kShift && C >= VEC && c0 + cc > C - VEC ? c0 + cc - (C - VEC) : 0;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            const char *src = x_lane + ((r0 + p * RPP) * ldx + c0) * ES;
+            const char *src = x_lane + ((r0 + p * RPP) * ldx + c0 - ahead) * ES;
             if constexpr (FULL) {
                 if constexpr (ALIGNED) raw[p] = __builtin_nontemporal_load((const bi8_v4u *)src);
                 else raw[p] = *(const bi8_v4u_unaligned *)src;
             } else {
                 raw[p] = bi8_v4u{0u, 0u, 0u, 0u};
-                if (r0 + p * RPP + lr < R && c0 + cc < C) {
-                    if (c0 + cc + VEC <= C) {
-                        raw[p] = *(const bi8_v4u_unaligned *)src;
-                    } else {                       // the row ends inside this chunk
+                if (r0 + p * RPP + lr >= R || c0 + cc >= C) continue;
+                if constexpr (ALIGNED) {
+                    raw[p] = *(const bi8_v4u *)src;
+                } else if (C >= VEC) {
+                    raw[p] = *(const bi8_v4u_unaligned *)src;
+                } else {                           // a row shorter than a chunk
 #pragma unroll
-                        for (int e = 0; e < VEC; ++e) {
-                            if (c0 + cc + e < C) {
-                                if constexpr (DT == BI8_F32) raw[p][e] = ((const uint32_t *)src)[e];
-                                else raw[p][e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
-                            }
+                    for (int e = 0; e < VEC - 1; ++e) {
+                        if (e < C) {
+                            if constexpr (DT == BI8_F32) raw[p][e] = ((const uint32_t *)src)[e];
+                            else raw[p][e >> 1] |= (uint32_t)((const uint16_t *)src)[e] << (16 * (e & 1));
                         }
                     }
                 }
             }
         }
+    };
+    // ... of which the last `pieces` times 16 bits come to the front
+    auto settle = [&](bi8_v4u v, int pieces) {
+        if (pieces & 4) v = bi8_v4u{v[2], v[3], 0u, 0u};
+        if (pieces & 2) v = bi8_v4u{v[1], v[2], v[3], 0u};
+        if constexpr (ES == 2)
+            if (pieces & 1) v = bi8_v4u{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+        return v;
     };
 
     if (first_tile >= ntiles) return;
@@ -156,11 +173,26 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
         const int next = tile + tile_step;
         int tr_n = 0, tc_n = 0;
         if (next < ntiles) coords(next, tr_n, tc_n);
+        const bool all_columns = FULL || cbase + TC <= Cp, all_rows = FULL || r0 + kTR <= Rp;      // ... of the tile are written
+        int ahead[NH];                             // how far behind its chunk's first element a lane's load begins, in 16-bit pieces
+        if constexpr (kShift) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                const int64_t n = cbase + h * kTC + cc - (C - VEC);
+                ahead[h] = n > 0 && n < VEC && C >= VEC ? (int)n * (ES / 2) : 0;
+            }
+        }
 
         // ---- along the rows, from the registers ----------------------------------------------------------------
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
             const int64_t row = r0 + p * RPP + lr;
+            if (!FULL && r0 + p * RPP >= R) break; // (nothing of these rows is stored)
+            if constexpr (kShift) {
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+                    if (__any(ahead[h] != 0)) raw[h][p] = settle(raw[h][p], ahead[h]);
+            }
             uint32_t bits[NH];
             float m[NH];
             bi8_v2u wq[NH];                        // (fp32: four codes, the first word)
@@ -217,18 +249,20 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
 #pragma unroll
             for (int h = 0; h < NH; ++h)
                 if ((tid % LB) == 0 && (B != 2 * kTC || h == 0)) lds.rs[(h * kTC + cc) / B][p * RPP + lr] = m[h];
-            if constexpr (FULL) {
+            if (all_columns) {
                 // (16-bit inputs, two halves: a lane's 8 codes of each half are exchanged with its neighbour's so that the
                 // even lane stores 16 consecutive codes of the left half and the odd lane 16 of the right half -- the eight lanes of
-                // a row then write the row's whole 128-byte line in one instruction instead of two halves in two)
-                if (wide_q) {
-                    if constexpr (VEC == 8 && NH == 2) {
+                // a row then write the row's whole 128-byte line in one instruction instead of two halves in two; not in the tiles at
+                // the matrix' ends, where it is the registers that spill)
+                constexpr bool kPairs = VEC == 8 && NH == 2;
+                if (wide_q && (FULL || !kPairs)) {
+                    if constexpr (kPairs) {
                         const bool odd = (tid & 1) != 0;
                         const bi8_v2u send = odd ? wq[0] : wq[NH - 1];        // what the neighbour stores of this lane's codes
                         const bi8_v2u recv = {bi8_dpp_bits<0xB1>(send[0]), bi8_dpp_bits<0xB1>(send[1])};     // quad_perm [1,0,3,2]
                         const bi8_v4u w = odd ? bi8_v4u{recv[0], recv[1], wq[NH - 1][0], wq[NH - 1][1]} : bi8_v4u{wq[0][0], wq[0][1], recv[0], recv[1]};
                         __builtin_nontemporal_store(w, (bi8_v4u *)(q + row * ldq + cbase + (odd ? kTC + cc - VEC : cc)));
-                    } else {
+                    } else if (FULL || row < R) {
 #pragma unroll
                         for (int h = 0; h < NH; ++h) {
                             int8_t *dst = q + row * ldq + cbase + h * kTC + cc;
@@ -236,7 +270,7 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
                             else __builtin_nontemporal_store(wq[h][0], (uint32_t *)dst);
                         }
                     }
-                } else {
+                } else if (FULL || row < R) {
 #pragma unroll
                     for (int h = 0; h < NH; ++h) {
                         int8_t *dst = q + row * ldq + cbase + h * kTC + cc;
@@ -244,18 +278,17 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
                         else *(bi8_u32_unaligned *)dst = wq[h][0];
                     }
                 }
-            } else {
+            } else if (row < R) {
 #pragma unroll
                 for (int h = 0; h < NH; ++h) {
                     const int64_t col = cbase + h * kTC + cc;
                     int8_t *dst = q + row * ldq + col;
-                    if (row < R && col + VEC <= Cp) {
+                    if (col + VEC <= Cp) {
                         if constexpr (VEC == 8) *(bi8_v2u_unaligned *)dst = wq[h];
                         else *(bi8_u32_unaligned *)dst = wq[h][0];
-                    } else if (row < R) {
-#pragma unroll
-                        for (int e = 0; e < VEC - 1; ++e)
-                            if (col + e < Cp) dst[e] = (int8_t)((wq[h][e / 4] >> (8 * (e & 3))) & 0xffu);
+                    } else {
+#pragma nounroll
+                        for (int e = 0; e < (int)(Cp - col); ++e) dst[e] = (int8_t)((wq[h][VEC == 8 && e >= 4 ? 1 : 0] >> (8 * (e & 3))) & 0xffu);
                     }
                 }
             }
@@ -269,7 +302,7 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
             // precedes its phase 4); then start the next tile's loads of this half
 #pragma unroll
             for (int p = 0; p < NP; ++p) *(bi8_v4u *)&lds.x[(p * RPP + lr) * L::kXPitch + (tid % LPR) * 16] = raw[h][p];
-            if (next < ntiles) load_half(tr_n, tc_n, h, raw[h]);
+            if (FULL && next < ntiles) load_half(tr_n, tc_n, h, raw[h]);
             __syncthreads();
             if (h == 0) {
 #pragma unroll
@@ -383,14 +416,15 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
                 const int seg = idx % (kTR / 16);
                 const int64_t orow = c0 + oc;
                 const int64_t ocol = r0 + seg * 16;
-                if (FULL || (orow < C && ocol < Rp)) {
-                    const bi8_v4u v = *(const bi8_v4u *)&lds.q[oc * kQPitch + seg * 16];
-                    int8_t *dst = qT + orow * ldqt + ocol;
-                    if (FULL || ocol + 16 <= Rp) {
-                        __builtin_nontemporal_store(v, (bi8_v4u *)dst);
-                    } else {
-                        for (int e = 0; e < (int)(Rp - ocol); ++e) dst[e] = (int8_t)((v[e >> 2] >> (8 * (e & 3))) & 0xffu);
-                    }
+                const bi8_v4u v = *(const bi8_v4u *)&lds.q[oc * kQPitch + seg * 16];
+                int8_t *dst = qT + orow * ldqt + ocol;
+                if (all_rows) {
+                    if (FULL || orow < C) __builtin_nontemporal_store(v, (bi8_v4u *)dst);
+                } else if (orow < C && ocol + 16 <= Rp) {
+                    *(bi8_v4u *)dst = v;
+                } else if (orow < C) {
+#pragma nounroll
+                    for (int e = 0; e < (int)(Rp - ocol); ++e) dst[e] = (int8_t)((v[e >> 2] >> (8 * (e & 3))) & 0xffu);
                 }
             }
         }
@@ -398,6 +432,10 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
         tile = next;
         tr = tr_n;
         tc = tc_n;
+        if constexpr (!FULL) {                     // (a workgroup rarely has two of these: not under the tile before, which would spill)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) load_half(tr, tc, h, raw[h]);
+        }
     }
 }
 
