@@ -230,7 +230,9 @@ def test_kernel_choice_by_shape():
     assert name(8192, 8192, 8192, 128) == "gemm_wide" and name(8192, 8192, 8192, 64) == "gemm_wide"
     assert name(8192, 8192, 8192, 32) == "gemm_wide"                 # (the 32x32x32-MFMA form of the 256x256 kernel)
     assert name(2048, 4096, 4096, 32) == "gemm_tile_128x128"         # block 32 has no 256x128 tile
-    assert name(2944, 2944, 4096, 128) == "gemm_wide"                # 12 x 12 = 144 tiles of 256x256
+    assert name(3840, 3840, 4096, 128) == "gemm_wide"                # 15 x 15 = 225 tiles of 256x256: one round
+    # ... 12 x 12 = 144 of them: one round of 12 x 16 = 192 tiles of 256x192 leaves fewer CUs idle
+    assert name(2944, 2944, 4096, 128) == "gemm_wide_256x192" and name(2007, 5697, 1920, 64) == "gemm_wide_256x192"
     assert name(2944, 2944, 512, 128) == "gemm_wide_128x96" and name(5200, 5101, 384, 128) == "gemm_wide_128x128"
     # a last round of 256x256 tiles that is mostly empty: whole rows (columns) of tiles cut off for a second launch
     assert name(1536, 11008, 4096, 128) == "gemm_wide+gemm_tile_128x128" and name(2048, 11008, 4096, 128) == "gemm_wide+gemm_wide_256x128"

@@ -438,7 +438,7 @@ def _run_nonfinite_few_rows(ops, A, W, block, g):
 
 # (M, N, K, kernel family)
 NONFINITE_SHAPES = [(300, 500, 512, "gemm_panel"), (1500, 1500, 256, "gemm_panel_square"), (16, 6400, 256, "gemm_panel_few_rows"),
-                    (1500, 1500, 256, "gemm_tile_128x128", 32), (1708, 5200, 384, "gemm_wide"), (4876, 5000, 384, "gemm_wide"),
+                    (1500, 1500, 256, "gemm_tile_128x128", 32), (3700, 4090, 384, "gemm_wide"), (1708, 5200, 384, "gemm_wide_256x192"), (4876, 5000, 384, "gemm_wide"),
                     (2600, 2900, 256, "gemm_wide_128x128"), (5200, 5100, 256, "gemm_wide_128x128"), (2944, 2900, 384, "gemm_wide_128x96"),
                     (4400, 4500, 256, "gemm_wide+gemm_tile_128x128"), (2048, 2304, 256, "gemm_wide_256x128"),
                     (8, 256, 512, "gemv_staged"), (24, 256, 512, "gemv_staged_two_row_groups"), (24, 256, 512, "gemm_skinny", 32),

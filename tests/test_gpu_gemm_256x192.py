@@ -22,5 +22,5 @@ CASES = [
 def test_shape(case):
     from blockwise_int8_linear_amd import _lib
     M, N, K, block = case[:4]
-    assert _lib.load().bi8_gemm_kernel_name(M, N, K, K, K, block, 0).decode() == "gemm_wide"
+    assert _lib.load().bi8_gemm_kernel_name(M, N, K, K, K, block, 0).decode() == "gemm_wide_256x192"
     shapes.test_random_shape(case)

@@ -72,8 +72,10 @@ def _device_codes(A, pitch):
 
 # (M, N, K, block, kernel the shipped operator runs on it)
 CASES = [
-    (1708, 5200, 512, 128, "gemm_wide"),            # 147 tiles of 256x256, four stages
-    (1796, 5000, 384, 128, "gemm_wide"),            # odd number of stages (the loop runs a padding stage), ragged edges
+    (3840, 3840, 512, 128, "gemm_wide"),            # 225 tiles of 256x256, four stages
+    (3700, 4090, 384, 128, "gemm_wide"),            # odd number of stages (the loop runs a padding stage), ragged edges
+    (1708, 5200, 512, 128, "gemm_wide_256x192"),    # 196 tiles of 256x192, four stages
+    (1796, 5000, 384, 128, "gemm_wide_256x192"),    # odd number of stages (the loop runs a padding stage), ragged edges
     (2324, 5200, 256, 64, "gemm_wide"),             # two K-blocks per stage
     (3116, 3841, 384, 64, "gemm_wide"),
     (2944, 2944, 512, 128, "gemm_wide_128x96"),     # 713 tiles of 128x96, two workgroups per CU: they walk on to a second tile
