@@ -1,5 +1,4 @@
-"""What the built library's gfx950 code holds: hints that the sources give and a compiler may drop without a word."""
-import collections
+"""What the built library's gfx950 code holds: hints and orders that the sources give and a compiler may drop without a word."""
 import os
 import re
 import shutil
@@ -11,8 +10,8 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 
 
 @pytest.fixture(scope="module")
-def stores(tmp_path_factory):
-    """{kernel: {(width of a global store, non-temporal): how many}} of libbi8.so"""
+def kernels(tmp_path_factory):
+    """{kernel: its instructions} of libbi8.so"""
     from blockwise_int8_linear_amd import _lib
     if not os.path.exists(OBJDUMP):
         pytest.skip("no llvm-objdump")
@@ -23,22 +22,35 @@ def stores(tmp_path_factory):
     found = {}
     for part in sorted(p for p in os.listdir(at) if "gfx950" in p):
         code = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--demangle", part], cwd=at, check=True, capture_output=True, text=True).stdout
-        count = None
+        lines = None
         for line in code.splitlines():
             head = re.match(r"[0-9a-f]+ <(.*)>:", line)
             if head:
-                name = head.group(1).replace("(anonymous namespace)::", "").replace("void ", "").split("(")[0]
-                count = found.setdefault(name, collections.Counter())
-                continue
-            store = re.match(r"\s+global_store_(\w+)(.*)", line)
-            if store and count is not None:
-                count[store.group(1), re.search(r"\bnt\b", store.group(2).split("//")[0]) is not None] += 1
+                lines = found.setdefault(head.group(1).replace("(anonymous namespace)::", "").replace("void ", "").split("(")[0], [])
+            elif lines is not None:
+                lines.append(line.split("//")[0].strip())
     return found
 
 
-def test_last_tile_leaves_non_temporally(stores):
+def test_last_tile_leaves_non_temporally(kernels):
     """gemm_wide's workgroups store their last tile non-temporally and the tiles before it plainly: as many stores of either kind"""
-    kernels = {n: c for n, c in stores.items() if n.startswith("gemm_wide<") and n.split(", ")[3] == "false"}
-    assert len(kernels) == 30                      # two blocks, three output types, five tiles
-    for name, count in kernels.items():
-        assert count["dwordx4", True] == count["dwordx4", False] > 0, name
+    wide = {n: c for n, c in kernels.items() if n.startswith("gemm_wide<") and n.split(", ")[3] == "false"}
+    assert len(wide) == 30                         # two blocks, three output types, five tiles
+    for name, code in wide.items():
+        stores = [line.split()[-1] == "nt" for line in code if line.startswith("global_store_dwordx4")]
+        assert 2 * sum(stores) == len(stores) > 0, name
+
+
+def test_early_bias_is_not_waited_for(kernels):
+    """the few-row kernels ask for a 16-bit bias in front of their streams and convert it behind them: loads of the streams are issued
+    between the bias' load and the first wait for loads after it"""
+    few = {n: c for n, c in kernels.items() if n.startswith(("gemv_rows<", "gemv_staged<"))}
+    assert few
+    for name, code in few.items():
+        bias = next(i for i, line in enumerate(code) if line.startswith("global_load_ushort"))
+        wait = next(i for i in range(bias, len(code)) if line_waits_for_loads(code[i]))
+        assert any(line.startswith("buffer_load") for line in code[bias:wait]), name
+
+
+def line_waits_for_loads(line):
+    return line.startswith("s_waitcnt") and "vmcnt" in line
