@@ -82,8 +82,9 @@ template <int DT, int B, bool SUM, int NH> struct DualLds {
 // with all these -> this (before the two kinds of tiles): block 64 fp32 100 x 11008 7.7 -> 6.0 (6.6), 500 x 4096 8.2 -> 6.6 (7.0), 11008 x 100 9.1 ->
 // 6.7 (7.6), bf16 300 x 5003 7.2 -> 6.2 (9.0), 300 x 32768 14.4 -> 14.0 (12.8); block 128 bf16 1000 x 5003 11.3 -> 9.8 (15.3), fp32 12.7 -> 10.7 (16.5)
 // at 4097 x 1023.
+// ALONE: there are no full tiles; the loads are non-temporal like theirs (see quantize_dual_ends).
 // The workgroup's tiles: first_tile, first_tile + tile_step, ...
-template <int DT, int B, bool ALIGNED, bool SUM, int NH, bool FULL>
+template <int DT, int B, bool ALIGNED, bool SUM, int NH, bool FULL, bool ALONE = false>
 __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const void *__restrict__ x, int8_t *__restrict__ q, float *__restrict__ scales,
                                            int8_t *__restrict__ qT, float *__restrict__ scalesT, float *__restrict__ colsum_part, int64_t R, int64_t C, int64_t ldx,
                                            int64_t ldq, int64_t ldqt, int64_t Rp, int64_t Cp, int first_tile, int tile_step) {
@@ -138,7 +139,8 @@ __device__ __forceinline__ void dual_tiles(DualLds<DT, B, SUM, NH> &lds, const v
                 raw[p] = bi8_v4u{0u, 0u, 0u, 0u};
                 if (r0 + p * RPP + lr >= R || c0 + cc >= C) continue;
                 if constexpr (ALIGNED) {
-                    raw[p] = *(const bi8_v4u *)src;
+                    if constexpr (ALONE) raw[p] = __builtin_nontemporal_load((const bi8_v4u *)src);
+                    else raw[p] = *(const bi8_v4u *)src;
                 } else if (C >= VEC) {
                     raw[p] = *(const bi8_v4u_unaligned *)src;
                 } else {                           // a row shorter than a chunk
@@ -457,6 +459,16 @@ BI8_DUAL_KERNEL void quantize_dual_tile(const Bi8DualTask task, float *__restric
     dual_matrix<DT, B, ALIGNED, SUM, NH>(task, colsum_part, blockIdx.x, gridDim.x);
 }
 
+// A matrix without a full tile (fewer than 128 rows, say), its rows on 16-byte boundaries.  us, by the kernel above with plain loads -> this: block 64 fp32
+// 16 x 4096 4.2 -> 4.0, 100 x 32768 9.2 -> 8.2, 120 x 8192 6.8 -> 6.3, bf16 100 x 32768 7.2 -> 6.6, 100 x 11008 5.3 -> 5.0; block 128 fp32 100 x 11008
+// 8.9 -> 8.2, bf16 100 x 32768 9.0 -> 8.2.
+// Not under full tiles' kernels: there it costs fp32 with column sums up to six more spilled registers (4096 x 4096, block 64 25.3 -> 27.0), and
+// behind full tiles non-temporal loads lose (fp32 500 x 16384 14.7 -> 15.1).  No such kernel with column sums.
+template <int DT, int B, int NH> BI8_DUAL_KERNEL void quantize_dual_ends(const Bi8DualTask t) {
+    __shared__ DualLds<DT, B, false, NH> lds;
+    dual_tiles<DT, B, true, false, NH, false, true>(lds, t.x, t.q, t.scales, t.qT, t.scalesT, nullptr, t.R, t.C, t.ldx, t.ldq, t.ldqt, t.Rp, t.Cp, blockIdx.x, gridDim.x);
+}
+
 // Two matrices: the grid's first blocks0 workgroups work on the first, the others on the second (a layer's X and W: one launch, and
 // the smaller of the two does not have the chip to itself half empty).
 struct DualPair {
@@ -477,6 +489,12 @@ template <int DT, int B, bool ALIGNED, int NH> int launch_one(const Bi8DualTask 
     const int64_t ntiles = ((t.Cp + NH * kTC - 1) / (NH * kTC)) * ((t.Rp + kTR - 1) / kTR);
     if (ntiles + resident > 0x7fffffffLL) return BI8_ERR_TOO_LARGE;
     const dim3 grid((unsigned)(ntiles < resident ? ntiles : resident));
+    if constexpr (ALIGNED) {
+        if (!colsum_part && (t.R < kTR || t.C < NH * kTC)) {
+            hipLaunchKernelGGL((quantize_dual_ends<DT, B, NH>), grid, dim3(kThreads), 0, st, t);
+            return bi8_launch_rc();
+        }
+    }
     if (colsum_part) hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, true, NH>), grid, dim3(kThreads), 0, st, t, colsum_part);
     else hipLaunchKernelGGL((quantize_dual_tile<DT, B, ALIGNED, false, NH>), grid, dim3(kThreads), 0, st, t, colsum_part);
     return bi8_launch_rc();
