@@ -522,15 +522,27 @@ template <int DT, int B, bool ALIGNED, int NH> int launch_pair(const Bi8DualTask
     return bi8_launch_rc();
 }
 
+// Whole tiles also where that is two for each CU and not a third but at the matrix' ends: as half tiles those at the ends are a workgroup's
+// second ones, which are not loaded under the first.  us, half / whole (before the two kinds of tiles; half ones), block 64: bf16 300 x 32768
+// 13.7 / 12.2 (12.8), 1000 x 8192 11.3 / 10.5 (11.5), 8192 x 1000 13.4 / 12.2 (13.6), 2048 x 4096 10.9 / 10.3 (11.0), 700 x 12288 12.4 / 11.7 (12.8), two of 1000 x
+// 4096 11.6 / 10.3 (10.8); fp32 8192 x 1000 16.7 / 16.0 (15.8), 500 x 16384 14.5 / 14.3 (14.5), 700 x 12288 16.0 / 15.6 (16.2).  With fewer elements (300 x 24576
+// bf16 11.2 / 11.6, fp32 13.9 / 15.0), a third tile (11008 x 768 bf16 11.2 / 12.1, fp32 15.1 / 17.1; 1000 x 11008 bf16 14.2 / 14.4), rows off 16-byte boundaries
+// (2000 x 5003 14.8 / 15.2, fp32 18.7 / 20.6), fp32 without ends (4096 x 2048 13.8 / 14.0) or with column sums (8192 x 1024 13.7 / 14.4): half ones.
+constexpr int64_t kTwoEachElems = 8000000;
 template <int DT, int B, bool ALIGNED> int launch_dual(const Bi8DualTask *task, int count, float *colsum_part, hipStream_t st) {
     // workgroups per CU: four with 16-bit inputs (30 KiB of LDS, at most 128 registers), three with fp32 (43 KiB, 168).  us with three
     // / four: bf16 [8192,4096] 29.5 / 28.6, [8192,3072] 22.7 / 22.7, fp32 [4096,4096] 23.5 / 27.9
     const int64_t resident = (DT == BI8_F32 ? 3 : 4) * 256;
     // inputs of fewer full tiles than the chip holds workgroups: half tiles, twice as many workgroups
-    int64_t full = 0;
-    for (int i = 0; i < count; ++i) full += ((task[i].Cp + 2 * kTC - 1) / (2 * kTC)) * ((task[i].Rp + kTR - 1) / kTR);
+    int64_t full = 0, inside = 0, elems = 0;
+    for (int i = 0; i < count; ++i) {
+        full += ((task[i].Cp + 2 * kTC - 1) / (2 * kTC)) * ((task[i].Rp + kTR - 1) / kTR);
+        inside += (task[i].C / (2 * kTC)) * (task[i].R / kTR);
+        elems += task[i].R * task[i].C;
+    }
     constexpr int kHalf = B <= kTC ? 1 : 2;
-    const bool half = full < resident;
+    const bool two_each = ALIGNED && elems >= kTwoEachElems && inside <= 2 * 256 && (DT != BI8_F32 || (!colsum_part && inside < full));
+    const bool half = full < resident && !two_each;
     if (count == 1)
         return half ? launch_one<DT, B, ALIGNED, kHalf>(task[0], colsum_part, resident, st) : launch_one<DT, B, ALIGNED, 2>(task[0], colsum_part, resident, st);
     const int rc = half ? launch_pair<DT, B, ALIGNED, kHalf>(task, resident, st) : launch_pair<DT, B, ALIGNED, 2>(task, resident, st);

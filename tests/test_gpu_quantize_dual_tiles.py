@@ -24,7 +24,8 @@ def _up(n, to=128):
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("R,C", [(128, 64), (5, 3), (260, 1032), (1000, 2304), (129, 70001), (4230, 4104), (3000, 5003), (2048, 8192),
                                  (130, 199), (131, 202), (132, 204), (97, 205), (33, 206), (40, 9), (7, 4),           # rows that end anywhere in 16 bytes
-                                 (1, 4096), (70, 4104), (127, 40000), (11008, 40)])                       # no tile inside the matrix
+                                 (1, 4096), (70, 4104), (127, 40000), (11008, 40),                        # no tile inside the matrix
+                                 (300, 32768), (8192, 1000), (8200, 1032), (2048, 4096)])                 # two whole tiles for each CU, and those at the ends
 def test_codes_and_scales(R, C, dtype, block):
     from blockwise_int8_linear_amd import _lib
     run = _lib.load().bi8x_quantize_dual
