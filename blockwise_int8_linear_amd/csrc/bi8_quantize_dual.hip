@@ -4,7 +4,8 @@
 // quantizes each of X, W and G twice, once per direction (block_linear.py:77-78, :92-94, :100-103): with this kernel
 // every one of them is read from HBM once.
 //
-// What bounds it: memory, at 5.0 TB/s of the 272 MB of bf16 [8192,8192], block 128 (a copy with these access widths: 6.2), behind it ~20
+// What bounds it: memory, at 4.7 to 5.0 TB/s (58 to 54 us, machine to machine) of the 272 MB of bf16 [8192,8192], block 128 (a copy with
+// these access widths: 6.2), behind it ~20
 // vector instructions per element.  us, a branch around every load and store, per-element NaN tests and the IEEE path inside each
 // row -> this: bf16 block 128 [8192,8192] 57.9 -> 54.2, [4096,11008] 44.4 -> 41.8, [11008,4096] 40.8 -> 39.0; block 64 [8192,3072] with
 // column sums 29.0 -> 23.2, [8192,50257] 414 -> 380 ([8192,50304]: 360 -> 345); fp32 [8192,8192] 114 -> 85 (three workgroups per CU for two).
@@ -12,8 +13,8 @@
 // A workgroup owns a 128 x 128 tile, held in registers as two 64-column halves (16 bytes per lane per row pass; the
 // next tile's loads are issued while this one is processed).  The row direction is finished straight from the
 // registers: the lanes of one row reduce their absmax with DPP, quantize and store their codes.  The column direction
-// runs half by half through LDS exactly as in bi8_quantize_transposed (tile kept in its own type, 16-byte LDS accesses).  Both outputs are bit for bit those of the
-// two separate entry points.
+// runs half by half through LDS exactly as in bi8_quantize_transposed (tile kept in its own type, 16-byte LDS accesses).  Both
+// outputs are bit for bit those of the two separate entry points.
 //
 // bi8_quantize_dual_colsum also returns the column sums of x (the bias gradient G.sum(dim=0) of block_linear.py:110,
 // when x is the output gradient G): the column walk has every element in a register anyway, so each thread adds up its
