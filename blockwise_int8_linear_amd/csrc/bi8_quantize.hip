@@ -197,18 +197,24 @@ int launch_rows(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, i
 // fp16 100 x 11008 2.3 / 2.7 / 3.0 (3.9), 300 x 16384 4.9 / 4.8 / 5.3 (5.4); fp32, block 32 1000 x 5004 7.6 / 7.5 / 7.0 (7.2).
 // Rows off 16-byte boundaries run with one whatever the size where a KiB of row holds at most eight blocks: bf16, block 128 1000 x 5003
 // 5.6 / 5.6 / 7.2 (9.1), 8192 x 50257 250 / 279 / 280 (278), block 64 267 / 290 / 287 (282); fp32, block 32 8192 x 50257 472 / 514 / 516 (505).
-// With one row per wave every scale is a 4-byte store by itself; smaller blocks, sixteen stores and more per KiB, go by the size: bf16,
-// block 32 8192 x 50257 320 / 317 / 297 (293), 8192 x 5001 32.4 / 30.2 / 30.5 (32.0); block 8 672 / 473 / 352 (343), 53.4 / 40.6 / 34.3 (35.9); fp32,
-// block 16 8192 x 50257 571 / 570 / 531 (530); with two at most where a row is short: block 32, fp16 20000 x 1001 18.7 / 20.4 / 22.4 (20.3), 65536 x 251
-// 28.7 / 25.5 / 29.0 (28.3).
+// With one row per wave every scale is a 4-byte store by itself; smaller blocks, sixteen stores and more per KiB, go with two rows in
+// larger calls: from the line for aligned rows on, L = 4 from the next, where codes in the caches are read behind it (quantize + dequantize,
+// bf16 block 32 2000 x 3001 12.0 with one, 13.5 with two; 2000 x 5003 17.2 / 16.7), and there not where a row of 16-bit elements is two to four
+// runs; with four only at L = 1.  us with 1 / 2 / 4, from memory: bf16, block 32 4810 x 3658 16.0 / 14.7 / 15.1 (with 4 before: 19.0), 6000 x 5003 25.2 /
+// 23.2 / 24.0, 8192 x 50257 320 / 317 / 297, 8192 x 2001 15.0 / 15.2 / 15.2; fp16, block 32 2000 x 5003 10.6 / 10.0 / 11.3 (13.0), 4810 x 3658 15.9 / 15.1 /
+// 17.6, 8192 x 2001 14.9 / 16.3 / 17.6, 20000 x 1001 17.9 / 19.8 / 21.6, 65536 x 251 28.7 / 25.5 / 29.0 (28.3); bf16, block 16 2000 x 5003 12.3 / 10.2 / 10.7, 8192 x
+// 2001 17.4 / 15.6 / 15.6; block 8 8192 x 50257 672 / 473 / 352 (343), 8192 x 5001 53.4 / 40.6 / 34.3 (35.9); fp32, block 16 4000 x 3001 16.8 / 15.3 / 15.4.
 constexpr int64_t kOneRowWaves = 24 * 256, kTwoRowWaves = 72 * 256;
 template <int DT, int L, bool ALIGNED>
 int launch_vec(const void *x, int8_t *q, float *scales, int64_t M, int64_t K, int64_t Kp, int64_t ldx, int64_t ldq, hipStream_t st) {
     constexpr int TE = BI8_WAVE * Bi8Vec<DT>::kElems;
     const int64_t runs = (Kp + TE - 1) / TE, waves = M * runs;
-    if constexpr (ALIGNED || L <= 4) {
+    if constexpr (ALIGNED || L == 1) {
         if (waves > kTwoRowWaves && (ALIGNED || runs > 4)) return launch_rows<DT, L, ALIGNED, 4>(x, q, scales, M, K, Kp, ldx, ldq, st);
         if (waves > kOneRowWaves) return launch_rows<DT, L, ALIGNED, 2>(x, q, scales, M, K, Kp, ldx, ldq, st);
+    } else if constexpr (L == 2 || L == 4) {
+        if (waves > (L == 4 ? kTwoRowWaves : kOneRowWaves) && (L == 2 || DT == BI8_F32 || runs > 4 || runs == 1))
+            return launch_rows<DT, L, ALIGNED, 2>(x, q, scales, M, K, Kp, ldx, ldq, st);
     }
     return launch_rows<DT, L, ALIGNED, 1>(x, q, scales, M, K, Kp, ldx, ldq, st);
 }

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("block", [8, 32, 128, 256])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("M,K", [(1, 256), (7, 264), (1025, 1544), (1023, 4104), (2051, 4104), (5003, 2056), (1030, 5003), (3, 17), (4097, 128), (9301, 523), (3101, 3011)])
+@pytest.mark.parametrize("M,K", [(1, 256), (7, 264), (1025, 1544), (1023, 4104), (2051, 4104), (5003, 2056), (1030, 5003), (3, 17), (4097, 128), (9301, 523), (3101, 3011), (18501, 203)])
 def test_codes_and_scales(M, K, dtype, block):
     import blockwise_int8_linear_amd as pkg
     g = torch.Generator().manual_seed(M + K)
