@@ -195,20 +195,24 @@ __global__ __launch_bounds__(kThreads) void dequantize_rows_generic(const int8_t
 // 6.0 / 5.4 (6.0), 65536 x 256 17.4 / 13.6 / 12.7 (13.6), 24000 x 512 9.9 / 9.0 / 7.6 (9.0), 36000 x 512 13.9 / 12.6 / 13.0 (12.6); fp32 12000 x 256 4.9 / 3.8 /
 // 3.8 (4.0), 24000 x 256 8.9 / 7.2 / 6.0 (7.2), 65536 x 256 21.0 / 16.5 / 17.4 (16.6).  Off 16-byte boundaries one or four: bf16 12000 x 251 6.2 for one, 7.2
 // for four (6.2), 65536 x 251 31.2 / 25.6 (26.5), fp32 33.0 / 28.6 (28.0).
-// Rows off 16-byte boundaries: one chunk per wave in larger calls too (fp32 larger than 16-bit ones), then, where a row has more than
-// two, one row of four chunks (a wave's run cuts lines at its two ends only).  Codes from memory / quantizer and this with all in the caches,
-// 1 x 1, 1 x 4, 2 x 2 (before): block 32 fp32 700 x 5003 8.0 / 10.9, 7.2 / 11.5, 8.0 / 11.6 (8.0 / 11.7), 1000 x 5003 10.3 / 13.5, 9.0 / 13.9, 9.6 / 13.9 (9.8 /
-// 14.1), 8192 x 5001 50.9 / 94.7, 46.3 / 94.7, 47.7 / 94.4 (50.0 / 94.7); bf16 1000 x 5003 8.0 / 11.6, 7.3 / 11.6, 8.6 / 12.7 (8.8 / 12.8), 2048 x 5001 11.8 /
-// 16.9, 10.2 / 17.0, 11.0 / 16.9 (10.6 / 16.9), 3000 x 5001 15.7 / 22.2, 15.1 / 22.0, 14.8 / 21.1 (14.7 / 21.4).
+// Rows off 16-byte boundaries: one chunk per wave in larger calls too (fp32 larger than 16-bit ones), then one row of four chunks (a wave's run
+// cuts lines at its two ends only) where these fill five of six waves' chunks at least and a chunk holds few scales (blocks from 32 on: a wave
+// of one row reads each from memory by itself).  Codes from memory, 1 x 1, 1 x 4, 2 x 2 (before: 2 x 2, loads that waited for one another): bf16
+// block 32 1500 x 5003 8.9, 8.4, 9.3 (9.3), 1900 x 5003 10.9, 9.9, 10.6 (10.5), 2600 x 5003 14.3, 13.3, 13.9 (13.8), 1300 x 10001 13.7, 13.0, 12.4 (12.1); block 128
+// 2300 x 5003 13.5, 11.5, 13.0 (12.4); fp32 block 32 1200 x 5003 11.4, 9.9, 10.2 (10.3), 900 x 10001 14.0, 12.8, 12.9 (13.0), 6000 x 5003 block 16 43, 42, 37 (40).  Filled less: bf16
+// block 32 4500 x 2049 10.1, 12.9, 8.9 (9.0), 2500 x 3001 8.0, 7.9, 8.6 (8.7), 4000 x 3001 13.1, 14.2, 12.5 (11.6), fp32 4000 x 1201 8.5, 8.3, 7.3 (7.4).  More scales: bf16 block 16
+// 1500 x 5003 9.1, 9.5, 10.0 (9.9), 3000 x 3001 10.3, 11.7, 9.9 (9.8), fp32 3000 x 3001 14.3, 15.0, 14.0 (13.7).
 constexpr int64_t kOneRunWaves = 24 * 256, kOneShortRowWavesRagged = 96 * 256;
-template <int DT> constexpr int64_t kOneRunWavesRagged = (DT == BI8_F32 ? 88 : 56) * 256;
-template <int DT> constexpr int64_t kOneRowWavesRagged = (DT == BI8_F32 ? 144 : 112) * 256;
+template <int DT> constexpr int64_t kOneRunWavesRagged = (DT == BI8_F32 ? 88 : 64) * 256;
+template <int DT> constexpr int64_t kOneRunWavesFilled = (DT == BI8_F32 ? 88 : 56) * 256;
+template <int DT> constexpr int64_t kOneRowWavesFilled = (DT == BI8_F32 ? 144 : 96) * 256;
 constexpr int64_t kTwoShortRowsWaves = 64 * 256, kFourLongerRowsWaves = 128 * 256;
 template <int DT, bool ALIGNED>
 int launch_vec(const int8_t *q, const float *scales, void *out, int64_t M, int64_t K, int64_t ldq, int64_t ldo, int block, hipStream_t st) {
     constexpr int kChunk = BI8_WAVE * Out<DT>::kElems;
-    const int64_t waves = M * ((K + kChunk - 1) / kChunk);
-    if (waves <= (ALIGNED ? kOneRunWaves : K <= kChunk ? kOneShortRowWavesRagged : kOneRunWavesRagged<DT>))
+    const int64_t runs = (K + kChunk - 1) / kChunk, waves = M * runs;
+    const bool filled = !ALIGNED && block >= 32 && 6 * runs >= 5 * 4 * ((runs + 3) / 4);      // ... with waves of one row of four chunks
+    if (waves <= (ALIGNED ? kOneRunWaves : K <= kChunk ? kOneShortRowWavesRagged : filled ? kOneRunWavesFilled<DT> : kOneRunWavesRagged<DT>))
         return launch_rows<DT, ALIGNED, 1, 1>(q, scales, out, M, K, ldq, ldo, block, st);
     if (K <= kChunk) {
         if constexpr (ALIGNED)
@@ -216,7 +220,7 @@ int launch_vec(const int8_t *q, const float *scales, void *out, int64_t M, int64
         return launch_rows<DT, ALIGNED, 4, 1>(q, scales, out, M, K, ldq, ldo, block, st);
     }
     if constexpr (!ALIGNED)
-        if (K > 2 * kChunk && waves <= kOneRowWavesRagged<DT>) return launch_rows<DT, ALIGNED, 1, 4>(q, scales, out, M, K, ldq, ldo, block, st);
+        if (filled && waves <= kOneRowWavesFilled<DT>) return launch_rows<DT, ALIGNED, 1, 4>(q, scales, out, M, K, ldq, ldo, block, st);
     return launch_rows<DT, ALIGNED, 2, 2>(q, scales, out, M, K, ldq, ldo, block, st);
 }
 

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("out", list(DTYPES))
 @pytest.mark.parametrize("M,K,B", [(6144, 256, 64), (6145, 248, 64), (6147, 512, 128), (3001, 2056, 32), (2051, 4104, 128), (24577, 255, 64), (9001, 2049, 128), (5003, 1028, 256), (17001, 128, 32), (33001, 256, 64),
-                                   (1027, 5003, 32), (1003, 3003, 64), (3007, 2049, 128), (7, 20001, 32)])
+                                   (1027, 5003, 32), (1003, 3003, 64), (3007, 2049, 128), (7, 20001, 32), (1701, 5003, 32), (1201, 5003, 64), (1701, 5003, 16), (4501, 2049, 32)])
 def test_values(M, K, B, out):
     import blockwise_int8_linear_amd as pkg
     g = torch.Generator().manual_seed(M + K)
