@@ -37,6 +37,12 @@ int bi8x_gemm(const int8_t *A, const int8_t *W, const float *sA, const float *sW
               int64_t M, int64_t N, int64_t K, int64_t kw, int64_t lda, int64_t ldw, int64_t ldc, int block, void *workspace,
               int64_t workspace_bytes, void *stream);
 
+/* y [M,N] = x [M,K] @ W.T + bias for 3 to 16 rows in one launch: x of C's type is quantized by the workgroups that multiply with it, the
+ * bits of y are those of bi8_quantize_rowwise and bi8_gemm_nt_dequant_ws.  W, sW: codes and scales; blocks 64 and 128, K a multiple of
+ * 128, x and W with 16-byte aligned rows, and up to 16 Ki activations (fp32: 8 Ki; BI8_ERR_UNSUPPORTED otherwise). */
+int bi8x_linear_rows(const void *x, int dtype, const int8_t *W, const float *sW, const void *bias, int bias_dtype, void *C, int64_t M,
+                     int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldc, int block, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -298,6 +298,16 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
     void *const stream = stream_of(x);
 
     if (fast_block(B) && M > 0 && N > 0 && K > 0) {
+        Tensor out = empty(with_last(x_in, N), cfg.out_type, x);
+        const Bias bias(bias_in, N);
+        // a few rows against codes that are ready: one launch, where the library covers it
+        if (M >= 3 && M <= 16 && !w.defined() && !need_xt && x_code == dtype_code(cfg.out_type) && cfg.scale_type == at::kFloat && w_state.scalar_type() == at::kFloat &&
+            w_state.is_contiguous() && w_int8.stride(1) == 1) {
+            const int rc = bi8x_linear_rows(x.data_ptr(), x_code, (const int8_t *)w_int8.data_ptr(), (const float *)w_state.data_ptr(), bias.ptr, bias.code, out.data_ptr(), M,
+                                            N, K, ld_of(x), ld_of(w_int8), N, (int)B, stream);
+            if (rc == BI8_OK) return out;
+            if (rc != BI8_ERR_UNSUPPORTED) check(rc, "bi8x_linear_rows");
+        }
         // one allocation for what does not outlive the call
         const Packed xq = pack(M, K, B), wq = pack(w.defined() ? N : 0, K, B, xq.end()), xtq = pack(K, M, B), wtq = pack(K, N, B, need_xt ? xtq.end() : 0);
         const bool pad = pad_contraction(M, N, K, B);
@@ -327,8 +337,6 @@ Tensor linear_forward(const Tensor &x_in, const Tensor &w_in, const Tensor &w_in
         } else if (w.defined()) {
             quantize_rows(w, t, wq, cfg, stream);
         }
-        Tensor out = empty(with_last(x_in, N), cfg.out_type, x);
-        const Bias bias(bias_in, N);
         void *const ws = need > 0 ? (uint8_t *)t.data_ptr() + ws_at : nullptr;
         if (w.defined()) {
             check(gemm_raw(xq.codes(t), xq.scales(t), xq.ld, wq.codes(t), wq.scales(t), wq.ld, bias, out.data_ptr(), float_code(out), M, N, kp, kp, B, ws, need, stream), "bi8x_gemm");
