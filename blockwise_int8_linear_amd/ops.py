@@ -177,7 +177,7 @@ _ws_need = {}                       # (M, N, K, block) -> bytes of scratch memor
 
 def _workspace(lib, M, N, K, block, device, stream):
     """Scratch memory for a GEMM of fewer output tiles than compute units (the library then splits K over the
-    workgroups and sums the pieces): (tensor or None, bytes).  What a shape wants is asked once; the memory (at most 32 MiB) is
+    workgroups and sums the pieces): (tensor or None, bytes).  What a shape wants is asked once; the memory (at most 48 MiB) is
     the call's own, from torch's allocator on the current stream: the split and its sum are two launches, and those of two
     threads that use one stream may be queued in between one another.
     (Up to 16 rows at blocks 64 / 128 run the one-pass decode kernels whatever they are given: not asked.)"""

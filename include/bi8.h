@@ -148,9 +148,10 @@ int bi8_gemm_nt_dequant_ws(const int8_t *A, const int8_t *W, const float *sA, co
  * cannot allocate -- code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  The call
  * makes no hipMalloc / hipFree and no allocating library call; the first call on a device looks up the array's
  * address there (hipGetSymbolAddress), so make one call on each device outside any capture.
- * Same kernels, same results (bit for bit) as bi8_gemm_nt_dequant_ws given bi8_gemm_workspace_bytes() of workspace.
- * A problem whose split wants more than the array holds returns BI8_ERR_SCRATCH_TOO_SMALL and launches nothing (with
- * the present split rule -- fewer than 512 slabs of 128 x 128 fp32 -- no problem does).
+ * Same kernels, same results (bit for bit) as bi8_gemm_nt_dequant_ws given a workspace of 32 MiB, or of
+ * bi8_gemm_workspace_bytes() where that is less: only the split of a long K of more than 512 rows ("gemm_wide_256x192_splitk")
+ * wants more than the array holds, and is not used here.  (BI8_ERR_SCRATCH_TOO_SMALL: a split that only fits a larger
+ * array; with the present rules there is none.)
  * All calls on one GPU share the array, which keeps the last call's contents (every call overwrites what it reads,
  * nothing has to start at zero): calls that overlap on one GPU -- two streams, two host threads -- race on it.
  * Serialize them on one stream, or give the overlapping ones their own workspace through bi8_gemm_nt_dequant_ws.
@@ -164,7 +165,7 @@ int bi8_gemm_nt_dequant_static(const int8_t *A, const int8_t *W, const float *sA
 /*
  * Name of the kernel family that bi8_gemm_nt_dequant_ws runs on a problem with 16-byte aligned operands and
  * `workspace_bytes` of scratch memory ("gemm_wide" for 256x256 tiles, "gemm_wide_256x192", "gemm_wide_256x128", "gemm_wide_128x128",
- * "gemm_wide_128x96", "gemm_wide_256x128_splitk", "gemm_tile_256x128", "gemm_tile_128x128", "gemm_tile_64x128", "gemm_tile_128x128_splitk", "gemm_tile_64x128_splitk", "gemm_panel", "gemm_panel_splitk", "gemv_rows",
+ * "gemm_wide_128x96", "gemm_wide_256x128_splitk", "gemm_wide_256x192_splitk", "gemm_tile_256x128", "gemm_tile_128x128", "gemm_tile_64x128", "gemm_tile_128x128_splitk", "gemm_tile_64x128_splitk", "gemm_panel", "gemm_panel_splitk", "gemv_rows",
  * "gemv_staged", "gemm_skinny", "gemm_generic"; "gemm_wide+<tile kernel>" for a problem that runs as two launches, the 256x256 kernel on the leading
  * rows or columns that fill whole rounds of workgroups and a tile kernel on the rest; "none" for an empty problem).
  * Static string.  The reference picks its kernel configuration with Triton's autotuner
