@@ -37,6 +37,19 @@ int bi8x_gemm(const int8_t *A, const int8_t *W, const float *sA, const float *sW
               int64_t M, int64_t N, int64_t K, int64_t kw, int64_t lda, int64_t ldw, int64_t ldc, int block, void *workspace,
               int64_t workspace_bytes, void *stream);
 
+/* One problem of bi8x_gemm_pair: what bi8x_gemm takes, without a bias. */
+typedef struct {
+    const int8_t *A, *W;
+    const float *sA, *sW;
+    void *C;
+    int64_t M, N, K, kw, lda, ldw, ldc;
+} Bi8Gemm;
+/* Both problems in one launch where that is expected to be faster than two (BI8_ERR_UNSUPPORTED otherwise: nothing is launched); outputs of type
+ * c_dtype, operands as for bi8x_gemm with rows on 16-byte boundaries, blocks 64 and 128, no scratch memory.  _name: the kernel whose
+ * tiles the launch runs, "" where there would be none. */
+int bi8x_gemm_pair(const Bi8Gemm *q, int c_dtype, int block, void *stream);
+const char *bi8x_gemm_pair_name(const Bi8Gemm *q, int block);
+
 /* y [M,N] = x [M,K] @ W.T + bias for 3 to 16 rows in one launch: x of C's type is quantized by the workgroups that multiply with it, the
  * bits of y are those of bi8_quantize_rowwise and bi8_gemm_nt_dequant_ws.  W, sW: codes and scales; blocks 64 and 128, K a multiple of
  * 128, x and W with 16-byte aligned rows, and up to 16 Ki activations (fp32: 8 Ki; BI8_ERR_UNSUPPORTED otherwise). */

@@ -406,8 +406,21 @@ torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &
             round_scales(t, gtq, cfg.scale_type);
         }
         const Bias none(Tensor(), 0);
-        if (need_gx) {
-            Tensor gx = empty(s.x_sizes, cfg.out_type, G);
+        Tensor gx = need_gx ? empty(s.x_sizes, cfg.out_type, G) : Tensor(), gw = need_gw ? empty({N, K}, cfg.out_type, G) : Tensor();
+        bool paired = false;                       // both in one launch, where the library would have it so
+        if (both && kx == gq.ld && kw == gtq.ld) {
+            const Tensor w = s.wt_packed ? Tensor() : rows_of(held[2]), ws = s.wt_packed ? Tensor() : scales_in(held[3]);
+            if (s.wt_packed || ready_operand(w, N, B)) {
+                const Bi8Gemm pair[2] = {{gq.codes(t), s.wt_packed ? wtq.codes(held[2]) : (const int8_t *)w.data_ptr(), gq.scales(t),
+                                          s.wt_packed ? wtq.scales(held[2]) : (const float *)ws.data_ptr(), gx.data_ptr(), M, K, kx, s.wt_packed ? kx : up(N, 16), gq.ld,
+                                          s.wt_packed ? wtq.ld : ld_of(w), std::max<int64_t>(K, 1)},
+                                         {gtq.codes(t), xtq.codes(held[0]), gtq.scales(t), xtq.scales(held[0]), gw.data_ptr(), N, K, kw, kw, gtq.ld, xtq.ld, std::max<int64_t>(K, 1)}};
+                const int rc = bi8x_gemm_pair(pair, float_code(gx), (int)B, stream);
+                if (rc != BI8_ERR_UNSUPPORTED) check(rc, "bi8x_gemm_pair");
+                paired = rc == BI8_OK;
+            }
+        }
+        if (need_gx && !paired) {
             void *const ws = need1 > 0 ? base + ws_at : nullptr;
             if (s.wt_packed) {
                 check(gemm_raw(gq.codes(t), gq.scales(t), gq.ld, wtq.codes(held[2]), wtq.scales(held[2]), wtq.ld, none, gx.data_ptr(), float_code(gx), M, K, kx, kx, B,
@@ -416,15 +429,14 @@ torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &
             } else {
                 multiply_ready(gq, t, held[2], held[3], N, none, gx, M, K, B, ws, need1, stream);
             }
-            result[0] = gx;
         }
-        if (need_gw) {
-            Tensor gw = empty({N, K}, cfg.out_type, G);
+        if (need_gw && !paired) {
             check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, kw, kw, B,
                            need2 > 0 ? base + ws_at : nullptr, need2, stream),
                   "bi8x_gemm");
-            result[1] = gw;
         }
+        result[0] = gx;
+        result[1] = gw;
         if (sums) {
             Tensor gb = empty({N}, G.scalar_type(), G);
             check(bi8x_colsum_finish((const float *)(base + part_at), gb.data_ptr(), g_code, M, N, stream), "bi8x_colsum_finish");

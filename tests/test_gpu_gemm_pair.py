@@ -1,0 +1,98 @@
+"""Two GEMMs in one launch (bi8x_gemm_pair): every tile that the rule chooses, both blocks, ragged edges, several tiles per workgroup, an odd number
+of stages and rows of W that hold less than the padded contraction; the bits of the one-pass kernels, and nothing beside the outputs."""
+import ctypes
+
+import pytest
+import torch
+
+from util import DTYPES
+
+_vp, _i64 = ctypes.c_void_p, ctypes.c_int64
+
+
+class Gemm(ctypes.Structure):
+    _fields_ = [(n, _vp) for n in ("A", "W", "sA", "sW", "C")] + [(n, _i64) for n in ("M", "N", "K", "kw", "lda", "ldw", "ldc")]
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from blockwise_int8_linear_amd import _lib
+    lib = _lib.load()
+    lib.bi8x_gemm_pair.argtypes = [_vp, ctypes.c_int, ctypes.c_int, _vp]
+    lib.bi8x_gemm_pair_name.argtypes, lib.bi8x_gemm_pair_name.restype = [_vp, ctypes.c_int], ctypes.c_char_p
+    lib.bi8x_gemm.argtypes = [_vp] * 5 + [ctypes.c_int, _vp, ctypes.c_int] + [_i64] * 7 + [ctypes.c_int, _vp, _i64, _vp]
+    return lib
+
+
+def _up(n, to):
+    return -(-n // to) * to
+
+
+def _sizes(tokens, k, n):
+    """grad_X and grad_W of a layer as (M, N, contraction)"""
+    return (tokens, k, n), (n, k, tokens)
+
+
+def _name(lib, sizes, block, at=4096, **over):
+    q = (Gemm * 2)(*(Gemm(at, at, at, at, at, m, n, _up(k, 128), _up(k, 128), _up(k, 128), _up(k, 128), n) for m, n, k in sizes))
+    for field, value in over.items():
+        setattr(q[1], field, value)
+    return lib.bi8x_gemm_pair_name(ctypes.byref(q), block).decode()
+
+
+# tokens, in, out, block, the tile
+CASES = [
+    (418, 1731, 578, 64, "gemm_wide_128x96"),        # ragged rows and columns, rows of C off 16-byte boundaries
+    (1497, 2001, 1500, 64, "gemm_wide_128x96"),      # more tiles than one round of either share
+    (133, 9536, 573, 128, "gemm_wide_128x96"),       # a second problem of two stages
+    (937, 1664, 897, 64, "gemm_wide_128x128"),
+    (458, 2689, 896, 128, "gemm_wide_128x128"),
+    (667, 5184, 1283, 64, "gemm_wide_256x128"),      # an odd number of stages
+    (1328, 2304, 1664, 128, "gemm_wide_256x128"),
+    (2136, 2368, 1746, 64, "gemm_wide_256x192"),
+    (2374, 1472, 3009, 128, "gemm_wide_256x192"),
+    (2420, 6656, 896, 64, "gemm_wide"),
+    (776, 7103, 1280, 128, "gemm_wide"),             # several tiles per workgroup
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("tokens,k,n,block,tile", CASES)
+def test_bits_of_the_one_pass_kernels(lib, tokens, k, n, block, tile, dtype):
+    sizes = _sizes(tokens, k, n)
+    assert _name(lib, sizes, block) == tile
+    gen = torch.Generator(device="cuda:0").manual_seed(tokens + k + n)
+    stream, code = torch.cuda.current_stream().cuda_stream, ["f32", "bf16", "f16"].index(dtype)
+    held, q, want, out = [], [], [], []
+    for i, (M, N, K) in enumerate(sizes):
+        kp, kw = _up(K, 128), _up(K, 16) if i == 0 else _up(K, 128)      # the first problem's W: a view of rows that are farther apart than kw
+        A, W = (torch.randint(-127, 128, (rows, kp), dtype=torch.int8, generator=gen, device="cuda:0") for rows in (M, N))
+        A[:, K:] = 0
+        sa, sw = torch.rand(kp // block, M, generator=gen, device="cuda:0") + 0.01, torch.rand(-(-kw // block), N, generator=gen, device="cuda:0") + 0.01
+        sa[-(-K // block):] = 0
+        guard = torch.full((M + 2, N), 7.0, dtype=DTYPES[dtype], device="cuda:0")
+        one = torch.empty(M, N, dtype=DTYPES[dtype], device="cuda:0")
+        assert lib.bi8x_gemm(A.data_ptr(), W.data_ptr(), sa.data_ptr(), sw.data_ptr(), None, 0, one.data_ptr(), code, M, N, kp, kw, kp, kp, N, block, None, 0, stream) == 0
+        held += [A, W, sa, sw]
+        q.append(Gemm(A.data_ptr(), W.data_ptr(), sa.data_ptr(), sw.data_ptr(), guard[1:].data_ptr(), M, N, kp, kw, kp, kp, N))
+        want.append(one)
+        out.append(guard)
+    pair = (Gemm * 2)(*q)
+    for _ in range(2):
+        assert lib.bi8x_gemm_pair(ctypes.byref(pair), code, block, stream) == 0
+        for got, one in zip(out, want):
+            assert torch.equal(got[1:-1], one) and (got[0] == 7).all() and (got[-1] == 7).all()
+            got[1:-1] = 3.0
+
+
+def test_where_the_rule_ends(lib):
+    for tokens, k, n, block, _ in CASES:
+        sizes = _sizes(tokens, k, n)
+        assert _name(lib, sizes, 32) == _name(lib, sizes, 256) == ""
+        for over in ({"A": 8}, {"sW": 2}, {"lda": _up(tokens, 128) + 8}, {"ldw": 1 << 23}, {"kw": 0}, {"kw": _up(tokens, 128) - 8}, {"K": _up(tokens, 128) - 64}, {"ldc": k - 1},
+                     {"C": 0}, {"ldw": 16}, {"N": (1 << 31) - 1, "ldc": 1 << 31}):
+            assert _name(lib, sizes, block, **over) == "", over
+    # few rows in either problem, a contraction that wants its split, two gemm_panels, outputs that are little else than written
+    for tokens, k, n, block in ((128, 9536, 573, 128), (937, 1664, 128, 64), (1141, 768, 19840, 64), (498, 896, 2304, 128), (4096, 4096, 11008, 128), (8192, 768, 3072, 64), (147, 10752, 13477, 64)):
+        assert _name(lib, _sizes(tokens, k, n), block) == "", (tokens, k, n)
