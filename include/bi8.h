@@ -166,8 +166,8 @@ int bi8_gemm_nt_dequant_static(const int8_t *A, const int8_t *W, const float *sA
  * Name of the kernel family that bi8_gemm_nt_dequant_ws runs on a problem with 16-byte aligned operands and
  * `workspace_bytes` of scratch memory ("gemm_wide" for 256x256 tiles, "gemm_wide_256x192", "gemm_wide_256x128", "gemm_wide_128x128",
  * "gemm_wide_128x96", "gemm_wide_256x128_splitk", "gemm_wide_256x192_splitk", "gemm_tile_256x128", "gemm_tile_128x128", "gemm_tile_64x128", "gemm_tile_128x128_splitk", "gemm_tile_64x128_splitk", "gemm_panel", "gemm_panel_splitk", "gemv_rows",
- * "gemv_staged", "gemm_skinny", "gemm_generic"; "gemm_wide+<tile kernel>" for a problem that runs as two launches, the 256x256 kernel on the leading
- * rows or columns that fill whole rounds of workgroups and a tile kernel on the rest; "none" for an empty problem).
+ * "gemv_staged", "gemm_skinny", "gemm_generic"; "gemm_wide+<tile kernel>" for a problem that runs in two parts, the 256x256 kernel on the leading
+ * rows or columns that fill whole rounds of workgroups and a tile kernel on the rest (256x128 tiles in the same launch, the others in a second one); "none" for an empty problem).
  * Static string.  The reference picks its kernel configuration with Triton's autotuner
  * (triton_functions.py:41-65) and offers no way to ask which one ran; tests and benchmarks use this to say so.
  */
