@@ -65,6 +65,21 @@ template <int DT> __device__ __forceinline__ void bi8_store_elem(void *p, int64_
     else ((uint16_t *)p)[i] = (uint16_t)bi8_f16_bits(v);
 }
 
+// Column c of per-tile column sums [tiles][C], added in ascending order: sixteen independent loads at a time (a chain of dependent ones costs a
+// memory latency each).
+__device__ __forceinline__ float bi8_sum_of_tiles(const float *__restrict__ part, int64_t tiles, int64_t C, int64_t c) {
+    float t = 0.0f;
+    for (int64_t t0 = 0; t0 < tiles; t0 += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = t0 + i < tiles ? part[(t0 + i) * C + c] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (t0 + i < tiles) t = (t0 + i == 0) ? v[i] : t + v[i];
+    }
+    return t;
+}
+
 // ---- 16-byte loads of floating-point elements -----------------------------------------------------
 template <int DT> struct Bi8Vec {
     static constexpr int kElems = (DT == BI8_F32) ? 4 : 8;     // elements per 16-byte load

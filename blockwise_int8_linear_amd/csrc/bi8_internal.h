@@ -44,11 +44,20 @@ typedef struct {
     void *C;
     int64_t M, N, K, kw, lda, ldw, ldc;
 } Bi8Gemm;
+/* The last step of column sums (bi8x_colsum_finish) as part of a launch that follows the quantizer: part [ceil(R/128), C] -> out [C] of type dtype. */
+typedef struct {
+    const float *part;
+    void *out;
+    int dtype;
+    int64_t R, C;
+} Bi8ColSums;
 /* Both problems in one launch where that is expected to be faster than two (BI8_ERR_UNSUPPORTED otherwise: nothing is launched); outputs of type
- * c_dtype, operands as for bi8x_gemm with rows on 16-byte boundaries, blocks 64 and 128, no scratch memory.  _name: the kernel whose
+ * c_dtype, operands as for bi8x_gemm with rows on 16-byte boundaries, blocks 64 and 128, no scratch memory; sums: in the same launch, or NULL.  _name: the kernel whose
  * tiles the launch runs, "" where there would be none. */
-int bi8x_gemm_pair(const Bi8Gemm *q, int c_dtype, int block, void *stream);
+int bi8x_gemm_pair(const Bi8Gemm *q, int c_dtype, int block, const Bi8ColSums *sums, void *stream);
 const char *bi8x_gemm_pair_name(const Bi8Gemm *q, int block);
+/* bi8x_gemm without a bias, and the column sums: in the GEMM's launches where one of its kernels takes them, else in one of their own. */
+int bi8x_gemm_sums(const Bi8Gemm *q, int c_dtype, int block, void *workspace, int64_t workspace_bytes, const Bi8ColSums *sums, void *stream);
 
 /* y [M,N] = x [M,K] @ W.T + bias for 3 to 16 rows in one launch: x of C's type is quantized by the workgroups that multiply with it, the
  * bits of y are those of bi8_quantize_rowwise and bi8_gemm_nt_dequant_ws.  W, sW: codes and scales; blocks 64 and 128, K a multiple of

@@ -606,17 +606,7 @@ template <int DT>
 __global__ __launch_bounds__(256) void colsum_finish(const float *__restrict__ part, void *__restrict__ out, int64_t tiles_r, int64_t C) {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= C) return;
-    // sixteen independent loads at a time (a chain of dependent ones costs a memory latency each), added in order
-    float t = 0.0f;
-    for (int64_t t0 = 0; t0 < tiles_r; t0 += 16) {
-        float v[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = t0 + i < tiles_r ? part[(t0 + i) * C + c] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (t0 + i < tiles_r) t = (t0 + i == 0) ? v[i] : t + v[i];
-    }
-    bi8_store_elem<DT>(out, c, t);
+    bi8_store_elem<DT>(out, c, bi8_sum_of_tiles(part, tiles_r, C, c));
 }
 
 template <int DT> int launch_colsum_finish(const float *part, void *out, int64_t tiles_r, int64_t C, hipStream_t st) {

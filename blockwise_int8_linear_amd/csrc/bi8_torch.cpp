@@ -407,6 +407,8 @@ torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &
         }
         const Bias none(Tensor(), 0);
         Tensor gx = need_gx ? empty(s.x_sizes, cfg.out_type, G) : Tensor(), gw = need_gw ? empty({N, K}, cfg.out_type, G) : Tensor();
+        if (sums) result[2] = empty({N}, G.scalar_type(), G);
+        const Bi8ColSums col_sums{(const float *)(base + part_at), sums ? result[2].data_ptr() : nullptr, g_code, M, N};
         bool paired = false;                       // both in one launch, where the library would have it so
         if (both && kx == gq.ld && kw == gtq.ld) {
             const Tensor w = s.wt_packed ? Tensor() : rows_of(held[2]), ws = s.wt_packed ? Tensor() : scales_in(held[3]);
@@ -415,7 +417,7 @@ torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &
                                           s.wt_packed ? wtq.scales(held[2]) : (const float *)ws.data_ptr(), gx.data_ptr(), M, K, kx, s.wt_packed ? kx : up(N, 16), gq.ld,
                                           s.wt_packed ? wtq.ld : ld_of(w), std::max<int64_t>(K, 1)},
                                          {gtq.codes(t), xtq.codes(held[0]), gtq.scales(t), xtq.scales(held[0]), gw.data_ptr(), N, K, kw, kw, gtq.ld, xtq.ld, std::max<int64_t>(K, 1)}};
-                const int rc = bi8x_gemm_pair(pair, float_code(gx), (int)B, stream);
+                const int rc = bi8x_gemm_pair(pair, float_code(gx), (int)B, sums ? &col_sums : nullptr, stream);
                 if (rc != BI8_ERR_UNSUPPORTED) check(rc, "bi8x_gemm_pair");
                 paired = rc == BI8_OK;
             }
@@ -431,17 +433,13 @@ torch::autograd::variable_list linear_backward(const Tensor &G_in, const Shape &
             }
         }
         if (need_gw && !paired) {
-            check(gemm_raw(gtq.codes(t), gtq.scales(t), gtq.ld, xtq.codes(held[0]), xtq.scales(held[0]), xtq.ld, none, gw.data_ptr(), float_code(gw), N, K, kw, kw, B,
-                           need2 > 0 ? base + ws_at : nullptr, need2, stream),
-                  "bi8x_gemm");
+            const Bi8Gemm q{gtq.codes(t), xtq.codes(held[0]), gtq.scales(t), xtq.scales(held[0]), gw.data_ptr(), N, K, kw, kw, gtq.ld, xtq.ld, std::max<int64_t>(K, 1)};
+            void *const ws = need2 > 0 ? base + ws_at : nullptr;
+            if (sums) check(bi8x_gemm_sums(&q, float_code(gw), (int)B, ws, need2, &col_sums, stream), "bi8x_gemm_sums");
+            else check(gemm_raw(q.A, q.sA, q.lda, q.W, q.sW, q.ldw, none, q.C, float_code(gw), N, K, kw, kw, B, ws, need2, stream), "bi8x_gemm");
         }
         result[0] = gx;
         result[1] = gw;
-        if (sums) {
-            Tensor gb = empty({N}, G.scalar_type(), G);
-            check(bi8x_colsum_finish((const float *)(base + part_at), gb.data_ptr(), g_code, M, N, stream), "bi8x_colsum_finish");
-            result[2] = gb;
-        }
     } else {
         if (need_gx) {
             auto [q, qs] = quantize_rowwise(G, B, cfg.scale_type);

@@ -14,14 +14,17 @@ class Gemm(ctypes.Structure):
     _fields_ = [(n, _vp) for n in ("A", "W", "sA", "sW", "C")] + [(n, _i64) for n in ("M", "N", "K", "kw", "lda", "ldw", "ldc")]
 
 
-@pytest.fixture(scope="module")
-def lib():
-    from blockwise_int8_linear_amd import _lib
-    lib = _lib.load()
-    lib.bi8x_gemm_pair.argtypes = [_vp, ctypes.c_int, ctypes.c_int, _vp]
+def with_types(lib):
+    lib.bi8x_gemm_pair.argtypes = [_vp, ctypes.c_int, ctypes.c_int, _vp, _vp]
     lib.bi8x_gemm_pair_name.argtypes, lib.bi8x_gemm_pair_name.restype = [_vp, ctypes.c_int], ctypes.c_char_p
     lib.bi8x_gemm.argtypes = [_vp] * 5 + [ctypes.c_int, _vp, ctypes.c_int] + [_i64] * 7 + [ctypes.c_int, _vp, _i64, _vp]
     return lib
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from blockwise_int8_linear_amd import _lib
+    return with_types(_lib.load())
 
 
 def _up(n, to):
@@ -80,7 +83,7 @@ def test_bits_of_the_one_pass_kernels(lib, tokens, k, n, block, tile, dtype):
         out.append(guard)
     pair = (Gemm * 2)(*q)
     for _ in range(2):
-        assert lib.bi8x_gemm_pair(ctypes.byref(pair), code, block, stream) == 0
+        assert lib.bi8x_gemm_pair(ctypes.byref(pair), code, block, None, stream) == 0
         for got, one in zip(out, want):
             assert torch.equal(got[1:-1], one) and (got[0] == 7).all() and (got[-1] == 7).all()
             got[1:-1] = 3.0
