@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from util import DTYPES
+from util import DTYPES, config_as
 
 _vp, _i64 = ctypes.c_void_p, ctypes.c_int64
 
@@ -99,3 +99,49 @@ def test_where_the_rule_ends(lib):
     # few rows in either problem, a contraction that wants its split, two gemm_panels, outputs that are little else than written
     for tokens, k, n, block in ((128, 9536, 573, 128), (937, 1664, 128, 64), (1141, 768, 19840, 64), (498, 896, 2304, 128), (4096, 4096, 11008, 128), (8192, 768, 3072, 64), (147, 10752, 13477, 64)):
         assert _name(lib, _sizes(tokens, k, n), block) == "", (tokens, k, n)
+
+
+# layers of which one gradient by itself is summed in pieces of K (or has a rest that is)
+PIECES = [
+    (293, 5888, 8192, 64), (425, 4544, 8000, 128), (411, 5312, 5504, 128), (2584, 768, 4992, 128), (979, 2560, 5824, 128),      # 128x128 and 256x128 tiles
+    (5676, 3008, 2496, 128), (5424, 4992, 3392, 64), (3314, 3264, 10303, 64),       # the rest of a cut
+    (2091, 2240, 15296, 128), (8117, 896, 4800, 128),                               # 256x192 tiles
+]
+
+
+def _own(lib, sizes, block):
+    return [lib.bi8_gemm_kernel_name(m, n, _up(k, 128), _up(k, 128), _up(k, 128), block, lib.bi8_gemm_workspace_bytes(m, n, _up(k, 128), block)).decode() for m, n, k in sizes]
+
+
+def test_pieces_of_k_stay_pieces(lib):
+    """one chain of sums over all of K has a larger error than its pieces: such a gradient keeps the launches it has by itself"""
+    for tokens, k, n, block in PIECES:
+        sizes = _sizes(tokens, k, n)
+        assert any("splitk" in name for name in _own(lib, sizes, block)), (tokens, k, n)
+        assert _name(lib, sizes, block) == "", (tokens, k, n)
+    taken = 0
+    for tokens in (129, 300, 511, 1000, 1500, 2600, 4100, 8000):
+        for k in (512, 1111, 2304, 4992, 11008):
+            for n in (640, 1999, 3456, 8320, 20000):
+                for block in (64, 128):
+                    sizes = _sizes(tokens, k, n)
+                    if _name(lib, sizes, block):
+                        taken += 1
+                        assert not any("splitk" in name for name in _own(lib, sizes, block)), (tokens, k, n, block)
+    assert taken > 50
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,k,n,block", [c[:4] for c in CASES] + PIECES[:1] + PIECES[2:4] + PIECES[6:8] + PIECES[9:])
+def test_bits_do_not_depend_on_the_other_gradient(tokens, k, n, block):
+    """x and the weight differentiated together, and each alone"""
+    import blockwise_int8_linear_amd as pkg
+    gen = torch.Generator(device="cuda:0").manual_seed(tokens + k + n)
+    x, w, g = (torch.randn(*s, generator=gen, device="cuda:0") for s in ((tokens, k), (n, k), (tokens, n)))
+    got = {}
+    with config_as(pkg, block, torch.float32):
+        for which in ("xw", "x", "w"):
+            leaves = {"x": x.clone().requires_grad_("x" in which), "w": w.clone().requires_grad_("w" in which)}
+            pkg.blockwise_int8_linear.apply(leaves["x"], leaves["w"], None).backward(g)
+            got[which] = {name: t.grad for name, t in leaves.items()}
+    assert torch.equal(got["xw"]["x"], got["x"]["x"]) and torch.equal(got["xw"]["w"], got["w"]["w"])
