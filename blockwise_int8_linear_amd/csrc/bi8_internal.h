@@ -55,7 +55,7 @@ typedef struct {
  * c_dtype, operands as for bi8x_gemm with rows on 16-byte boundaries, blocks 64 and 128, no scratch memory; sums: in the same launch, or NULL.  _name: the kernel whose
  * tiles the launch runs, "" where there would be none. */
 int bi8x_gemm_pair(const Bi8Gemm *q, int c_dtype, int block, const Bi8ColSums *sums, void *stream);
-const char *bi8x_gemm_pair_name(const Bi8Gemm *q, int block);
+const char *bi8x_gemm_pair_name(const Bi8Gemm *q, int c_dtype, int block);
 /* bi8x_gemm without a bias, and the column sums: in the GEMM's launches where one of its kernels takes them, else in one of their own. */
 int bi8x_gemm_sums(const Bi8Gemm *q, int c_dtype, int block, void *workspace, int64_t workspace_bytes, const Bi8ColSums *sums, void *stream);
 

@@ -16,7 +16,7 @@ class Gemm(ctypes.Structure):
 
 def with_types(lib):
     lib.bi8x_gemm_pair.argtypes = [_vp, ctypes.c_int, ctypes.c_int, _vp, _vp]
-    lib.bi8x_gemm_pair_name.argtypes, lib.bi8x_gemm_pair_name.restype = [_vp, ctypes.c_int], ctypes.c_char_p
+    lib.bi8x_gemm_pair_name.argtypes, lib.bi8x_gemm_pair_name.restype = [_vp, ctypes.c_int, ctypes.c_int], ctypes.c_char_p
     lib.bi8x_gemm.argtypes = [_vp] * 5 + [ctypes.c_int, _vp, ctypes.c_int] + [_i64] * 7 + [ctypes.c_int, _vp, _i64, _vp]
     return lib
 
@@ -36,11 +36,11 @@ def _sizes(tokens, k, n):
     return (tokens, k, n), (n, k, tokens)
 
 
-def _name(lib, sizes, block, at=4096, **over):
+def _name(lib, sizes, block, at=4096, dtype="bf16", **over):
     q = (Gemm * 2)(*(Gemm(at, at, at, at, at, m, n, _up(k, 128), _up(k, 128), _up(k, 128), _up(k, 128), n) for m, n, k in sizes))
     for field, value in over.items():
         setattr(q[1], field, value)
-    return lib.bi8x_gemm_pair_name(ctypes.byref(q), block).decode()
+    return lib.bi8x_gemm_pair_name(ctypes.byref(q), ["f32", "bf16", "f16"].index(dtype), block).decode()
 
 
 # tokens, in, out, block, the tile
@@ -99,6 +99,13 @@ def test_where_the_rule_ends(lib):
     # few rows in either problem, a contraction that wants its split, two gemm_panels, outputs that are little else than written
     for tokens, k, n, block in ((128, 9536, 573, 128), (937, 1664, 128, 64), (1141, 768, 19840, 64), (498, 896, 2304, 128), (4096, 4096, 11008, 128), (8192, 768, 3072, 64), (147, 10752, 13477, 64)):
         assert _name(lib, _sizes(tokens, k, n), block) == "", (tokens, k, n)
+    # a gemm_panel of 60 stages or more, many outputs per stage beside a problem that fills the chip by itself (fp32 ones count twice), little to save at block 64
+    for tokens, k, n, block, dtype in ((1016, 3456, 17984, 128, "bf16"), (1922, 1728, 14464, 128, "f16"), (1788, 2176, 21632, 128, "f32"), (695, 11328, 6144, 128, "bf16"),
+                                       (796, 9472, 7708, 128, "f16"), (2021, 12096, 512, 128, "f32"), (6548, 10624, 1024, 64, "f32"), (292, 1472, 576, 64, "bf16")):
+        assert _name(lib, _sizes(tokens, k, n), block, dtype=dtype) == "", (tokens, k, n)
+    # ... and on the near side of these lines
+    for tokens, k, n, block, dtype in ((7340, 3072, 832, 128, "f16"), (226, 11072, 1381, 128, "bf16"), (768, 8448, 3136, 128, "f32"), (323, 2304, 576, 64, "f16")):
+        assert _name(lib, _sizes(tokens, k, n), block, dtype=dtype) != "", (tokens, k, n)
 
 
 # layers of which one gradient by itself is summed in pieces of K (or has a rest that is)
