@@ -45,3 +45,6 @@ def test_where_the_rule_ends(lib):  # noqa: F811
     assert name(8192, 768, 50304, 64) == NAME and name(2304, 2304, 7168, 128) == NAME
     for other in ((8192, 768, 7040, 128), (8192, 768, 14208, 64), (512, 11008, 32768, 128), (8192, 769, 16384, 128), (8192, 768, 16384, 32), (8192, 768, 16384, 128, 32 << 20)):
         assert name(*other) != NAME, other
+    # at block 128 more than 110 tiles want a stage more each, except for up to 640 rows
+    assert all(name(*taken) == NAME for taken in ((7814, 640, 9472, 128), (5440, 896, 7168, 128), (513, 8000, 7296, 128), (640, 8000, 7168, 128), (7832, 640, 14336, 64)))
+    assert all(name(*other) != NAME for other in ((7832, 640, 8064, 128), (8128, 768, 8064, 128), (2560, 2240, 7168, 128), (641, 8000, 7168, 128)))
