@@ -314,7 +314,7 @@ def test_kernel_choice_by_shape():
     assert name(300, 500, 500, 128) == "gemm_generic" and name(300, 500, 512, 128, 0, 520) == "gemm_generic"
     assert name(300, 500, 512, 48) == "gemm_generic"
     assert name(0, 500, 512, 128) == "none"
-    # a split never wants more than the static scratch array holds: workgroups + tiles - 1 < 512 slabs of 128 x 128 fp32
+    # these want no more than the static scratch array holds: workgroups + tiles - 1 < 512 slabs of 128 x 128 fp32 (what may: the test below)
     for M in (33, 64, 100, 128, 256, 512, 1000, 2048, 3072, 4000):
         for N in (128, 768, 1024, 4096, 11008, 50257):
             for K in (1024, 4096, 11008 , 8192 * 4):
@@ -340,6 +340,25 @@ def test_kernel_choice_by_shape():
         ops._workspace(_Probe(), M, 4096, 11008, 128, None, None)
         ops._ws_need.pop((M, 4096, 11008, 128), None)
     assert asked == [(17, 4096, 11008, 128)]
+
+
+def test_only_the_256x192_split_wants_more_than_the_static_array():
+    """bi8_gemm_nt_dequant_static gives the bits of bi8_gemm_nt_dequant_ws wherever the array holds what the split wants: always up to 512 rows,
+    and beyond them but for the 256x192 tiles' two pieces, which want up to 48 MiB"""
+    lib = _lib.load()
+    held = lib.bi8_static_scratch_bytes()
+    most = 0
+    for M in (17, 64, 129, 256, 257, 384, 385, 511, 512, 513, 700, 1100, 2048, 2305, 5632, 8192, 16384):
+        for N in (384, 768, 1536, 2304, 4800, 6000, 8192, 8256, 10944, 11008, 12288, 16448, 24576):
+            for K in (2048, 7040, 7168, 14208, 14336, 16384, 32768, 50304):
+                for block in (32, 64, 128):
+                    need = lib.bi8_gemm_workspace_bytes(M, N, K, block)
+                    assert need <= 48 << 20
+                    if need > held:
+                        assert M > 512 and lib.bi8_gemm_kernel_name(M, N, K, K, K, block, need) == b"gemm_wide_256x192_splitk", (M, N, K, block)
+                        assert b"256x192_splitk" not in lib.bi8_gemm_kernel_name(M, N, K, K, K, block, held)
+                    most = max(most, need)
+    assert most == lib.bi8_gemm_workspace_bytes(8192, 768, 50304, 64) == 48 << 20
 
 
 def test_every_gemm_has_scratch_memory_of_its_own():

@@ -1,9 +1,11 @@
 """The bias gradient of a layer, whose last step runs beside a GEMM of the backward pass (gemm_panel, gemm_wide_pair, splitk_reduce) or in a launch of its
 own: the bits of bi8_quantize_dual_colsum, whichever kernel it is, at numbers of columns around those of a workgroup and of rows around a tile's 128."""
+import ctypes
+
 import pytest
 import torch
 
-from util import DTYPES, config_as
+from util import DTYPES, config_as, kernel_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +43,40 @@ def test_bits(tokens, k, n, block, kernel, dtype):
         bias.grad = None
         pkg.blockwise_int8_linear.apply(x, w, bias).backward(g)
     assert torch.equal(alone, want) and torch.equal(bias.grad, want)
+
+
+class _ColSums(ctypes.Structure):
+    _fields_ = [("part", ctypes.c_void_p), ("out", ctypes.c_void_p), ("dtype", ctypes.c_int), ("R", ctypes.c_int64), ("C", ctypes.c_int64)]
+
+
+@pytest.mark.parametrize("tokens,k,n,block,kernel", [c for c in CASES if c[4]])
+def test_launches(tokens, k, n, block, kernel):
+    """the sums take no launch of their own beside gemm_panel, the pair and a split's reduction, and one beside the other kernels"""
+    from blockwise_int8_linear_amd import _lib
+    import test_gpu_gemm_pair as pairs
+    lib, dev = pairs.with_types(_lib.load()), "cuda:0"
+    sizes = [(m, c, pairs._up(d, 128)) for m, c, d in pairs._sizes(tokens, k, n)]
+    part, out = torch.zeros(-(-tokens // 128), n, device=dev), torch.empty(n, device=dev)
+    sums = _ColSums(part.data_ptr(), out.data_ptr(), 0, tokens, n)
+    held, problems = [], []
+    for M, N, K in sizes:
+        held.append([torch.zeros(M, K, dtype=torch.int8, device=dev), torch.zeros(N, K, dtype=torch.int8, device=dev), torch.ones(K // block, M, device=dev),
+                     torch.ones(K // block, N, device=dev), torch.empty(M, N, dtype=torch.bfloat16, device=dev)])
+        problems.append(pairs.Gemm(*(t.data_ptr() for t in held[-1]), M, N, K, K, K, K, N))
+    if kernel == "pair":
+        both = (pairs.Gemm * 2)(*problems)
+
+        def call():
+            assert lib.bi8x_gemm_pair(ctypes.byref(both), 1, block, ctypes.byref(sums), torch.cuda.current_stream().cuda_stream) == 0
+
+        assert kernel_launches(call) == 1
+        return
+    M, N, K = sizes[1]
+    need = lib.bi8_gemm_workspace_bytes(M, N, K, block)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    lib.bi8x_gemm_sums.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
+
+    def call():
+        assert lib.bi8x_gemm_sums(ctypes.byref(problems[1]), 1, block, ws.data_ptr() if need else None, need, ctypes.byref(sums), torch.cuda.current_stream().cuda_stream) == 0
+
+    assert kernel_launches(call) == (1 if kernel == "gemm_panel" else 2)      # (a split: with its reduction; the others: with bi8x_colsum_finish)

@@ -2,8 +2,10 @@
 several rounds, ragged ends, odd numbers of stages, a single stage in all, with and without a bias, against the checks of
 test_gpu_gemm_random_shapes (CPU checker on sampled rows, the whole output against a float64 product, guard rows)."""
 import pytest
+import torch
 
 import test_gpu_gemm_random_shapes as shapes
+from util import DTYPES, kernel_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -27,3 +29,27 @@ def test_shape(case):
     M, N, K, block = case[:4]
     assert _lib.load().bi8_gemm_kernel_name(M, N, K, K, K, block, 0).decode() == "gemm_wide+gemm_wide_256x128"
     shapes.test_random_shape(case)
+
+
+# cuts whose rest is on other tiles: a launch of its own, or two where it is split over K
+OTHER_CUTS = [(1300, 11008, 128, 64, "bf16", False, False, 2), (4128, 5000, 128, 64, "f32", True, False, 2), (2100, 8192, 4096, 128, "bf16", True, True, 3)]
+
+
+@pytest.mark.parametrize("case", [c + (1,) for c in CASES] + OTHER_CUTS, ids=lambda c: f"{c[0]}x{c[1]}x{c[2]}-b{c[3]}-{c[7]}")
+def test_launches(case):
+    from blockwise_int8_linear_amd import _lib
+    lib = _lib.load()
+    M, N, K, block, dtype, with_bias, with_scratch, launches = case
+    need = lib.bi8_gemm_workspace_bytes(M, N, K, block) if with_scratch else 0
+    name = lib.bi8_gemm_kernel_name(M, N, K, K, K, block, need).decode()
+    assert name.startswith("gemm_wide+") and (name == "gemm_wide+gemm_wide_256x128") == (launches == 1) and ("splitk" in name) == (launches == 3)
+    dev = "cuda:0"
+    A, W = (torch.zeros(rows, K, dtype=torch.int8, device=dev) for rows in (M, N))
+    sa, sw = (torch.ones(K // block, rows, device=dev) for rows in (M, N))
+    C, bias, ws = torch.empty(M, N, dtype=DTYPES[dtype], device=dev), torch.zeros(N, device=dev), torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+
+    def call():
+        assert lib.bi8_gemm_nt_dequant_ws(A.data_ptr(), W.data_ptr(), sa.data_ptr(), sw.data_ptr(), bias.data_ptr() if with_bias else None, 0, C.data_ptr(),
+                                          list(DTYPES).index(dtype), M, N, K, K, K, N, block, ws.data_ptr() if need else None, need, torch.cuda.current_stream().cuda_stream) == 0
+
+    assert kernel_launches(call) == launches

@@ -1,6 +1,7 @@
 """Helpers shared by the tests: golden-vector loading and seeded workload construction."""
 from __future__ import annotations
 
+import ctypes
 import json
 import os
 
@@ -97,3 +98,23 @@ def assert_close_rms(got, ref, tol, bias=None):
         i = (err - bound).argmax()
         raise AssertionError(f"{int((err > bound).sum())} of {err.numel()} outside the bound; worst at flat index {i.item()}: got "
                              f"{got.reshape(-1)[i].item()} want {ref.reshape(-1)[i].item()} (rms {rms:.3e})")
+
+
+def kernel_launches(call) -> int:
+    """How many kernels one call launches: the kernel nodes of a HIP graph that records it (after an eager call; the graph is not run)."""
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        held = call()
+    hip = ctypes.CDLL(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so"))
+    recorded, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(recorded, None, ctypes.byref(count)) == 0
+    nodes = (ctypes.c_void_p * count.value)()
+    assert hip.hipGraphGetNodes(recorded, nodes, ctypes.byref(count)) == 0
+    kind, kernels = ctypes.c_int(-1), 0
+    for node in nodes:
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        kernels += kind.value == 0                 # hipGraphNodeTypeKernel
+    del held
+    return kernels
