@@ -42,7 +42,7 @@ extern "C" {
 #define BI8_ERR_BAD_SHAPE 4   /* negative size, or a leading dimension smaller than the row length */
 #define BI8_ERR_TOO_LARGE 5   /* a dimension exceeds what one launch can index */
 #define BI8_ERR_UNSUPPORTED 6 /* valid arguments outside what this entry point covers; nothing was launched */
-#define BI8_ERR_SCRATCH_TOO_SMALL 7 /* the problem wants more scratch memory than the library's static buffer holds */
+#define BI8_ERR_SCRATCH_TOO_SMALL 7 /* reserved: the static buffer cannot hold what a problem needs (no call returns it at present) */
 #define BI8_ERR_HIP_BASE 1000 /* BI8_ERR_HIP_BASE + hipError_t */
 
 /* ABI version of this header (bumped on any signature change). */
@@ -149,9 +149,9 @@ int bi8_gemm_nt_dequant_ws(const int8_t *A, const int8_t *W, const float *sA, co
  * makes no hipMalloc / hipFree and no allocating library call; the first call on a device looks up the array's
  * address there (hipGetSymbolAddress), so make one call on each device outside any capture.
  * Same kernels, same results (bit for bit) as bi8_gemm_nt_dequant_ws given a workspace of 32 MiB, or of
- * bi8_gemm_workspace_bytes() where that is less: only the split of a long K of more than 512 rows ("gemm_wide_256x192_splitk")
- * wants more than the array holds, and is not used here.  (BI8_ERR_SCRATCH_TOO_SMALL: a split that only fits a larger
- * array; with the present rules there is none.)
+ * bi8_gemm_workspace_bytes() where that is less, as it is for up to 512 rows whatever the problem: only the split of a long
+ * K of more rows ("gemm_wide_256x192_splitk", up to 48 MiB) wants more than the array holds, and such a problem runs here in one
+ * pass, in another order of its fp32 sums.  No call returns BI8_ERR_SCRATCH_TOO_SMALL.
  * All calls on one GPU share the array, which keeps the last call's contents (every call overwrites what it reads,
  * nothing has to start at zero): calls that overlap on one GPU -- two streams, two host threads -- race on it.
  * Serialize them on one stream, or give the overlapping ones their own workspace through bi8_gemm_nt_dequant_ws.
